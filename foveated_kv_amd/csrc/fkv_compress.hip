@@ -205,25 +205,55 @@ __global__ __launch_bounds__(256) void compress_kernel(CompressArgs a) {
 // ---------------------------------------------------------------------------
 
 constexpr int kScaleThreads = 256;
+constexpr int kScaleRows = 4;      // rows a lane group loads together
+constexpr int kScaleBlocks = 2048; // workgroups the reduction aims for
 
-// One workgroup per (batch, head): the far rows are positions mid_start..
-// (far_idx NULL) or far_idx[bh][f]; out-of-range indices are zero rows.
+// Workgroups per (batch, head) of the reduction: each takes at least
+// kScaleRows rows per lane group, so their maxima (one fp32 each) always fit
+// the head's F * D bytes of far codes, where they wait for kscale_finish.
+__host__ __device__ inline int kscale_parts(int F, int D, int BH) {
+    const int64_t rows = (int64_t)kScaleRows * (kScaleThreads / (D / 8));
+    int64_t p = cdiv(F, rows);
+    const int64_t most = cdiv(kScaleBlocks, BH);
+    if (p > most) p = most;
+    return p < 1 ? 1 : (int)p;
+}
+
+// Bound by the one read of the far keys.  A maximum does not depend on the
+// order, so the rows of a (batch, head) are dealt over as many workgroups as
+// fill the chip (one workgroup per head read 121 MB of keys at 8 heads x 59K
+// rows in 3,690 us: eight CUs; the whole call went from 4,070 to 414 us), and
+// each lane group has kScaleRows rows in flight.  Far rows are positions mid_start.. (far_idx NULL) or
+// far_idx[bh][f]; out-of-range indices are zero rows.
 template <int D>
 __global__ __launch_bounds__(kScaleThreads) void kscale_kernel(CompressArgs a, const int32_t* __restrict__ far_idx,
-                                                               float* __restrict__ out) {
+                                                               float* __restrict__ part_max) {
     constexpr int LPR = D / 8, RPB = kScaleThreads / LPR;
     __shared__ float red[kScaleThreads / kWave];
-    const int bh = blockIdx.x, sub = threadIdx.x % LPR;
+    const int bh = blockIdx.y, sub = threadIdx.x % LPR, parts = gridDim.x;
     const int F = a.tb.far_count;
     float amax = 0.f;
-    for (int f = threadIdx.x / LPR; f < F; f += RPB) {
-        const int t = far_idx ? far_idx[(int64_t)bh * F + f] : a.tb.mid_start + f;
-        if (t < 0 || t >= a.S) continue;
-        uint16_t kx[8];
-        load8(a.k, a.dtype, ((int64_t)bh * a.S + t) * D + sub * 8, kx);
+    for (int64_t f0 = (int64_t)blockIdx.x * kScaleRows * RPB + threadIdx.x / LPR; f0 < F;
+         f0 += (int64_t)parts * kScaleRows * RPB) {
+        int t[kScaleRows];
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (((kx[i] >> 10) & 0x1f) != 0x1f) amax = fmaxf(amax, fabsf(h2f(kx[i])));
+        for (int u = 0; u < kScaleRows; u++) {
+            const int64_t f = f0 + u * RPB;
+            t[u] = f >= F ? -1 : far_idx ? far_idx[(int64_t)bh * F + f] : a.tb.mid_start + (int)f;
+        }
+        uint16_t kx[kScaleRows][8];
+#pragma unroll
+        for (int u = 0; u < kScaleRows; u++) {
+            const bool in = t[u] >= 0 && t[u] < a.S;
+            // a row outside the sequence reads row 0 and is left out below
+            load8(a.k, a.dtype, ((int64_t)bh * a.S + (in ? t[u] : 0)) * D + sub * 8, kx[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kScaleRows; u++)
+            if (t[u] >= 0 && t[u] < a.S)
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    if (((kx[u][i] >> 10) & 0x1f) != 0x1f) amax = fmaxf(amax, fabsf(h2f(kx[u][i])));
     }
     amax = wave_max(amax);
     if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = amax;
@@ -231,8 +261,18 @@ __global__ __launch_bounds__(kScaleThreads) void kscale_kernel(CompressArgs a, c
     if (threadIdx.x == 0) {
         float m = 0.f;
         for (int w = 0; w < kScaleThreads / kWave; w++) m = fmaxf(m, red[w]);
-        out[bh] = m > 0.f ? m / 240.0f : 1.0f;
+        part_max[(int64_t)bh * parts + blockIdx.x] = m;
     }
+}
+
+// One wave per (batch, head): the largest of its workgroups' maxima -> scale.
+__global__ __launch_bounds__(kWave) void kscale_finish_kernel(const float* __restrict__ part_max, int parts,
+                                                              float* __restrict__ out) {
+    const int bh = blockIdx.x;
+    float m = 0.f;
+    for (int i = threadIdx.x; i < parts; i += kWave) m = fmaxf(m, part_max[(int64_t)bh * parts + i]);
+    m = wave_max(m);
+    if (threadIdx.x == 0) out[bh] = m > 0.f ? m / 240.0f : 1.0f;
 }
 
 // ---------------------------------------------------------------------------
@@ -455,8 +495,17 @@ int compress_launch(const char* fn, const fkv_tier_config* cfg, fkv::CompressArg
     const bool g32 = cfg->v_group == 32;
     if (cfg->k_scale) {
         if (!far_k_scale) return fkv::set_error(std::string(fn) + ": k_scale needs far_k_scale");
-        hipLaunchKernelGGL(D == 128 ? fkv::kscale_kernel<128> : fkv::kscale_kernel<64>, dim3((unsigned)(B * H)),
-                           dim3(fkv::kScaleThreads), 0, st, a, near_idx ? far_idx : nullptr, far_k_scale);
+        const int parts = fkv::kscale_parts(a.tb.far_count, D, B * H);
+        // the far code buffer holds the workgroups' maxima until they are
+        // reduced (the compress launch then writes the codes over them); with
+        // no far rows there is no buffer: the scales are 1
+        float* part_max = a.tb.far_count > 0 ? (float*)a.far_k : nullptr;
+        if (part_max)
+            hipLaunchKernelGGL(D == 128 ? fkv::kscale_kernel<128> : fkv::kscale_kernel<64>,
+                               dim3((unsigned)parts, (unsigned)(B * H)), dim3(fkv::kScaleThreads), 0, st, a,
+                               near_idx ? far_idx : nullptr, part_max);
+        hipLaunchKernelGGL(fkv::kscale_finish_kernel, dim3((unsigned)(B * H)), dim3(fkv::kWave), 0, st, part_max,
+                           part_max ? parts : 0, far_k_scale);
         a.kscale = far_k_scale;
     }
     const int rpb = 256 / (D / 8);
