@@ -297,15 +297,171 @@ __device__ inline uint64_t rank_key(const float* row, int pos) {
 }
 
 constexpr int kPartThreads = 1024;
+constexpr int kPartWaves = kPartThreads / kWave;
+
+// Fixed slots of a near index row: sinks, window, headroom.
+__device__ inline void fixed_slots(int32_t* nrow, int S, const fkv_tiers& tb, int tid) {
+    const int k = tb.near_from_mid;
+    for (int i = tid; i < tb.n_near_padded; i += kPartThreads) {
+        if (i < tb.n_sinks) nrow[i] = i;
+        else if (i >= tb.n_sinks + k && i < tb.r_actual) nrow[i] = S - tb.window + (i - tb.n_sinks - k);
+        else if (i >= tb.r_actual) nrow[i] = -1;
+    }
+}
+
+constexpr int kPartRegs = 64;  // most tokens per thread held in registers
+constexpr int kPartBits = 11, kPartBins = 1 << kPartBits, kPartCopies = 4;
+
+// Partition of a (batch, head) whose middle fits the workgroup's registers,
+// R tokens per thread (at most kPartThreads * R in all).  Bound by one CU's
+// chain of passes, not by memory, so the row is read once: wave w holds
+// order_key of the middle's tokens w * R * 64 .. in position order (register
+// r: 64 consecutive tokens).  A radix select of 11 + 11 + 10 bits over the
+// registers (LDS histograms, one per wave modulo kPartCopies; one per lane
+// modulo 16, free of bank conflicts, was no faster: the passes are bound by
+// their vector instructions) finds
+// the near_from_mid-th largest key v and how many tokens equal to it stay
+// near (the last ones in position order: the later token wins a tie, which
+// is what the 64-bit rank key orders by).  The compaction needs no block
+// step per chunk: a token's far row is its position less the near tokens
+// before it, and those follow from one scan of the waves' counts and
+// ballots.  64K tokens x 8 heads: 190 us with 8-bit passes that each re-read
+// the row and a block scan per 1,024 tokens, 53 us here.
+template <int R>
+__global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const float* __restrict__ imp, int S,
+                                                                     fkv_tiers tb, int32_t* __restrict__ near_idx,
+                                                                     int32_t* __restrict__ far_idx) {
+    __shared__ uint32_t hist[kPartCopies][kPartBins];
+    __shared__ uint32_t wtot[kPartWaves], wgt[kPartWaves], weq[kPartWaves];
+    __shared__ uint32_t s_bin, s_rem, s_cnt;
+    const int bh = blockIdx.x, tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+    const int npad = tb.n_near_padded, F = tb.far_count, m0 = tb.mid_start;
+    const int mlen = tb.mid_end > tb.mid_start ? tb.mid_end - tb.mid_start : 0;
+    const int k = tb.near_from_mid;
+    const float* row = imp + (int64_t)bh * S + m0;
+    int32_t* nrow = near_idx + (int64_t)bh * npad;
+    int32_t* frow = far_idx + (int64_t)bh * F;
+    const int i0 = wave * R * kWave + lane;  // the lane's first token of the middle
+    const bool all = k >= mlen, none = k <= 0;
+    uint32_t key[R];
+    uint32_t v = 0, equal_far = 0;  // near <=> key > v, or key == v and not among the first equal_far such
+    if (!all && !none) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int i = i0 + r * kWave;
+            key[r] = order_key(i < mlen ? row[i] : 0.f);
+        }
+        fixed_slots(nrow, S, tb, tid);
+        uint32_t rem = k;
+        constexpr int shift[3] = {32 - kPartBits, 32 - 2 * kPartBits, 0};
+        constexpr int bits[3] = {kPartBits, kPartBits, 32 - 2 * kPartBits};
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            for (int i = tid; i < kPartCopies * kPartBins; i += kPartThreads) (&hist[0][0])[i] = 0;
+            __syncthreads();
+            const uint32_t high = p == 0 ? 0u : ~0u << (shift[p] + bits[p]);  // digits already known
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (i0 + r * kWave < mlen && ((key[r] ^ v) & high) == 0)
+                    atomicAdd(&hist[wave % kPartCopies][(key[r] >> shift[p]) & ((1u << bits[p]) - 1)], 1u);
+            __syncthreads();
+            // thread t takes bins top - 2t and top - 2t - 1: an inclusive scan
+            // over the threads counts the keys from the top bin down
+            const int hi = kPartBins - 1 - 2 * tid;
+            uint32_t c1 = 0, c0 = 0;
+#pragma unroll
+            for (int q = 0; q < kPartCopies; q++) {
+                c1 += hist[q][hi];
+                c0 += hist[q][hi - 1];
+            }
+            uint32_t inc = c1 + c0;
+#pragma unroll
+            for (int d = 1; d < kWave; d <<= 1) {
+                const uint32_t t = __shfl_up(inc, d, kWave);
+                if (lane >= d) inc += t;
+            }
+            if (lane == kWave - 1) wtot[wave] = inc;
+            __syncthreads();
+            uint32_t above = inc - c1 - c0;
+#pragma unroll
+            for (int w = 0; w < kPartWaves; w++)
+                if (w < wave) above += wtot[w];
+            if (above < rem && above + c1 >= rem) {
+                s_bin = hi;
+                s_rem = rem - above;
+                s_cnt = c1;
+            } else if (above + c1 < rem && above + c1 + c0 >= rem) {
+                s_bin = hi - 1;
+                s_rem = rem - above - c1;
+                s_cnt = c0;
+            }
+            __syncthreads();
+            v |= s_bin << shift[p];
+            rem = s_rem;
+        }
+        equal_far = s_cnt - rem;
+        uint32_t gt = 0, eq = 0;  // the wave's tokens above and at v
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const bool in = i0 + r * kWave < mlen;
+            gt += __popcll(__ballot(in && key[r] > v));
+            eq += __popcll(__ballot(in && key[r] == v));
+        }
+        if (lane == 0) {
+            wgt[wave] = gt;
+            weq[wave] = eq;
+        }
+        __syncthreads();
+    } else {
+        fixed_slots(nrow, S, tb, tid);
+    }
+    uint32_t near_before = 0, eq_before = 0;  // in the waves before this one
+    if (!all && !none) {
+#pragma unroll
+        for (int w = 0; w < kPartWaves; w++)
+            if (w < wave) {
+                near_before += wgt[w];
+                eq_before += weq[w];
+            }
+        near_before += eq_before > equal_far ? eq_before - equal_far : 0u;
+    } else if (all) {
+        near_before = min(wave * R * kWave, mlen);
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int i = i0 + r * kWave;
+        const bool in = i < mlen;
+        bool nf = in && all;
+        if (!all && !none) {
+            const uint64_t em = __ballot(in && key[r] == v);
+            const uint32_t rank = eq_before + __builtin_amdgcn_mbcnt_hi((uint32_t)(em >> 32),
+                                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)em, 0u));
+            nf = in && (key[r] > v || (key[r] == v && rank >= equal_far));
+            eq_before += __popcll(em);
+        }
+        const uint64_t nm = __ballot(nf);
+        const int before = (int)(near_before + __builtin_amdgcn_mbcnt_hi((uint32_t)(nm >> 32),
+                                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)nm, 0u)));
+        if (nf) {
+            if (before < k) nrow[tb.n_sinks + before] = m0 + i;
+        } else if (in && i - before < F) {
+            frow[i - before] = m0 + i;
+        }
+        near_before += __popcll(nm);
+    }
+}
 
 // One workgroup per (batch, head).  The near_from_mid-th largest rank key
 // is found by an 8-pass MSB-first radix select (256-bin LDS histograms);
 // then the middle is compacted in position order into near slots
 // n_sinks.. and far slots 0.. with a block-wide scan per 1024-token chunk.
+// For middles of more than kPartThreads * kPartRegs tokens, which do not fit
+// partition_regs_kernel's registers.
 __global__ __launch_bounds__(kPartThreads) void partition_kernel(const float* __restrict__ imp, int S, fkv_tiers tb,
                                                                 int32_t* __restrict__ near_idx,
                                                                 int32_t* __restrict__ far_idx) {
-    constexpr int NW = kPartThreads / 64;
+    constexpr int NW = kPartWaves;
     __shared__ uint32_t hist[NW][256];  // one histogram per wave (less atomic contention)
     __shared__ uint64_t s_prefix;
     __shared__ int s_rem;
@@ -319,12 +475,7 @@ __global__ __launch_bounds__(kPartThreads) void partition_kernel(const float* __
     const int k = tb.near_from_mid;
     int32_t* nrow = near_idx + (int64_t)bh * npad;
     int32_t* frow = far_idx + (int64_t)bh * F;
-    // fixed slots: sinks, window, headroom
-    for (int i = tid; i < npad; i += kPartThreads) {
-        if (i < tb.n_sinks) nrow[i] = i;
-        else if (i >= tb.n_sinks + k && i < tb.r_actual) nrow[i] = S - tb.window + (i - tb.n_sinks - k);
-        else if (i >= tb.r_actual) nrow[i] = -1;
-    }
+    fixed_slots(nrow, S, tb, tid);
     const bool all = k >= mlen, none = k <= 0;
     uint64_t thr = 0;  // near <=> rank key >= thr
     if (!all && !none) {
@@ -550,8 +701,15 @@ extern "C" int fkv_partition_importance(const fkv_tier_config* cfg, const float*
     if (int rc = fkv_tier_boundaries(cfg, S, &tb)) return rc;
     if ((S > 0 && !importance) || !near_idx || (tb.far_count > 0 && !far_idx))
         return set_error("fkv_partition_importance: NULL argument");
-    hipLaunchKernelGGL(fkv::partition_kernel, dim3((unsigned)(B * H)), dim3(fkv::kPartThreads), 0,
-                       (hipStream_t)stream, importance, S, tb, near_idx, far_idx);
+    // tokens per thread: the smallest compiled count that holds the middle
+    // (a larger one only adds empty registers to every pass)
+    const int64_t per = fkv::cdiv(tb.mid_end - tb.mid_start, fkv::kPartThreads);
+    auto* kern = per <= 4    ? fkv::partition_regs_kernel<4>
+                 : per <= 16 ? fkv::partition_regs_kernel<16>
+                 : per <= fkv::kPartRegs ? fkv::partition_regs_kernel<fkv::kPartRegs>
+                                         : fkv::partition_kernel;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(B * H)), dim3(fkv::kPartThreads), 0, (hipStream_t)stream, importance, S,
+                       tb, near_idx, far_idx);
     return fkv::check_hip(hipGetLastError(), "partition_kernel launch");
 }
 

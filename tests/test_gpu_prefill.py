@@ -56,3 +56,31 @@ def test_k_scale_reduction_edges(fkv, B, H, D, S, near_pct):
         cl = ext.CompressHandle(cfg).compress_layer(kk, kk, with_archive=False)
         want = np.full((B, H), np.float32(77.0) / np.float32(240.0), np.float32)
         assert np.array_equal(cl.far_k_scale.cpu().numpy(), want)
+
+
+# the edges of the tokens a thread holds (4, 16, 64 per thread of 1,024),
+# the first middle past them, and one whose last wave is partly empty
+@pytest.mark.parametrize("mid", [1, 63, 65, 4096, 4097, 16384, 16385, 50001, 65536, 65537])
+@pytest.mark.parametrize("kind", ["normal", "ties", "equal", "special"])
+def test_partition_size_edges(orc, fkv, mid, kind):
+    from foveated_kv_amd import ext
+
+    S = mid + 36
+    rng = np.random.default_rng(mid)
+    imp = rng.standard_normal((1, 2, S)).astype(np.float32)
+    if kind == "ties":
+        imp = rng.integers(-1, 2, imp.shape).astype(np.float32)
+    elif kind == "equal":
+        imp[:] = 3.25
+    elif kind == "special":
+        imp.reshape(-1)[rng.integers(0, imp.size, imp.size // 3)] = np.nan
+        imp.reshape(-1)[rng.integers(0, imp.size, imp.size // 9)] = -np.inf
+        imp.reshape(-1)[rng.integers(0, imp.size, imp.size // 9)] = np.finfo(np.float32).min
+        imp.reshape(-1)[rng.integers(0, imp.size, imp.size // 9)] = -0.0
+    for pct in (0.1, 0.9):
+        flush(f"partition mid={mid} {kind} near_pct={pct}")
+        near, far = ext.partition_importance(_cfg(near_pct=pct), torch.from_numpy(imp).cuda(), 1, 2, S)
+        torch.cuda.synchronize()
+        wn, wf, _ = orc.partition_importance(imp, S, 1, 2, promo_headroom_min=8, near_pct=pct)
+        assert np.array_equal(near.cpu().numpy(), wn)
+        assert np.array_equal(far.cpu().numpy(), wf)
