@@ -43,102 +43,141 @@ struct CompressArgs {
     const float* kscale;
 };
 
-__device__ inline uint8_t encode_e4m3(uint16_t bits) {
-    const uint32_t sign = (uint32_t)(bits >> 15) << 7;
-    const int ex = (bits >> 10) & 0x1f;
-    const uint32_t man = bits & 0x3ffu;
-    if (ex == 0) return (uint8_t)sign;
-    if (ex == 31) return (uint8_t)(sign | 0x7eu);
-    int e8 = ex - 8;
-    if (e8 >= 15) return (uint8_t)(sign | 0x7eu);
-    if (e8 <= 0) return (uint8_t)sign;
-    uint32_t m3 = man >> 7;
-    const bool up = ((man >> 6) & 1u) && ((man & 0x3fu) || (m3 & 1u));
-    if (up) {
-        m3++;
-        if (m3 == 8) {
-            m3 = 0;
-            e8++;
-            if (e8 >= 15) return (uint8_t)(sign | 0x7eu);
-        }
-    }
-    return (uint8_t)(sign | ((uint32_t)e8 << 3) | m3);
+// Packed-half integer operations (two fp16 bit patterns per dword).
+typedef uint16_t fkv_us2 __attribute__((ext_vector_type(2)));
+typedef short fkv_s2 __attribute__((ext_vector_type(2)));
+__device__ inline fkv_us2 as_us2(uint32_t w) { return __builtin_bit_cast(fkv_us2, w); }
+
+// The reference's encoder on eight fp16 values (four dwords of two) with the
+// hardware's converter, which rounds to nearest even as well but keeps
+// subnormal codes and the values 256..448: magnitudes below 2^-6 (0x2400)
+// become zero first, infinities, NaN and magnitudes above 448 (0x5F00)
+// become 448, and afterwards every code of exponent 15 -- whatever reached
+// 256, before rounding or by it -- becomes 0x7E.  About six instructions per
+// value; bit tests and selects on each value took twenty, which bound the
+// long-context compress with every option (see far_row).
+__device__ inline uint32_t e4m3_flush_clamp(uint32_t w) {
+    const fkv_us2 m = as_us2(w & 0x7FFF7FFFu);
+    const fkv_us2 one = {1, 1}, top = {0x5F00, 0x5F00}, low = {0x23FF, 0x23FF};
+    const fkv_us2 keep = -__builtin_elementwise_min(__builtin_elementwise_sub_sat(m, low), one);  // 0xFFFF from 2^-6 on
+    const uint32_t c = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(m, top) & keep);
+    return c | (w & 0x80008000u);
+}
+__device__ inline uint32_t encode_e4m3x4(uint32_t w0, uint32_t w1) {
+    const fkv_s2 none = {0, 0};
+    fkv_s2 c = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(none, as_h2(e4m3_flush_clamp(w0)), 1.0f, false);
+    c = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(c, as_h2(e4m3_flush_clamp(w1)), 1.0f, true);
+    const uint32_t codes = __builtin_bit_cast(uint32_t, c);
+    const uint32_t t = ((codes & 0x78787878u) + 0x08080808u) & 0x80808080u;  // exponent 15
+    const uint32_t mask = t - (t >> 7);                                     // 0x7F there
+    return (codes & ~mask) | (mask & 0x7E7E7E7Eu);
 }
 
-// 8 consecutive elements as fp16 bits (astype(float16) semantics: RNE)
-__device__ inline void load8(const void* base, int dtype, int64_t elem, uint16_t (&o)[8]) {
-    if (dtype == FKV_F16) {
+// 8 consecutive elements as packed fp16 bits (astype(float16) semantics: RNE)
+__device__ inline uint4 load8(const void* base, int dtype, int64_t elem) {
+    if (dtype == FKV_F16) return *(const uint4*)((const uint16_t*)base + elem);
+    auto pk = [](float a, float b) { return (uint32_t)f2h(a) | ((uint32_t)f2h(b) << 16); };
+    if (dtype == FKV_BF16) {
         const uint4 w = *(const uint4*)((const uint16_t*)base + elem);
-        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            o[2 * i] = (uint16_t)(ws[i] & 0xffff);
-            o[2 * i + 1] = (uint16_t)(ws[i] >> 16);
-        }
-    } else if (dtype == FKV_BF16) {
-        const uint4 w = *(const uint4*)((const uint16_t*)base + elem);
-        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            o[2 * i] = f2h(bf2f((uint16_t)(ws[i] & 0xffff)));
-            o[2 * i + 1] = f2h(bf2f((uint16_t)(ws[i] >> 16)));
-        }
-    } else {
-        const float4* p = (const float4*)((const float*)base + elem);
-        const float4 a = p[0], b = p[1];
-        const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) o[i] = f2h(f[i]);
+        auto two = [&](uint32_t u) { return pk(__uint_as_float(u << 16), __uint_as_float(u & 0xFFFF0000u)); };
+        return make_uint4(two(w.x), two(w.y), two(w.z), two(w.w));
     }
+    const float4* p = (const float4*)((const float*)base + elem);
+    const float4 a = p[0], b = p[1];
+    return make_uint4(pk(a.x, a.y), pk(a.z, a.w), pk(b.x, b.y), pk(b.z, b.w));
 }
 
-__device__ inline uint4 pack8(const uint16_t (&x)[8]) {
-    return make_uint4(x[0] | ((uint32_t)x[1] << 16), x[2] | ((uint32_t)x[3] << 16),
-                      x[4] | ((uint32_t)x[5] << 16), x[6] | ((uint32_t)x[7] << 16));
+// a / b rounded to nearest even, from y = 1.0f / b (so rounded itself):
+// Markstein's correction of a * y.  One step gives the correctly rounded
+// quotient where a * y is within one unit in the last place; a second one
+// (STEPS = 2) holds for any rounding of a * y.  A non-finite b gives NaN
+// where the division gives 0 or NaN.
+template <int STEPS>
+__device__ inline float div_by(float a, float b, float y) {
+    float q = a * y;
+#pragma unroll
+    for (int i = 0; i < STEPS; i++) q = fmaf(fmaf(-b, q, a), y, q);
+    return q;
+}
+
+// The fp16 value a key is encoded from with a per-head scale: fp16(key /
+// scale), fp32 division rounded to nearest even.  One correction step is
+// enough for every fp16 key and every scale that is an fp16 amax over 240
+// (all pairs checked) but turns -0 into +0, so the sign is the key's;
+// infinities and NaN, which the scale leaves out, go to the encoder as they
+// are.
+__device__ inline uint32_t scaled_keys(uint32_t w, float scale, float rscale) {
+    const uint16_t lo = (uint16_t)w, hi = (uint16_t)(w >> 16);
+    const uint16_t ql = f2h(div_by<1>(h2f(lo), scale, rscale)), qh = f2h(div_by<1>(h2f(hi), scale, rscale));
+    const uint32_t q = ((lo & 0x7C00u) == 0x7C00u ? lo : ql) | ((uint32_t)((hi & 0x7C00u) == 0x7C00u ? hi : qh) << 16);
+    return (q & 0x7FFF7FFFu) | (w & 0x80008000u);
+}
+
+// Minimum and maximum over the RL lanes (4, 8 or 16, aligned) of a row by DPP: lane
+// pairs, quads, then the mirrored halves of 8 and of 16 lanes.
+template <int CTRL>
+__device__ inline float dpp_f32(float v) {
+    const int i = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, true));
+}
+template <int RL>
+__device__ inline void row_minmax(float& mn, float& mx) {
+    static_assert(RL == 4 || RL == 8 || RL == 16, "rows of 4, 8 or 16 lanes");
+    mn = fminf(mn, dpp_f32<0xB1>(mn));  // quad_perm 1,0,3,2
+    mx = fmaxf(mx, dpp_f32<0xB1>(mx));
+    mn = fminf(mn, dpp_f32<0x4E>(mn));  // quad_perm 2,3,0,1
+    mx = fmaxf(mx, dpp_f32<0x4E>(mx));
+    if (RL >= 8) {
+        mn = fminf(mn, dpp_f32<0x141>(mn));  // row_half_mirror
+        mx = fmaxf(mx, dpp_f32<0x141>(mx));
+    }
+    if (RL >= 16) {
+        mn = fminf(mn, dpp_f32<0x140>(mn));  // row_mirror
+        mx = fmaxf(mx, dpp_f32<0x140>(mx));
+    }
 }
 
 // One far row (fr = bh * F + f) from its fp16 K / V (8 elements per lane):
 // E4M3 keys, INT4 values per token (VG = 0) or per VG-dim group, archive.
-// The fp16 value a key is encoded from: the key itself, or with a per-head
-// scale fp16(key / scale) (fp32 division, rounded to nearest even).
-__device__ inline uint16_t scaled_key(uint16_t k, const float* kscale, int bh) {
-    return kscale ? f2h(h2f(k) / kscale[bh]) : k;
-}
-
+// Meant to be bound by memory; the arithmetic per value is kept to what that
+// leaves room for (one division per row and lane instead of one per value,
+// the converter for the keys, lane reductions by DPP instead of LDS
+// permutes): the 64K x 8 head layer from bf16 with key scales and group-32
+// values took 191 us without (3.4 TB/s), 124 us now (5.3 TB/s); the 8 x 8 x
+// 16K fp16 layer was at the memory's rate before (219 us) and still is (218).
 template <int D, int VG>
-__device__ inline void far_row(const CompressArgs& a, int64_t fr, int sub, const uint16_t (&kx)[8],
-                               const uint16_t (&vx)[8]) {
+__device__ inline void far_row(const CompressArgs& a, int bh, int64_t fr, int sub, uint4 kw, uint4 vw) {
     constexpr int LPR = D / 8;
+    if (a.arc_k) *(uint4*)(a.arc_k + fr * D + sub * 8) = kw;
+    if (a.arc_v) *(uint4*)(a.arc_v + fr * D + sub * 8) = vw;
     // far K: E4M3 codes
-    const int bh = a.tb.far_count > 0 ? (int)(fr / a.tb.far_count) : 0;
-    uint32_t c0 = 0, c1 = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        c0 |= (uint32_t)encode_e4m3(scaled_key(kx[i], a.kscale, bh)) << (8 * i);
-        c1 |= (uint32_t)encode_e4m3(scaled_key(kx[4 + i], a.kscale, bh)) << (8 * i);
+    if (a.kscale) {
+        const float scale = a.kscale[bh], rscale = 1.0f / scale;
+        kw = make_uint4(scaled_keys(kw.x, scale, rscale), scaled_keys(kw.y, scale, rscale),
+                        scaled_keys(kw.z, scale, rscale), scaled_keys(kw.w, scale, rscale));
     }
-    *(uint2*)(a.far_k + fr * D + sub * 8) = make_uint2(c0, c1);
+    *(uint2*)(a.far_k + fr * D + sub * 8) = make_uint2(encode_e4m3x4(kw.x, kw.y), encode_e4m3x4(kw.z, kw.w));
     // far V: INT4 per token (VG = 0) or per 32-dim group
     constexpr int RL = VG ? VG / 8 : LPR;  // lanes of one quantisation row
+    const uint32_t vs[4] = {vw.x, vw.y, vw.z, vw.w};
     float vf[8];
     float mn = INFINITY, mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        vf[i] = h2f(vx[i]);
+        vf[i] = h2f((uint16_t)(vs[i / 2] >> (16 * (i & 1))));
         mn = fminf(mn, vf[i]);
         mx = fmaxf(mx, vf[i]);
     }
-#pragma unroll
-    for (int o = RL / 2; o >= 1; o >>= 1) {
-        mn = fminf(mn, __shfl_xor(mn, o, LPR));
-        mx = fmaxf(mx, __shfl_xor(mx, o, LPR));
-    }
-    const float scale = fmaxf((mx - mn) / 15.0f, 1e-8f);
+    row_minmax<RL>(mn, mx);
+    const float scale = fmaxf((mx - mn) / 15.0f, 1e-8f), rscale = 1.0f / scale;
     uint32_t packed = 0;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const float q = fminf(fmaxf(roundf((vf[i] - mn) / scale), 0.0f), 15.0f);
-        packed |= (uint32_t)q << (4 * i);
+        // round half away from zero of a quotient >= 0, clamped to 15 (NaN: 0)
+        const float q = div_by<2>(vf[i] - mn, scale, rscale);
+        uint32_t c = (uint32_t)fminf(fmaxf(q, 0.0f), 15.0f);
+        c += q - (float)c >= 0.5f ? 1u : 0u;
+        packed |= min(c, 15u) << (4 * i);
     }
     *(uint32_t*)(a.far_v + fr * (D / 2) + sub * 4) = packed;
     if (sub % RL == 0) {
@@ -146,8 +185,6 @@ __device__ inline void far_row(const CompressArgs& a, int64_t fr, int sub, const
         a.fvs[si] = f2h(scale);
         a.fvz[si] = f2h(mn);
     }
-    if (a.arc_k) *(uint4*)(a.arc_k + fr * D + sub * 8) = pack8(kx);
-    if (a.arc_v) *(uint4*)(a.arc_v + fr * D + sub * 8) = pack8(vx);
 }
 
 // VG = 0: one INT4 scale / zero per token (the reference); VG = 32: one per
@@ -179,17 +216,15 @@ __global__ __launch_bounds__(256) void compress_kernel(CompressArgs a) {
     else if (t >= tb.mid_start && t < tb.near_mid_start) f = t - tb.mid_start;
 
     const int64_t src = ((int64_t)bh * a.S + t) * D + sub * 8;
-    uint16_t kx[8], vx[8];
-    load8(a.k, a.dtype, src, kx);
-    load8(a.v, a.dtype, src, vx);
+    const uint4 kw = load8(a.k, a.dtype, src), vw = load8(a.v, a.dtype, src);
     if (slot >= 0) {
         const int64_t o = ((int64_t)bh * npad + slot) * D + sub * 8;
-        *(uint4*)(a.near_k + o) = pack8(kx);
-        *(uint4*)(a.near_v + o) = pack8(vx);
+        *(uint4*)(a.near_k + o) = kw;
+        *(uint4*)(a.near_v + o) = vw;
         return;
     }
     if (f < 0) return;  // unreachable: every position is near or far
-    far_row<D, VG>(a, (int64_t)bh * F + f, sub, kx, vx);
+    far_row<D, VG>(a, bh, (int64_t)bh * F + f, sub, kw, vw);
 }
 
 
@@ -241,19 +276,23 @@ __global__ __launch_bounds__(kScaleThreads) void kscale_kernel(CompressArgs a, c
             const int64_t f = f0 + u * RPB;
             t[u] = f >= F ? -1 : far_idx ? far_idx[(int64_t)bh * F + f] : a.tb.mid_start + (int)f;
         }
-        uint16_t kx[kScaleRows][8];
+        uint4 kx[kScaleRows];
 #pragma unroll
         for (int u = 0; u < kScaleRows; u++) {
             const bool in = t[u] >= 0 && t[u] < a.S;
             // a row outside the sequence reads row 0 and is left out below
-            load8(a.k, a.dtype, ((int64_t)bh * a.S + (in ? t[u] : 0)) * D + sub * 8, kx[u]);
+            kx[u] = load8(a.k, a.dtype, ((int64_t)bh * a.S + (in ? t[u] : 0)) * D + sub * 8);
         }
 #pragma unroll
         for (int u = 0; u < kScaleRows; u++)
-            if (t[u] >= 0 && t[u] < a.S)
+            if (t[u] >= 0 && t[u] < a.S) {
+                const uint32_t w[4] = {kx[u].x, kx[u].y, kx[u].z, kx[u].w};
 #pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (((kx[u][i] >> 10) & 0x1f) != 0x1f) amax = fmaxf(amax, fabsf(h2f(kx[u][i])));
+                for (int i = 0; i < 8; i++) {
+                    const uint16_t h = (uint16_t)(w[i / 2] >> (16 * (i & 1)));
+                    if (((h >> 10) & 0x1f) != 0x1f) amax = fmaxf(amax, fabsf(h2f(h)));
+                }
+            }
     }
     amax = wave_max(amax);
     if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = amax;
@@ -575,23 +614,23 @@ __global__ __launch_bounds__(256) void compress_gather_kernel(CompressArgs a, co
     const int npad = tb.n_near_padded;
     const int F = tb.far_count;
     if (r >= npad + F) return;  // whole row group leaves together
-    uint16_t kx[8] = {0, 0, 0, 0, 0, 0, 0, 0}, vx[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    uint4 kw = make_uint4(0, 0, 0, 0), vw = kw;
     const bool near = r < npad;
     int t = -1;
     if (near) t = r < tb.r_actual ? near_idx[(int64_t)bh * npad + r] : -1;
     else t = far_idx[(int64_t)bh * F + (r - npad)];
     if (t >= 0 && t < a.S) {
         const int64_t src = ((int64_t)bh * a.S + t) * D + sub * 8;
-        load8(a.k, a.dtype, src, kx);
-        load8(a.v, a.dtype, src, vx);
+        kw = load8(a.k, a.dtype, src);
+        vw = load8(a.v, a.dtype, src);
     }
     if (near) {
         const int64_t o = ((int64_t)bh * npad + r) * D + sub * 8;
-        *(uint4*)(a.near_k + o) = pack8(kx);
-        *(uint4*)(a.near_v + o) = pack8(vx);
+        *(uint4*)(a.near_k + o) = kw;
+        *(uint4*)(a.near_v + o) = vw;
         return;
     }
-    far_row<D, VG>(a, (int64_t)bh * F + (r - npad), sub, kx, vx);
+    far_row<D, VG>(a, bh, (int64_t)bh * F + (r - npad), sub, kw, vw);
 }
 
 }  // namespace fkv

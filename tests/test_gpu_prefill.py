@@ -84,3 +84,60 @@ def test_partition_size_edges(orc, fkv, mid, kind):
         wn, wf, _ = orc.partition_importance(imp, S, 1, 2, promo_headroom_min=8, near_pct=pct)
         assert np.array_equal(near.cpu().numpy(), wn)
         assert np.array_equal(far.cpu().numpy(), wf)
+
+
+def _int4_numpy(v, group):
+    """The INT4 quantiser on fp16 rows, fp32 as the format defines it
+    (foveated_compress.metal:153-205): NaN ignored by the extrema and coded 0."""
+    f = v.astype(np.float32).reshape(v.shape[:-1] + (-1, group))
+    with np.errstate(all="ignore"):
+        # the extrema start from +inf / -inf: what a row of NaN keeps
+        mn = np.fmin.reduce(f, -1, keepdims=True, initial=np.inf)
+        mx = np.fmax.reduce(f, -1, keepdims=True, initial=-np.inf)
+        scale = np.fmax((mx - mn) / np.float32(15), np.float32(1e-8))
+        q = (f - mn) / scale
+        code = np.fmin(np.fmax(np.trunc(q) + (q - np.trunc(q) >= 0.5), 0), 15)
+    code = np.nan_to_num(code).astype(np.uint8).reshape(v.shape)
+    return code[..., 0::2] | (code[..., 1::2] << 4), scale[..., 0].astype(np.float16), mn[..., 0].astype(np.float16)
+
+
+@pytest.mark.parametrize("D,vg", [(64, 0), (128, 0), (64, 32), (128, 32)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32])
+@pytest.mark.parametrize("importance", [False, True])
+def test_far_rows_special_values(fkv, D, vg, dt, importance):
+    """Far rows with infinities, NaN, -0, subnormals, constant rows and exact
+    ties, with and without key scales: codes as the formats define them."""
+    from foveated_kv_amd import ext
+
+    H, S = 2, 700
+    rng = np.random.default_rng(D + vg)
+    x = rng.standard_normal((1, H, S, D)).astype(np.float16)
+    x[0, 0, 40:60] = rng.integers(-15, 16, (20, D))     # ties: half-integer quotients
+    x[0, 0, 60:70] *= np.float16(2.0 ** -20)            # subnormal rows
+    x[0, 0, 70:75] = 3.5                                # constant rows
+    x[0, 0, 75, :8] = [-0.0, 0.0, 2.0 ** -24, -2.0 ** -24, 65504, -65504, 247.9, 248]
+    x[0, 1, 40:100, 3] = np.nan
+    x[0, 1, 50:60, 5] = np.inf
+    x[0, 1, 60:70, 7] = -np.inf
+    x[0, 1, 70] = np.nan
+    x[0, 1, 71] = np.inf
+    t = torch.from_numpy(x).cuda().to(dt)
+    imp = torch.arange(S, dtype=torch.float32, device="cuda") if importance else None
+    for ks in (0, 1):
+        flush(f"special values D={D} v_group={vg} {dt} importance={importance} k_scale={ks}")
+        cl = ext.CompressHandle(_cfg(v_group=vg, k_scale=ks)).compress_layer(t, t, importance=imp)
+        far = cl.archive_k.cpu().numpy()
+        m0 = 4
+        assert np.array_equal(far.view(np.uint16), x[:, :, m0:m0 + far.shape[2]].view(np.uint16))
+        codes, scale, zero = _int4_numpy(far, vg or D)
+        assert np.array_equal(cl.far_v.cpu().numpy(), codes)
+        gs, gz = cl.far_v_scale.cpu().numpy().reshape(scale.shape), cl.far_v_zero.cpu().numpy().reshape(zero.shape)
+        assert np.array_equal(gs, scale, equal_nan=True) and np.array_equal(gz, zero, equal_nan=True)
+        import oracle
+
+        if ks:
+            want = oracle.encode_fp8_scaled(far, oracle.k_head_scale(far))
+            assert np.array_equal(cl.far_k_scale.cpu().numpy(), oracle.k_head_scale(far))
+        else:
+            want = oracle.encode_fp8(far)
+        assert np.array_equal(cl.far_k.cpu().numpy(), want)
