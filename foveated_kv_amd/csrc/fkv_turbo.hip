@@ -114,7 +114,6 @@ __global__ void tq_pack_sn_kernel(const void* __restrict__ vscale, const void* _
     }
 }
 
-// out[j][i] = in[i][j] for a (D, D) fp32 matrix.
 // Pi and S -> the rotation MFMAs' fp16 operands (tq_rot_index).
 __global__ void rot_operand_kernel(const float* __restrict__ Pi, const float* __restrict__ S,
                                    uint16_t* __restrict__ rot, int D) {
@@ -126,15 +125,6 @@ __global__ void rot_operand_kernel(const float* __restrict__ Pi, const float* __
     }
 }
 
-__global__ void transpose_kernel(const float* __restrict__ in, float* __restrict__ out, int D) {
-    const int64_t n = (int64_t)D * D;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / D), c = (int)(i % D);
-        out[(int64_t)c * D + r] = in[i];
-    }
-}
-
 // ---------------------------------------------------------------------------
 // per-call query preparation (csrc/foveated_attn.cpp:415-421)
 // ---------------------------------------------------------------------------
@@ -142,112 +132,377 @@ __global__ void transpose_kernel(const float* __restrict__ in, float* __restrict
 // ---------------------------------------------------------------------------
 // compression (src/foveated_kv/turbo_quantize.py:25-91, 139-178), fp32
 // ---------------------------------------------------------------------------
-
-constexpr int kTqTok = 32;  // tokens per workgroup of the key compressor
-
-// One workgroup (256 threads) per 32 tokens.  Thread (dim i, token group)
-// accumulates 32 / (256 / D) tokens' outputs for dim i; the matrix rows are
-// read once per workgroup (coalesced across i), the token rows from LDS.
+//
 //   n = |k|; y = (k / max(n, 1e-8)) Pi^T; idx = [y >= b0] + [y >= b1] + [y >= b2]
 //   r = k - n * (cb[idx] Pi); gamma = |r|; sign = (r S^T >= 0)
-template <int D>
-__global__ __launch_bounds__(256) void tq_compress_keys_kernel(const void* __restrict__ keys, int dtype, int64_t n_tok,
-                                                               const float* __restrict__ PiT,
-                                                               const float* __restrict__ Pi,
-                                                               const float* __restrict__ ST, float4 cbv, float4 bdv,
-                                                               uint8_t* __restrict__ out_idx,
-                                                               uint8_t* __restrict__ out_sgn,
-                                                               uint16_t* __restrict__ out_norm,
-                                                               uint16_t* __restrict__ out_gamma) {
-    constexpr int TG = 256 / D, TPT = kTqTok / TG;  // token groups, tokens per thread
-    __shared__ float kf[kTqTok][D];   // k, later r
-    __shared__ float kn[kTqTok][D];   // k / max(n, 1e-8), later cb[idx]
-    __shared__ uint8_t codes[kTqTok][D];
-    __shared__ float nrm[kTqTok], gam[kTqTok];
-    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const int i = tid % D, tg = tid / D;
-    const int64_t t0 = (int64_t)blockIdx.x * kTqTok;
-    const float cb[4] = {cbv.x, cbv.y, cbv.z, cbv.w};
-    for (int e = tid; e < kTqTok * D; e += 256) {
-        const int tt = e / D, d = e % D;
-        const int64_t t = t0 + tt;
-        kf[tt][d] = t < n_tok ? h2f(load_as_f16(keys, t * D + d, dtype)) : 0.f;
-    }
-    __syncthreads();
-    for (int tt = wave; tt < kTqTok; tt += 4) {
-        float ss = 0.f;
-        for (int d = lane; d < D; d += 64) ss += kf[tt][d] * kf[tt][d];
-        ss = wave_sum(ss);
-        if (lane == 0) nrm[tt] = sqrtf(ss);
-    }
-    __syncthreads();
-    for (int e = tid; e < kTqTok * D; e += 256) {
-        const int tt = e / D, d = e % D;
-        kn[tt][d] = kf[tt][d] / fmaxf(nrm[tt], 1e-8f);
-    }
-    __syncthreads();
-    float acc[TPT];
-#pragma unroll
-    for (int u = 0; u < TPT; u++) acc[u] = 0.f;
-    for (int j = 0; j < D; j++) {
-        const float m = PiT[j * D + i];
-#pragma unroll
-        for (int u = 0; u < TPT; u++) acc[u] = fmaf(kn[tg * TPT + u][j], m, acc[u]);
-    }
-    __syncthreads();  // every y is computed: kn may be overwritten with the centroids
-#pragma unroll
-    for (int u = 0; u < TPT; u++) {
-        const float y = acc[u];
-        const int c = (y >= bdv.x) + (y >= bdv.y) + (y >= bdv.z);
-        codes[tg * TPT + u][i] = (uint8_t)c;
-        kn[tg * TPT + u][i] = cb[c];
-        acc[u] = 0.f;
-    }
-    __syncthreads();
-    for (int j = 0; j < D; j++) {  // (cb[idx] Pi)_i = sum_j cb[idx_j] Pi[j][i]
-        const float m = Pi[j * D + i];
-#pragma unroll
-        for (int u = 0; u < TPT; u++) acc[u] = fmaf(kn[tg * TPT + u][j], m, acc[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < TPT; u++) {
-        const int tt = tg * TPT + u;
-        kf[tt][i] = kf[tt][i] - nrm[tt] * acc[u];  // residual
-        acc[u] = 0.f;
-    }
-    __syncthreads();
-    for (int tt = wave; tt < kTqTok; tt += 4) {
-        float ss = 0.f;
-        for (int d = lane; d < D; d += 64) ss += kf[tt][d] * kf[tt][d];
-        ss = wave_sum(ss);
-        if (lane == 0) gam[tt] = sqrtf(ss);
-    }
-    for (int j = 0; j < D; j++) {  // (r S^T)_i = sum_j r_j ST[j][i]
-        const float m = ST[j * D + i];
-#pragma unroll
-        for (int u = 0; u < TPT; u++) acc[u] = fmaf(kf[tg * TPT + u][j], m, acc[u]);
-    }
-    __syncthreads();  // residual reads done, gamma written
-#pragma unroll
-    for (int u = 0; u < TPT; u++) kn[tg * TPT + u][i] = acc[u] >= 0.f ? 1.f : 0.f;
-    __syncthreads();
-    for (int e = tid; e < kTqTok * (D / 4); e += 256) {
-        const int tt = e / (D / 4), by = e % (D / 4);
-        const int64_t t = t0 + tt;
-        if (t >= n_tok) continue;
-        const uint8_t* c = &codes[tt][4 * by];
-        out_idx[t * (D / 4) + by] = (uint8_t)(c[0] | (c[1] << 2) | (c[2] << 4) | (c[3] << 6));
-        if (by < D / 8) {
-            uint32_t b = 0;
-            for (int k = 0; k < 8; k++) b |= (kn[tt][8 * by + k] != 0.f ? 1u : 0u) << k;
-            out_sgn[t * (D / 8) + by] = (uint8_t)b;
+//
+// Three D x D products per token, all on the matrix cores
+// (v_mfma_f32_32x32x16_f16) at fp32 precision: every fp32 operand is split
+// into fp16 hi + lo / 2048 after a power-of-two scale that puts its row's
+// (token's) largest value near 1, the keys are fp16 already, products of
+// fp16 values are exact and summed in fp32, and the lo products run first
+// in the same accumulators, which are scaled by 1 / 2048 before the hi ones
+// (lo x lo, below 2^-24, is left out).  Against 64 bits over N(0, 1) keys
+// with outlier channels, 60 x 262,112 tokens: 99 codes and 201 signs off of
+// 2.0e9 at D = 128 (207 and 338 with fp32 FMA chains), 42 and 104 of 1.0e9
+// at D = 64 (70 and 125).
+// The matrix is the A operand (rows = output dims) and the tokens are the B
+// operand (columns), so a lane's accumulators hold its own token's output
+// dims 32 rb + 8 a + 4 (lane / 32) + b; every product's K slots are numbered
+// in that order too, so one product's results are the next one's B operand
+// without leaving the lane's registers.
+
+typedef _Float16 fkv_h8 __attribute__((ext_vector_type(8)));
+typedef float fkv_f16v __attribute__((ext_vector_type(16)));
+
+constexpr int kTqTok = 128;  // tokens per workgroup of the key compressor (32 per wave)
+constexpr float kTqLo = 2048.0f;
+
+// The key compressor's prepared constants: per product (Pi, Pi^T, S) the lo
+// and the hi operand, [part][row block][K step][lane][8 halves]; the inverse
+// row scales of the first two products (the second times the centroids'
+// inverse scale); the boundaries ascending; the codes' centroids as hi | lo << 16.
+__host__ __device__ constexpr size_t tq_op_bytes(int D) { return (size_t)4 * D * D; }
+__host__ __device__ constexpr size_t tq_scale_section(int D) { return 3 * tq_op_bytes(D); }
+__host__ __device__ constexpr size_t tq_const_section(int D) { return tq_scale_section(D) + (size_t)8 * D; }
+__host__ __device__ constexpr size_t tq_prep_bytes(int D) { return tq_const_section(D) + 32; }
+
+// Power of two that brings |x| <= m near 1, and its inverse.
+__device__ inline float pow2_scale(float m, float& inv) {
+    const int e = min((int)((__float_as_uint(m) >> 23) & 0xFF), 253);
+    inv = e ? __uint_as_float((uint32_t)e << 23) : 0x1p-127f;
+    return m < INFINITY ? __uint_as_float((uint32_t)(254 - e) << 23) : (inv = 1.0f);
+}
+__device__ inline void split_half(float x, uint16_t& hi, uint16_t& lo) {
+    hi = f2h(x);
+    lo = f2h((x - h2f(hi)) * kTqLo);
+}
+
+// Blocks 0 .. 3 D - 1: one output row of one product (64 threads); the last
+// block: the scalar constants.
+__global__ __launch_bounds__(kWave) void tq_prep_kernel(const float* __restrict__ Pi, const float* __restrict__ S,
+                                                        const float* __restrict__ cb, const float* __restrict__ bd,
+                                                        int D, uint8_t* __restrict__ prep) {
+    const int lane = threadIdx.x;
+    float* const scales = (float*)(prep + tq_scale_section(D));
+    float cinv;
+    const float cscale =
+        pow2_scale(fmaxf(fmaxf(fabsf(cb[0]), fabsf(cb[1])), fmaxf(fabsf(cb[2]), fabsf(cb[3]))), cinv);
+    if (blockIdx.x == 3 * D) {
+        if (lane != 0) return;
+        // ascending (the code counts the boundaries at or below y); NaN, which none reaches, last
+        float b[3];
+        for (int i = 0; i < 3; i++) b[i] = bd[i] == bd[i] ? bd[i] : INFINITY;
+        for (int i : {0, 1, 0})
+            if (b[i] > b[i + 1]) {
+                const float t = b[i];
+                b[i] = b[i + 1];
+                b[i + 1] = t;
+            }
+        float* const c = (float*)(prep + tq_const_section(D));
+        for (int i = 0; i < 3; i++) c[i] = b[i];
+        for (int i = 0; i < 4; i++) {
+            uint16_t hi, lo;
+            split_half(cb[i] * cscale, hi, lo);
+            ((uint32_t*)c)[4 + i] = (uint32_t)hi | ((uint32_t)lo << 16);
         }
-        if (by == 0) {
-            out_norm[t] = f2h(nrm[tt]);
-            out_gamma[t] = f2h(gam[tt]);
+        return;
+    }
+    const int op = blockIdx.x / D, i = blockIdx.x % D;
+    auto at = [&](int j) { return op == 1 ? Pi[(int64_t)j * D + i] : (op ? S : Pi)[(int64_t)i * D + j]; };
+    float m = 0.f;
+    for (int j = lane; j < D; j += kWave) m = fmaxf(m, fabsf(at(j)));
+    m = wave_max(m);
+    float inv;
+    const float scale = pow2_scale(m, inv);
+    if (op < 2 && lane == 0) scales[op * D + i] = op == 1 ? inv * cinv : inv;
+    uint16_t* const out = (uint16_t*)(prep + op * tq_op_bytes(D));
+    for (int j = lane; j < D; j += kWave) {
+        uint16_t hi, lo;
+        split_half(at(j) * scale, hi, lo);
+        // K step j / 16, lane half (j % 8) / 4, slot 4 ((j % 16) / 8) + j % 4
+        const int64_t o = ((int64_t)((i / 32) * (D / 16) + j / 16) * 64 + (i % 32) + 32 * ((j % 8) / 4)) * 8 +
+                          4 * ((j % 16) / 8) + j % 4;
+        out[o] = lo;
+        out[(int64_t)D * D + o] = hi;
+    }
+}
+
+template <int D>
+struct TqGemm {
+    static constexpr int NB = D / 32, NS = D / 16;
+    const uint8_t* op;  // the product's operands in LDS
+    int lane;
+    fkv_f16v acc[NB];
+    __device__ inline void clear() {
+#pragma unroll
+        for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[rb][i] = 0.f;
+    }
+    // acc += A_part B.  The next step's operands are read while this step's
+    // are multiplied, and the address is opaque, so that no pass keeps
+    // operands in registers for a later one (32 fragments of 4 VGPRs: spills).
+    __device__ inline void add(int part, const fkv_h8 (&b)[NS]) {
+        int o = part * (2 * D * D) + lane * 16;
+        asm volatile("" : "+v"(o));
+        const fkv_h8* f = (const fkv_h8*)(op + o);
+        fkv_h8 cur[NB], nxt[NB];
+#pragma unroll
+        for (int rb = 0; rb < NB; rb++) cur[rb] = f[rb * NS * 64];
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+#pragma unroll
+            for (int rb = 0; rb < NB; rb++)
+                if (s + 1 < NS) nxt[rb] = f[(rb * NS + s + 1) * 64];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int rb = 0; rb < NB; rb++)
+                acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur[rb], b[s], acc[rb], 0, 0, 0);
+#pragma unroll
+            for (int rb = 0; rb < NB; rb++) cur[rb] = nxt[rb];
+        }
+    }
+    __device__ inline void lo_done() {
+#pragma unroll
+        for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[rb][i] *= 1.0f / kTqLo;
+    }
+    // fp32-precision product with the split operand hi + lo / kTqLo
+    __device__ inline void split(const fkv_h8 (&hi)[NS], const fkv_h8 (&lo)[NS]) {
+        clear();
+        add(0, hi);
+        add(1, lo);
+        lo_done();
+        add(1, hi);
+    }
+};
+
+// Sum of eight partial sums of this lane and of lane ^ 32 (the token's other dims).
+__device__ inline float tq_half_sum(const float (&p)[8]) {
+    const float s = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    return s + __shfl_xor(s, 32);
+}
+
+// One workgroup of four waves per 128 tokens, two workgroups per CU (64 KB of
+// LDS each at D = 128): one's vector work overlaps the other's matrix work.
+// Each product's operands come to LDS by LDS DMA once the previous product
+// is done with them, while its results are turned into codes, residuals or
+// signs.  WIDE: keys and code buffers 16-byte aligned (else element loads
+// and byte stores).  Bound by issue: per 32 tokens of a wave 256 MFMAs (27 us
+// over 262K tokens at D = 128) and 2,300 vector instructions (31 us), and the
+// LDS reads of the operands (27 us).  4 x 8 heads x 8,191 tokens: 869 us with
+// fp32 FMA chains (30 TFLOP/s), 84 us now.
+template <int D, bool WIDE>
+__global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __restrict__ keys, int dtype, int64_t n_tok,
+                                                                  const uint8_t* __restrict__ prep,
+                                                                  uint8_t* __restrict__ out_idx,
+                                                                  uint8_t* __restrict__ out_sgn,
+                                                                  uint16_t* __restrict__ out_norm,
+                                                                  uint16_t* __restrict__ out_gamma) {
+    constexpr int NB = D / 32, NS = D / 16;
+    __shared__ __attribute__((aligned(16))) uint8_t op_s[tq_op_bytes(D)];
+    __shared__ __attribute__((aligned(16))) float sc_s[2 * D];
+    const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int h = lane >> 5;
+    const uint32_t upper = h ? ~0u : 0u;  // selects by mask (a select between array elements became an indexed access)
+    const int64_t t = (int64_t)blockIdx.x * kTqTok + wave * 32 + (lane & 31);
+    const bool live = t < n_tok;
+    auto fetch = [&](int op) __attribute__((always_inline)) {
+        constexpr int CH = (int)tq_op_bytes(D) / 1024 / 4;  // 1-KB chunks per wave
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const size_t o = (size_t)(wave * CH + c) * 1024;
+            __builtin_amdgcn_global_load_lds((const void*)(prep + op * tq_op_bytes(D) + o + lane * 16),
+                                             (__attribute__((address_space(3))) void*)(op_s + o), 16, 0, 0);
+        }
+    };
+    auto ready = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+    fetch(0);
+    for (int i = tid; i < 2 * D; i += 256) sc_s[i] = ((const float*)(prep + tq_scale_section(D)))[i];
+    const float* const cst = (const float*)(prep + tq_const_section(D));
+    float b0 = cst[0], b1 = cst[1], b2 = cst[2];
+    uint32_t cw[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) cw[i] = ((const uint32_t*)cst)[4 + i];
+    // the token's keys as the B operand: slots 0..3 of step s are dims 16 s +
+    // 4 h .., slots 4..7 dims 16 s + 8 + 4 h ..
+    fkv_h8 kb[NS];
+    if (WIDE && dtype != FKV_F32) {
+        // lane half h loads dims 16 s + 8 h .. + 7; the halves then exchange
+        // their outer four dims
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            uint4 w = make_uint4(0, 0, 0, 0);
+            if (live) w = *(const uint4*)((const uint16_t*)keys + t * D + 16 * s + 8 * h);
+            if (dtype == FKV_BF16) {
+                auto two = [](uint32_t u) {
+                    return (uint32_t)f2h(__uint_as_float(u << 16)) |
+                           ((uint32_t)f2h(__uint_as_float(u & 0xFFFF0000u)) << 16);
+                };
+                w = make_uint4(two(w.x), two(w.y), two(w.z), two(w.w));
+            }
+            // given to the other half: h = 0 its dims 4..7, h = 1 its dims 8..11
+            const uint32_t g0 = __shfl_xor(h ? w.x : w.z, 32), g1 = __shfl_xor(h ? w.y : w.w, 32);
+            const uint4 o = h ? make_uint4(g0, g1, w.z, w.w) : make_uint4(w.x, w.y, g0, g1);
+            kb[s] = __builtin_bit_cast(fkv_h8, o);
+        }
+    } else if (WIDE) {
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f), y = x;
+            if (live) {
+                x = *(const float4*)((const float*)keys + t * D + 16 * s + 4 * h);
+                y = *(const float4*)((const float*)keys + t * D + 16 * s + 8 + 4 * h);
+            }
+            kb[s] = fkv_h8{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w,
+                           (_Float16)y.x, (_Float16)y.y, (_Float16)y.z, (_Float16)y.w};
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                kb[s][e] = live ? __builtin_bit_cast(_Float16, load_as_f16(keys, t * D + 16 * s + 8 * (e / 4) + 4 * h + e % 4,
+                                                                           dtype))
+                                : (_Float16)0.f;
+    }
+    // eight partial sums, added pairwise: the norm's rounding moves every boundary
+    float ss[8] = {};
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) ss[e] = fmaf((float)kb[s][e], (float)kb[s][e], ss[e]);
+    const float nrm = sqrtf(tq_half_sum(ss));
+    {
+        // y >= b  <=>  k Pi^T >= b max(n, 1e-8); no code of a non-finite norm
+        const float nc = fmaxf(nrm, 1e-8f), nan = __uint_as_float(0x7FC00000u);
+        b0 = nc < INFINITY ? b0 * nc : nan;
+        b1 = nc < INFINITY ? b1 * nc : nan;
+        b2 = nc < INFINITY ? b2 * nc : nan;
+    }
+    TqGemm<D> g{op_s, lane, {}};
+    // ---- codes ----
+    ready();
+    g.clear();
+    g.add(0, kb);
+    g.lo_done();
+    g.add(1, kb);
+    __syncthreads();  // every wave is done with the operands
+    fetch(1);
+    fkv_h8 hi[NS], lo[NS];
+    uint32_t w[NB];
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++) {
+        w[rb] = 0;
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const float4 sc = *(const float4*)&sc_s[32 * rb + 8 * a + 4 * h];
+            const float f[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const float y = g.acc[rb][4 * a + b] * f[b];
+                const bool p0 = y >= b0, p1 = y >= b1, p2 = y >= b2;
+                uint32_t code = p2 ? 3u : p1 ? 2u : p0 ? 1u : 0u;
+                uint32_t c = p2 ? cw[3] : p1 ? cw[2] : p0 ? cw[1] : cw[0];
+                asm volatile("" : "+v"(code), "+v"(c));  // here, so that the masks end (they were spilled)
+                w[rb] |= code << (8 * a + 2 * b);
+                const int s = 2 * rb + a / 2, e = 4 * (a % 2) + b;
+                hi[s][e] = __builtin_bit_cast(_Float16, (uint16_t)c);
+                lo[s][e] = __builtin_bit_cast(_Float16, (uint16_t)(c >> 16));
+            }
+        }
+    }
+    // byte 8 rb + 2 a + h of the token's codes: dword pairs interleave the halves' bytes
+    uint32_t ix[2 * NB];
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++) {
+        const uint32_t o = __shfl_xor(w[rb], 32), w0 = h ? o : w[rb], w1 = h ? w[rb] : o;
+        ix[2 * rb] = __builtin_amdgcn_perm(w1, w0, 0x05010400u);
+        ix[2 * rb + 1] = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
+    }
+    if (live) {
+        uint8_t* const dst = out_idx + t * (D / 4) + h * (D / 8);  // each half writes half the token's bytes
+        uint32_t mine[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) mine[i] = (ix[i] & ~upper) | (ix[NB + i] & upper);
+        if (WIDE) {
+            if constexpr (NB == 4) *(uint4*)dst = make_uint4(mine[0], mine[1], mine[2], mine[3]);
+            else *(uint2*)dst = make_uint2(mine[0], mine[1]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4 * NB; i++) dst[i] = (uint8_t)(mine[i / 4] >> (8 * (i % 4)));
+        }
+    }
+    // ---- residual ----
+    ready();
+    g.split(hi, lo);
+    __syncthreads();
+    fetch(2);
+#pragma unroll
+    for (int e = 0; e < 8; e++) ss[e] = 0.f;
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const float4 sc = *(const float4*)&sc_s[D + 32 * rb + 8 * a + 4 * h];
+            const float f[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const int s = 2 * rb + a / 2, e = 4 * (a % 2) + b;
+                const float r = fmaf(-nrm, g.acc[rb][4 * a + b] * f[b], (float)kb[s][e]);
+                g.acc[rb][4 * a + b] = r;
+                ss[e] = fmaf(r, r, ss[e]);
+            }
+        }
+    const float gamma = sqrtf(tq_half_sum(ss));
+    if (live && h == 0) {
+        out_norm[t] = f2h(nrm);
+        out_gamma[t] = f2h(gamma);
+    }
+    // the residual scaled so that its largest value is at most 2 (only the
+    // sign of its projections is kept); a non-finite one gives no sign
+    const int ge = (int)((__float_as_uint(gamma) >> 23) & 0xFF);
+    const float rs = gamma < INFINITY ? __uint_as_float((uint32_t)(254 - min(ge, 253)) << 23) : 0.f;
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            uint16_t vh, vl;
+            split_half(g.acc[rb][i] * rs, vh, vl);
+            hi[2 * rb + i / 8][i % 8] = __builtin_bit_cast(_Float16, vh);
+            lo[2 * rb + i / 8][i % 8] = __builtin_bit_cast(_Float16, vl);
+        }
+    // ---- signs ----
+    ready();
+    g.split(hi, lo);
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++) {
+        w[rb] = 0;
+#pragma unroll
+        for (int i = 0; i < 16; i++) w[rb] |= (g.acc[rb][i] >= 0.f ? 1u : 0u) << (8 * (i / 4) + i % 4);
+        w[rb] <<= 4 * h;
+        w[rb] |= __shfl_xor(w[rb], 32);
+    }
+    if (live) {
+        uint8_t* const dst = out_sgn + t * (D / 8) + h * (D / 16);
+        uint32_t mine[NB / 2];
+#pragma unroll
+        for (int i = 0; i < NB / 2; i++) mine[i] = (w[i] & ~upper) | (w[NB / 2 + i] & upper);
+        if (WIDE) {
+            if constexpr (NB == 4) *(uint2*)dst = make_uint2(mine[0], mine[1]);
+            else *(uint32_t*)dst = mine[0];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2 * NB; i++) dst[i] = (uint8_t)(mine[i / 4] >> (8 * (i % 4)));
         }
     }
 }
+
 
 // One thread per (token, 32-dim group): scale = max(max|v|, 1e-8), code =
 // clip(rint((v / scale + 1) * 1.5), 0, 3) (round half to even, as mx.round).
@@ -357,32 +612,20 @@ int fkv_turbo_compress_keys(const void* keys, int32_t dtype, int64_t n_tokens, i
     if (!keys || !Pi || !S || !centroids || !boundaries || !out_idx || !out_signs || !out_norm || !out_gamma)
         return set_error("fkv_turbo_compress_keys: NULL argument");
     hipStream_t st = (hipStream_t)stream;
-    float cbh[8];
-    int rc = check_hip(hipMemcpyAsync(cbh, centroids, 4 * sizeof(float), hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
-    if (!rc) rc = check_hip(hipMemcpyAsync(cbh + 4, boundaries, 3 * sizeof(float), hipMemcpyDeviceToHost, st),
-                            "hipMemcpyAsync");
-    if (!rc) rc = check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
-    float* PiT = nullptr;
-    float* ST = nullptr;
-    const size_t mat = (size_t)D * D * sizeof(float);
-    if (!rc) rc = check_hip(hipMallocAsync((void**)&PiT, mat, st), "hipMallocAsync");
-    if (!rc) rc = check_hip(hipMallocAsync((void**)&ST, mat, st), "hipMallocAsync");
-    if (!rc) {
-        hipLaunchKernelGGL(fkv::transpose_kernel, dim3(fkv::grid_for((int64_t)D * D, 256)), dim3(256), 0, st, Pi, PiT, D);
-        hipLaunchKernelGGL(fkv::transpose_kernel, dim3(fkv::grid_for((int64_t)D * D, 256)), dim3(256), 0, st, S, ST, D);
-        const float4 cbv = make_float4(cbh[0], cbh[1], cbh[2], cbh[3]);
-        const float4 bdv = make_float4(cbh[4], cbh[5], cbh[6], 0.f);
-        const dim3 grid((unsigned)fkv::cdiv(n_tokens, fkv::kTqTok));
-        if (D == 128)
-            hipLaunchKernelGGL(fkv::tq_compress_keys_kernel<128>, grid, dim3(256), 0, st, keys, dtype, n_tokens, PiT, Pi,
-                               ST, cbv, bdv, out_idx, out_signs, (uint16_t*)out_norm, (uint16_t*)out_gamma);
-        else
-            hipLaunchKernelGGL(fkv::tq_compress_keys_kernel<64>, grid, dim3(256), 0, st, keys, dtype, n_tokens, PiT, Pi,
-                               ST, cbv, bdv, out_idx, out_signs, (uint16_t*)out_norm, (uint16_t*)out_gamma);
-        rc = check_hip(hipGetLastError(), "tq_compress_keys_kernel launch");
-    }
-    if (PiT) (void)hipFreeAsync(PiT, st);
-    if (ST) (void)hipFreeAsync(ST, st);
+    uint8_t* prep = nullptr;
+    int rc = check_hip(hipMallocAsync((void**)&prep, fkv::tq_prep_bytes(D), st), "hipMallocAsync");
+    if (rc) return rc;
+    hipLaunchKernelGGL(fkv::tq_prep_kernel, dim3((unsigned)(3 * D + 1)), dim3(fkv::kWave), 0, st, Pi, S, centroids,
+                       boundaries, D, prep);
+    // vector loads and stores where the caller's arrays are 16-byte aligned
+    // (a token's rows then are too)
+    const bool wide = (((uintptr_t)keys | (uintptr_t)out_idx | (uintptr_t)out_signs) & 15) == 0;
+    auto* kern = D == 128 ? (wide ? fkv::tq_compress_keys_kernel<128, true> : fkv::tq_compress_keys_kernel<128, false>)
+                          : (wide ? fkv::tq_compress_keys_kernel<64, true> : fkv::tq_compress_keys_kernel<64, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)fkv::cdiv(n_tokens, fkv::kTqTok)), dim3(256), 0, st, keys, dtype, n_tokens,
+                       prep, out_idx, out_signs, (uint16_t*)out_norm, (uint16_t*)out_gamma);
+    rc = check_hip(hipGetLastError(), "tq_compress_keys_kernel launch");
+    (void)hipFreeAsync(prep, st);
     return rc;
 }
 

@@ -141,3 +141,125 @@ def test_far_rows_special_values(fkv, D, vg, dt, importance):
         else:
             want = oracle.encode_fp8(far)
         assert np.array_equal(cl.far_k.cpu().numpy(), want)
+
+
+def _unpack(p, bits):
+    per = 8 // bits
+    return ((p[..., None] >> (bits * np.arange(per))) & ((1 << bits) - 1)).reshape(p.shape[:-1] + (-1,))
+
+
+def _check_turbo_keys(k, Pi, S, cb, bd, got):
+    """Codes, signs and norms against fp64.  A decision may differ only where
+    its fp64 value lies within a worst-case fp32 evaluation of its boundary:
+    D sums and the operands' rounding, (D + 16) 2^-24 of the sum of the
+    products' magnitudes; the residual follows from the codes returned."""
+    idx, sgn, nrm, gam = (t.cpu().numpy() for t in got)
+    k, Pi, S, cb, bd = (np.asarray(a, np.float64) for a in (k, Pi, S, cb, bd))
+    D = k.shape[-1]
+    eps = (D + 16) * 2.0 ** -24
+    n = np.linalg.norm(k, axis=-1, keepdims=True)
+    y, tol = k @ Pi.T, eps * (np.abs(k) @ np.abs(Pi).T)
+    codes = _unpack(idx, 2)
+    nc = np.maximum(n, np.float64(np.float32(1e-8)))
+    lo = sum((y - tol >= b * nc + abs(b) * nc * 2.0 ** -23).astype(int) for b in bd)
+    hi = sum((y + tol >= b * nc - abs(b) * nc * 2.0 ** -23).astype(int) for b in bd)
+    assert ((codes >= lo) & (codes <= hi)).all()
+    c = cb[codes]
+    r = k - n * (c @ Pi)
+    rtol = 2.0 ** -22 * np.abs(k) + n * eps * (np.abs(c) @ np.abs(Pi))
+    p, ptol = r @ S.T, rtol @ np.abs(S).T + eps * (np.abs(r) @ np.abs(S).T)
+    signs = _unpack(sgn, 1).astype(bool)
+    assert (signs == (p >= 0))[np.abs(p) > ptol].all()
+    g = np.linalg.norm(r, axis=-1)
+    assert (np.abs(nrm - n[..., 0]) <= 2.0 ** -11 * n[..., 0] + 2.0 ** -24).all()
+    assert (np.abs(gam - g) <= 2.0 ** -11 * g + np.linalg.norm(rtol, axis=-1) + 2.0 ** -24).all()
+
+
+def _turbo_keys(_lib, k, Pi, S, cb, bd, offset=0):
+    """fkv_turbo_compress_keys on (n, D) keys, the buffers ``offset`` elements
+    past a 16-byte boundary."""
+    n, D = k.shape
+
+    def at(numel, dtype):
+        return torch.zeros(numel + offset, dtype=dtype, device="cuda")[offset:]
+
+    kk = at(n * D, k.dtype)
+    kk.copy_(k.reshape(-1))
+    idx, sgn = at(n * D // 4, torch.uint8), at(n * D // 8, torch.uint8)
+    nrm, gam = at(n, torch.float16), at(n, torch.float16)
+    ms = [torch.as_tensor(np.asarray(a, np.float32)).cuda().contiguous() for a in (Pi, S, cb, bd)]
+    _lib.check(_lib.load().fkv_turbo_compress_keys(
+        _lib.ptr(kk), _lib.dtype_code(k.dtype), n, D, *(_lib.ptr(m) for m in ms), _lib.ptr(idx), _lib.ptr(sgn),
+        _lib.ptr(nrm), _lib.ptr(gam), _lib.stream_ptr(torch.device("cuda"))), "fkv_turbo_compress_keys")
+    torch.cuda.synchronize()
+    return idx.view(n, D // 4), sgn.view(n, D // 8), nrm, gam
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 127, 128, 129, 1000])
+@pytest.mark.parametrize("dt,offset", [(torch.float16, 0), (torch.bfloat16, 0), (torch.float32, 0),
+                                       (torch.float16, 1), (torch.bfloat16, 3), (torch.float32, 1)])
+def test_turbo_keys_edges(fkv, D, n, dt, offset):
+    """Token counts at the edges of a wave and a workgroup, every input type,
+    unaligned buffers; keys of very different magnitudes."""
+    from foveated_kv_amd import _lib
+    from foveated_kv_amd.turbo import get_turbo_constants
+
+    flush(f"turbo keys D={D} n={n} {dt} offset={offset}")
+    rng = np.random.default_rng(n + D)
+    k = rng.standard_normal((n, D)) * 2.0 ** rng.integers(-12, 11, (n, 1))
+    k[:, :4] *= 8
+    k[n // 2] = 0
+    kt = torch.from_numpy(k.astype(np.float32)).cuda().to(dt)
+    c = get_turbo_constants(D)
+    args = [t.numpy() for t in (c.Pi, c.S, c.centroids, c.boundaries)]
+    got = _turbo_keys(_lib, kt, *args, offset=offset)
+    _check_turbo_keys(kt.half().cpu().numpy(), *args, got)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_turbo_keys_general_matrices(fkv, D):
+    """Any matrices, centroids and boundaries the entry point takes: rows of
+    very different scales, a zero row, centroids far from 1, boundaries not
+    in order."""
+    from foveated_kv_amd import _lib
+
+    rng = np.random.default_rng(D)
+    Pi = rng.standard_normal((D, D)).astype(np.float32) * 2.0 ** rng.integers(-9, 10, (D, 1)).astype(np.float32)
+    S = rng.standard_normal((D, D)).astype(np.float32) * np.float32(1e-6)
+    Pi[3] = 0
+    for cb, bd in (([-300.0, -7.0, 12.0, 500.0], [0.3, -0.4, 0.05]), ([-3e-7, -1e-7, 2e-7, 4e-7], [0.0, 1.0, -1.0])):
+        cb, bd = np.asarray(cb, np.float32), np.asarray(bd, np.float32)
+        kt = torch.from_numpy(rng.standard_normal((200, D)).astype(np.float16)).cuda()
+        flush(f"turbo keys general D={D} cb={cb} bd={bd}")
+        got = _turbo_keys(_lib, kt, Pi, S, cb, bd)
+        idx, sgn, nrm, gam = got
+        ok = torch.isfinite(gam)  # residual norms past fp16 are infinite, as before
+        assert (ok | (gam == float("inf"))).all()
+        g = gam.clone()
+        g[~ok] = 0
+        sel = ok.cpu().numpy()
+        if sel.any():
+            _check_turbo_keys(kt.cpu().numpy()[sel], Pi, S, cb, bd, (idx[ok], sgn[ok], nrm[ok], gam[ok]))
+
+
+def test_turbo_keys_non_finite(fkv):
+    """A key row with an infinity or NaN: code 0 and sign 0 everywhere, as a
+    sum of NaN compares; the other rows are untouched by it."""
+    from foveated_kv_amd import _lib
+    from foveated_kv_amd.turbo import get_turbo_constants
+
+    for D in (64, 128):
+        rng = np.random.default_rng(7)
+        k = rng.standard_normal((64, D)).astype(np.float16)
+        k[5, 3], k[6, 9], k[7, 0] = np.inf, -np.inf, np.nan
+        c = get_turbo_constants(D)
+        args = [t.numpy() for t in (c.Pi, c.S, c.centroids, c.boundaries)]
+        flush(f"turbo keys non-finite D={D}")
+        got = _turbo_keys(_lib, torch.from_numpy(k).cuda(), *args)
+        bad = torch.tensor([5, 6, 7], device="cuda")
+        assert (got[0][bad] == 0).all() and (got[1][bad] == 0).all() and not torch.isfinite(got[2][bad]).any()
+        keep = np.ones(64, bool)
+        keep[[5, 6, 7]] = False
+        m = torch.from_numpy(keep).cuda()
+        _check_turbo_keys(k[keep], *args, tuple(t[m] for t in got))
