@@ -6,6 +6,8 @@
 
 #include <string>
 
+#include "../../include/fkv.h"
+
 typedef _Float16 fkv_h2 __attribute__((ext_vector_type(2)));
 typedef float fkv_f2 __attribute__((ext_vector_type(2)));
 
@@ -67,6 +69,41 @@ __device__ inline float wave_min(float v) {
     for (int o = 32; o >= 1; o >>= 1) v = fminf(v, wave_xor(v, o));
     return v;
 }
+
+// 8 consecutive elements as packed fp16 bits (astype(float16) semantics: RNE)
+__device__ inline uint4 load8(const void* base, int dtype, int64_t elem) {
+    if (dtype == FKV_F16) return *(const uint4*)((const uint16_t*)base + elem);
+    auto pk = [](float a, float b) { return (uint32_t)f2h(a) | ((uint32_t)f2h(b) << 16); };
+    if (dtype == FKV_BF16) {
+        const uint4 w = *(const uint4*)((const uint16_t*)base + elem);
+        auto two = [&](uint32_t u) { return pk(__uint_as_float(u << 16), __uint_as_float(u & 0xFFFF0000u)); };
+        return make_uint4(two(w.x), two(w.y), two(w.z), two(w.w));
+    }
+    const float4* p = (const float4*)((const float*)base + elem);
+    const float4 a = p[0], b = p[1];
+    return make_uint4(pk(a.x, a.y), pk(a.z, a.w), pk(b.x, b.y), pk(b.z, b.w));
+}
+
+// a / b rounded to nearest even, from y = 1.0f / b (so rounded itself):
+// Markstein's correction of a * y.  One step gives the correctly rounded
+// quotient where a * y is within one unit in the last place; a second one
+// (STEPS = 2) holds for any rounding of a * y.  A non-finite b gives NaN
+// where the division gives 0 or NaN.
+template <int STEPS>
+__device__ inline float div_by(float a, float b, float y) {
+    float q = a * y;
+#pragma unroll
+    for (int i = 0; i < STEPS; i++) q = fmaf(fmaf(-b, q, a), y, q);
+    return q;
+}
+
+// v of another lane by DPP (a quad_perm or row mirror control).
+template <int CTRL>
+__device__ inline float dpp_f32(float v) {
+    const int i = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, true));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;  // quad_perm 1,0,3,2 and 2,3,0,1
 
 // Wave-wide (max, first index) reduction: larger value wins, ties go to the
 // smaller index.  Lanes with no candidate hold (-inf, INT_MAX).

@@ -73,33 +73,6 @@ __device__ inline uint32_t encode_e4m3x4(uint32_t w0, uint32_t w1) {
     return (codes & ~mask) | (mask & 0x7E7E7E7Eu);
 }
 
-// 8 consecutive elements as packed fp16 bits (astype(float16) semantics: RNE)
-__device__ inline uint4 load8(const void* base, int dtype, int64_t elem) {
-    if (dtype == FKV_F16) return *(const uint4*)((const uint16_t*)base + elem);
-    auto pk = [](float a, float b) { return (uint32_t)f2h(a) | ((uint32_t)f2h(b) << 16); };
-    if (dtype == FKV_BF16) {
-        const uint4 w = *(const uint4*)((const uint16_t*)base + elem);
-        auto two = [&](uint32_t u) { return pk(__uint_as_float(u << 16), __uint_as_float(u & 0xFFFF0000u)); };
-        return make_uint4(two(w.x), two(w.y), two(w.z), two(w.w));
-    }
-    const float4* p = (const float4*)((const float*)base + elem);
-    const float4 a = p[0], b = p[1];
-    return make_uint4(pk(a.x, a.y), pk(a.z, a.w), pk(b.x, b.y), pk(b.z, b.w));
-}
-
-// a / b rounded to nearest even, from y = 1.0f / b (so rounded itself):
-// Markstein's correction of a * y.  One step gives the correctly rounded
-// quotient where a * y is within one unit in the last place; a second one
-// (STEPS = 2) holds for any rounding of a * y.  A non-finite b gives NaN
-// where the division gives 0 or NaN.
-template <int STEPS>
-__device__ inline float div_by(float a, float b, float y) {
-    float q = a * y;
-#pragma unroll
-    for (int i = 0; i < STEPS; i++) q = fmaf(fmaf(-b, q, a), y, q);
-    return q;
-}
-
 // The fp16 value a key is encoded from with a per-head scale: fp16(key /
 // scale), fp32 division rounded to nearest even.  One correction step is
 // enough for every fp16 key and every scale that is an fp16 amax over 240
@@ -115,18 +88,13 @@ __device__ inline uint32_t scaled_keys(uint32_t w, float scale, float rscale) {
 
 // Minimum and maximum over the RL lanes (4, 8 or 16, aligned) of a row by DPP: lane
 // pairs, quads, then the mirrored halves of 8 and of 16 lanes.
-template <int CTRL>
-__device__ inline float dpp_f32(float v) {
-    const int i = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, true));
-}
 template <int RL>
 __device__ inline void row_minmax(float& mn, float& mx) {
     static_assert(RL == 4 || RL == 8 || RL == 16, "rows of 4, 8 or 16 lanes");
-    mn = fminf(mn, dpp_f32<0xB1>(mn));  // quad_perm 1,0,3,2
-    mx = fmaxf(mx, dpp_f32<0xB1>(mx));
-    mn = fminf(mn, dpp_f32<0x4E>(mn));  // quad_perm 2,3,0,1
-    mx = fmaxf(mx, dpp_f32<0x4E>(mx));
+    mn = fminf(mn, dpp_f32<kDppXor1>(mn));
+    mx = fmaxf(mx, dpp_f32<kDppXor1>(mx));
+    mn = fminf(mn, dpp_f32<kDppXor2>(mn));
+    mx = fmaxf(mx, dpp_f32<kDppXor2>(mx));
     if (RL >= 8) {
         mn = fminf(mn, dpp_f32<0x141>(mn));  // row_half_mirror
         mx = fmaxf(mx, dpp_f32<0x141>(mx));

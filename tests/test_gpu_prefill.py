@@ -263,3 +263,40 @@ def test_turbo_keys_non_finite(fkv):
         keep[[5, 6, 7]] = False
         m = torch.from_numpy(keep).cuda()
         _check_turbo_keys(k[keep], *args, tuple(t[m] for t in got))
+
+
+@pytest.mark.parametrize("dt,offset", [(torch.float16, 0), (torch.float16, 1), (torch.bfloat16, 3), (torch.float32, 0),
+                                       (torch.float32, 1)])
+@pytest.mark.parametrize("D,n", [(32, 1), (64, 3), (128, 67), (96, 1001)])
+def test_turbo_values_edges(fkv, D, n, dt, offset):
+    """TurboQuant values bit for bit against fp32 numpy: ties, zero groups,
+    infinities, NaN, subnormals, any head dim of whole groups, unaligned values."""
+    from foveated_kv_amd import _lib
+
+    flush(f"turbo values D={D} n={n} {dt} offset={offset}")
+    rng = np.random.default_rng(D + n)
+    v = rng.standard_normal((n, D)).astype(np.float32)
+    v[0, :32] = 0
+    v[0, :9] = [3, -3, 1, -1, 0.5, 2, -2, -0.0, 0]
+    flat = v.reshape(-1, 32)
+    if len(flat) > 40:
+        flat[7] = 0
+        flat[8] *= 2.0 ** -22
+        flat[9, 3], flat[10, 4], flat[11, 5] = np.inf, -np.inf, np.nan
+        flat[12] = np.nan
+        flat[13] = rng.integers(-6, 7, 32)
+    buf = torch.zeros(n * D + offset, dtype=dt, device="cuda")[offset:]
+    buf.copy_(torch.from_numpy(v.reshape(-1)).cuda().to(dt))
+    packed = torch.empty(n * D // 4, dtype=torch.uint8, device="cuda")
+    scale = torch.empty(n * D // 32, dtype=torch.float16, device="cuda")
+    _lib.check(_lib.load().fkv_turbo_compress_values(_lib.ptr(buf), _lib.dtype_code(dt), n, D, _lib.ptr(packed),
+                                                     _lib.ptr(scale), _lib.stream_ptr(torch.device("cuda"))),
+               "fkv_turbo_compress_values")
+    f = buf.half().float().cpu().numpy().reshape(-1, 32)
+    with np.errstate(all="ignore"):
+        sc = np.fmax(np.fmax.reduce(np.abs(f), -1, keepdims=True, initial=0), np.float32(1e-8))
+        x = np.rint((f / sc + np.float32(1)) * np.float32(1.5))
+        codes = np.nan_to_num(np.fmin(np.fmax(x, 0), 3)).astype(np.uint8)
+    want = (codes.reshape(-1, 4) << np.array([0, 2, 4, 6], np.uint8)).sum(-1).astype(np.uint8)
+    assert np.array_equal(packed.cpu().numpy(), want)
+    assert np.array_equal(scale.cpu().numpy(), sc[:, 0].astype(np.float16))
