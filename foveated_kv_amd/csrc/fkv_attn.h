@@ -23,15 +23,16 @@ namespace fkv {
 //        16c..16c+15
 //   | V: 32*D bytes of INT4 nibbles, lane l = dim 64*dh + l
 //   | SZ: 64 x u32 = fp16 scale | fp16 zero << 16 per token ]
-//   near_valid : [Hkv] u32
+//   near_valid : [Hkv] u32, then one u32: bad far codes found while packing
 //   kscale     : [B*Hkv] fp32 per-head fp8 key scale (1 unless set with
 //                fkv_attn_set_k_scale; the kernel multiplies far scores by it)
+//   rot        : fmt 1 only: Pi and S as fp16 operands (tq_rot_index)
 // A TurboQuant blob (fmt 1) keeps the near tiers and near_valid and stores
 // the far tier as TurboQuant records instead (layout below).
 struct BlobLayout {
     int B, Hkv, D, Na, F, Na_pad, F_pad;
     int fmt;  // 0: fp8-E4M3 K / INT4 V far records, 1: TurboQuant, 2: fp8 K / group-32 INT4 V
-    size_t near_k, near_v, far, far_rec, near_valid, kscale, total;
+    size_t near_k, near_v, far, far_rec, near_valid, kscale, rot, total;
 };
 
 BlobLayout make_layout(int B, int Hkv, int D, int Na, int F, int fmt = 0);
@@ -121,7 +122,7 @@ __device__ inline uint16_t load_as_f16(const void* p, int64_t i, int dtype) {
 // sketch MFMAs (tq_rot_index).
 struct TurboConsts {
     float alpha = 0.f, beta = 0.f, gamma = 0.f, delta = 0.f, lvh = 0.f, lvl = 0.f;
-    uint16_t* rot = nullptr;  // 4 * D * D bytes of fp16 operands
+    const uint16_t* rot = nullptr;  // the blob's fp16 operands
 };
 
 // Pi (mat 0) and S (mat 1) as fp16, laid out so that lane l of a wave
@@ -202,11 +203,36 @@ LaunchPlan plan_launch(const BlobLayout& L, int Hq, int n_decode, int target_wgs
 // for every launch plan of that head count (any decode length).
 size_t workspace_floats(const BlobLayout& L, int Hq);
 int workspace_rows(const BlobLayout& L, int Hq);
-// Handle construction shared by the fp8 and TurboQuant formats: allocates
-// the blob (zeroed), packs the near tiers and near_valid (stream-ordered).
-int attn_begin(fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const void* near_k,
-               const void* near_v, int near_dtype, const int32_t* near_valid, float margin, hipStream_t st);
-// Synchronous end of construction: reads near_valid back for the split plan.
-int attn_finish(fkv_attn_impl* h, hipStream_t st);
+// A handle's sources: the tier arrays in the types the entry points take
+// (far_* for fmt 0 / 2, the rest for TurboQuant).
+struct PackSrc {
+    const void* near_k;
+    const void* near_v;
+    int near_dtype;
+    const int32_t* near_valid;
+    const uint8_t* far_k;
+    const uint8_t* far_v;
+    const void* far_v_scale;
+    const void* far_v_zero;
+    int sz_dtype;
+    const uint8_t* k_idx;
+    const uint8_t* k_signs;
+    const void* k_norm;
+    const void* k_gamma;
+    const uint8_t* v_packed;
+    const void* v_scale;
+    int nz_dtype;
+    const float* Pi;
+    const float* S;
+};
+// The whole blob from its sources (stream-ordered; every tile, padding included).
+int pack_blob(const PackSrc& s, const BlobLayout& L, uint8_t* blob, hipStream_t st);
+// Handle construction shared by the formats: allocates the blob and packs it
+// (stream-ordered).
+int attn_begin(fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const PackSrc& s, float margin,
+               hipStream_t st);
+// Synchronous end of construction: reads near_valid back for the split plan
+// and whether the far codes held one the reference never emits (FKV_EDATA).
+int attn_finish(const char* fn, fkv_attn_impl* h, hipStream_t st);
 
 }  // namespace fkv

@@ -72,177 +72,20 @@ BlobLayout make_layout(int B, int Hkv, int D, int Na, int F, int fmt) {
     L.near_v = place(bkv * L.Na_pad * D * 2);
     L.far_rec = (size_t)(fmt == 1 ? tq_record_bytes(D) : fmt == 2 ? g32_record_bytes(D) : far_record_bytes(D));
     L.far = place(bkv * (L.F_pad / kTile) * L.far_rec);
-    L.near_valid = place((size_t)Hkv * 4);
+    L.near_valid = place(((size_t)Hkv + 1) * 4);
     L.kscale = place(bkv * 4);
+    L.rot = place(fmt == 1 ? (size_t)4 * D * D : 0);
     L.total = off;
     return L;
 }
 
-// ---------------------------------------------------------------------------
-// Blob packing kernels (handle construction; csrc/foveated_attn.cpp:83-128)
-// ---------------------------------------------------------------------------
-
-// One thread per (bkv, token, 16-dim block): near K and V into their tile
-// layouts (fkv_attn.h); slots >= Na are zero.
-__global__ void pack_near_kernel(const void* __restrict__ nk, const void* __restrict__ nv,
-                                 int dtype, BlobLayout L, uint8_t* __restrict__ blob) {
-    const int D = L.D, NB = D / 16;
-    const int64_t n = (int64_t)L.B * L.Hkv * L.Na_pad * NB;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int blk = (int)(i % NB);
-        const int64_t r = i / NB;
-        const int t = (int)(r % L.Na_pad);
-        const int64_t bkv = r / L.Na_pad;
-        uint16_t* kd = (uint16_t*)(blob + L.near_k) + bkv * (int64_t)L.Na_pad * D;
-        uint16_t* vd = (uint16_t*)(blob + L.near_v) + bkv * (int64_t)L.Na_pad * D;
-        for (int e = 0; e < 16; e++) {
-            const int d = blk * 16 + e;
-            const int64_t src = (bkv * L.Na + t) * D + d;
-            kd[near_k_index(t, d, D)] = t < L.Na ? load_as_f16(nk, src, dtype) : 0;
-            vd[near_v_index(t, d, D)] = t < L.Na ? load_as_f16(nv, src, dtype) : 0;
-        }
-    }
-}
-
-// Far K codes into the tile layout; exponent-0 codes are written as signed
-// zero (the reference LUT ignores their mantissa); NaN codes 0x7F/0xFF are
-// reported through *bad.
-__global__ void pack_far_k_kernel(const uint8_t* __restrict__ fk, BlobLayout L,
-                                  uint8_t* __restrict__ blob, unsigned* __restrict__ bad) {
-    const int D = L.D, NB = D / 16;
-    const int64_t n = (int64_t)L.B * L.Hkv * L.F_pad * NB;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int blk = (int)(i % NB);
-        const int64_t r = i / NB;
-        const int t = (int)(r % L.F_pad);
-        const int64_t bkv = r / L.F_pad;
-        uint8_t* dst = blob + L.far + far_rec_index(L, bkv, t / kTile) * (int64_t)L.far_rec;
-        for (int e = 0; e < 16; e++) {
-            const int d = blk * 16 + e;
-            uint8_t b = 0;
-            if (t < L.F) {
-                b = fk[(bkv * L.F + t) * D + d];
-                if ((b & 0x7F) == 0x7F) atomicOr(bad, 1u);
-                if ((b & 0x78) == 0) b &= 0x80;
-            }
-            dst[far_k_index(t, d)] = b;
-        }
-    }
-}
-
-// Far V nibbles: one thread builds one dword of the tile layout (8 nibbles:
-// 2 four-token groups of one dim); thread (kg=0 lanes) also packs the
-// per-token scale / zero.
-__global__ void pack_far_v_kernel(const uint8_t* __restrict__ fv, const void* __restrict__ fvs,
-                                  const void* __restrict__ fvz, int sz_dtype, BlobLayout L,
-                                  uint8_t* __restrict__ blob) {
-    const int D = L.D;
-    const int64_t words_per_bkv = (int64_t)L.F_pad * D / 8;
-    const int64_t n = (int64_t)L.B * L.Hkv * words_per_bkv;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t bkv = i / words_per_bkv;
-        const int64_t w = i % words_per_bkv;
-        // invert the dword position: tile, chunk, lane, word-in-chunk
-        const int tile = (int)(w / (8 * D));
-        const int rem = (int)(w % (8 * D));
-        const int c = rem / 256, lane = (rem % 256) / 4, q = rem % 4;
-        const int u = c * 4 + q, dh = u / 8, spair = u % 8;
-        const int d = dh * 64 + lane;
-        uint32_t word = 0;
-        for (int bp = 0; bp < 2; bp++)
-            for (int e = 0; e < 4; e++) {
-                const int t = tile * 64 + (2 * spair + bp) * 4 + e;
-                uint32_t code = 0;
-                if (t < L.F) code = (fv[(bkv * L.F + t) * (D / 2) + d / 2] >> (4 * (d & 1))) & 15u;
-                word |= code << (bp * 8 + (e & 1) * 16 + (e >> 1) * 4);
-            }
-        ((uint32_t*)(blob + L.far + far_rec_index(L, bkv, tile) * (int64_t)L.far_rec +
-                     far_v_section(D)))[rem] = word;
-    }
-    const int64_t nt = (int64_t)L.B * L.Hkv * L.F_pad;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nt;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int t = (int)(i % L.F_pad);
-        const int64_t bkv = i / L.F_pad;
-        uint32_t sz = 0;
-        if (t < L.F) {
-            const int64_t k = bkv * L.F + t;
-            sz = (uint32_t)load_as_f16(fvs, k, sz_dtype) | ((uint32_t)load_as_f16(fvz, k, sz_dtype) << 16);
-        }
-        ((uint32_t*)(blob + L.far + far_rec_index(L, bkv, t / kTile) * (int64_t)L.far_rec +
-                     far_sz_section(D)))[t % kTile] = sz;
-    }
-}
-
-// Group-32 far V (fmt 2): one thread per output dword of the V section
-// (chunk c = 2*dh + half-select, lane, word u), and per token the group
-// scale | zero words.
-__global__ void pack_far_v_g32_kernel(const uint8_t* __restrict__ fv, const void* __restrict__ fvs,
-                                      const void* __restrict__ fvz, int sz_dtype, BlobLayout L,
-                                      uint8_t* __restrict__ blob) {
-    const int D = L.D, NG = D / 32;
-    const int64_t words_per_tile = (int64_t)8 * D;  // 32*D bytes of nibbles
-    const int64_t nt = L.F_pad / kTile;
-    const int64_t n = (int64_t)L.B * L.Hkv * nt * words_per_tile;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int rem = (int)(i % words_per_tile);
-        const int64_t r = i / words_per_tile;
-        const int tile = (int)(r % nt);
-        const int64_t bkv = r / nt;
-        const int c = rem / 256, lane = (rem % 256) / 4, u = rem % 4;
-        const int dh = c >> 1, other = c & 1;
-        const int d = dh * 64 + lane;
-        const int half = lane >> 5;
-        const int base = 32 * (other ? 1 - half : half);
-        uint32_t word = 0;
-        for (int bp = 0; bp < 2; bp++)
-            for (int e = 0; e < 4; e++) {
-                const int t = tile * kTile + base + (2 * u + bp) * 4 + e;
-                uint32_t code = 0;
-                if (t < L.F) code = (fv[(bkv * L.F + t) * (D / 2) + d / 2] >> (4 * (d & 1))) & 15u;
-                word |= code << (bp * 8 + (e & 1) * 16 + (e >> 1) * 4);
-            }
-        ((uint32_t*)(blob + L.far + far_rec_index(L, bkv, tile) * (int64_t)L.far_rec + far_v_section(D)))[rem] = word;
-    }
-    const int64_t ntok = (int64_t)L.B * L.Hkv * L.F_pad;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ntok;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int t = (int)(i % L.F_pad);
-        const int64_t bkv = i / L.F_pad;
-        uint32_t* sz = (uint32_t*)(blob + L.far + far_rec_index(L, bkv, t / kTile) * (int64_t)L.far_rec +
-                                   g32_sz_section(D)) + (t % kTile) * NG;
-        for (int g = 0; g < NG; g++) {
-            uint32_t w = 0;
-            if (t < L.F) {
-                const int64_t k = (bkv * L.F + t) * NG + g;
-                w = (uint32_t)load_as_f16(fvs, k, sz_dtype) | ((uint32_t)load_as_f16(fvz, k, sz_dtype) << 16);
-            }
-            sz[g] = w;
-        }
-    }
-}
-
-__global__ void pack_valid_kernel(const int32_t* __restrict__ nv, int Hkv, BlobLayout L,
-                                  uint8_t* __restrict__ blob) {
-    int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h < Hkv) {
-        int v = nv[h];
-        v = v < 0 ? 0 : (v > L.Na ? L.Na : v);
-        ((uint32_t*)(blob + L.near_valid))[h] = (uint32_t)v;
-    }
-}
-
-// The blob's per-head fp8 key scales: 1 (src NULL) or src[i]; a scale that
-// is not a positive finite number raises *bad.
+// The blob's per-head fp8 key scales; one that is not a positive finite
+// number raises *bad.
 __global__ void fill_kscale_kernel(const float* __restrict__ src, int n, BlobLayout L, uint8_t* __restrict__ blob,
                                    unsigned* bad) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float v = src ? src[i] : 1.0f;
+    const float v = src[i];
     if (!(v > 0.f && v <= 3.402823466e38f)) *bad = 1u;
     ((float*)(blob + L.kscale))[i] = v;
 }
@@ -1148,8 +991,8 @@ int xcd_rule(int dev, hipStream_t st, int* mod) {
     return FKV_OK;
 }
 
-int attn_begin(fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const void* near_k,
-               const void* near_v, int near_dtype, const int32_t* near_valid, float margin, hipStream_t st) {
+int attn_begin(fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const PackSrc& s, float margin,
+               hipStream_t st) {
     h->L = make_layout(B, Hkv, D, Na, F, fmt);
     h->margin = margin;
     // tuning knobs are read once here, never on the call path
@@ -1158,30 +1001,24 @@ int attn_begin(fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, 
     h->fused_merge = env_int("FKV_FUSED_MERGE", 1) != 0;
     int rc = check_hip(hipGetDevice(&h->device), "hipGetDevice");
     if (!rc) rc = check_hip(hipMalloc(&h->blob, h->L.total), "hipMalloc(blob)");
-    if (!rc) rc = check_hip(hipMemsetAsync(h->blob, 0, h->L.total, st), "hipMemsetAsync(blob)");
-    if (rc) return rc;
-    const int blk = 256;
-    const BlobLayout L = h->L;
-    if (Na > 0)
-        hipLaunchKernelGGL(pack_near_kernel, dim3(grid_for((int64_t)B * Hkv * L.Na_pad * (D / 16), blk)), dim3(blk),
-                           0, st, near_k, near_v, near_dtype, L, h->blob);
-    hipLaunchKernelGGL(pack_valid_kernel, dim3(grid_for(Hkv, blk)), dim3(blk), 0, st, near_valid, Hkv, L, h->blob);
-    hipLaunchKernelGGL(fill_kscale_kernel, dim3(grid_for((int64_t)B * Hkv, blk)), dim3(blk), 0, st, nullptr, B * Hkv,
-                       L, h->blob, nullptr);
-    return check_hip(hipGetLastError(), "pack kernels");
+    return rc ? rc : pack_blob(s, h->L, h->blob, st);
 }
 
-int attn_finish(fkv_attn_impl* h, hipStream_t st) {
+int attn_finish(const char* fn, fkv_attn_impl* h, hipStream_t st) {
     if (int rc = xcd_rule(h->device, st, &h->xcd_mod)) return rc;
     if (env_int("FKV_XCD_LOCAL", 1) == 0) h->xcd_mod = 0;  // read once per handle, at creation
-    std::vector<uint32_t> nv_h(h->L.Hkv, 0);
-    int rc = check_hip(hipMemcpyAsync(nv_h.data(), h->blob + h->L.near_valid, h->L.Hkv * sizeof(uint32_t),
+    std::vector<uint32_t> nv_h(h->L.Hkv + 1, 0);  // near_valid, then the bad-code flag
+    int rc = check_hip(hipMemcpyAsync(nv_h.data(), h->blob + h->L.near_valid, nv_h.size() * sizeof(uint32_t),
                                       hipMemcpyDeviceToHost, st), "hipMemcpyAsync(near_valid)");
     if (!rc) rc = check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
     if (rc) return rc;
     uint32_t mx = 0;
-    for (uint32_t v : nv_h) mx = v > mx ? v : mx;
+    for (int i = 0; i < h->L.Hkv; i++) mx = nv_h[i] > mx ? nv_h[i] : mx;
     h->near_plan = (int)cdiv(mx, kTile);
+    if (nv_h[h->L.Hkv]) {
+        set_error(std::string(fn) + ": far_k holds E4M3 NaN codes 0x7F/0xFF, which the reference encoder never emits");
+        return FKV_EDATA;
+    }
     return FKV_OK;
 }
 
@@ -1208,33 +1045,18 @@ int create_fp8(const char* fn, int fmt, fkv_attn** out, int32_t B, int32_t Hkv, 
         return set_error(name + ": NULL tier array");
     hipStream_t st = (hipStream_t)stream;
     fkv_attn* h = new fkv_attn();
-    unsigned* bad = nullptr;
-    int rc = fkv::attn_begin(h, B, Hkv, D, Na, F, fmt, near_k, near_v, near_dtype, near_valid, spike_margin, st);
-    if (!rc) rc = check_hip(hipMalloc(&bad, sizeof(unsigned)), "hipMalloc(flag)");
-    if (!rc) rc = check_hip(hipMemsetAsync(bad, 0, sizeof(unsigned), st), "hipMemsetAsync");
-    if (!rc && F > 0) {
-        const int blk = 256;
-        const fkv::BlobLayout L = h->L;
-        hipLaunchKernelGGL(fkv::pack_far_k_kernel, dim3(fkv::grid_for((int64_t)B * Hkv * L.F_pad * (D / 16), blk)),
-                           dim3(blk), 0, st, far_k, L, h->blob, bad);
-        if (fmt == 2)
-            hipLaunchKernelGGL(fkv::pack_far_v_g32_kernel,
-                               dim3(fkv::grid_for((int64_t)B * Hkv * L.F_pad * (D / 8), blk)), dim3(blk), 0, st,
-                               far_v, far_v_scale, far_v_zero, sz_dtype, L, h->blob);
-        else
-            hipLaunchKernelGGL(fkv::pack_far_v_kernel,
-                               dim3(fkv::grid_for((int64_t)B * Hkv * L.F_pad * (D / 8), blk)), dim3(blk), 0, st,
-                               far_v, far_v_scale, far_v_zero, sz_dtype, L, h->blob);
-        rc = check_hip(hipGetLastError(), "far pack kernels");
-    }
-    unsigned bad_h = 0;
-    if (!rc) rc = check_hip(hipMemcpyAsync(&bad_h, bad, sizeof(unsigned), hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
-    if (!rc) rc = fkv::attn_finish(h, st);
-    if (bad) (void)hipFree(bad);
-    if (!rc && bad_h) {
-        set_error(name + ": far_k holds E4M3 NaN codes 0x7F/0xFF, which the reference encoder never emits");
-        rc = FKV_EDATA;
-    }
+    fkv::PackSrc src{};
+    src.near_k = near_k;
+    src.near_v = near_v;
+    src.near_dtype = near_dtype;
+    src.near_valid = near_valid;
+    src.far_k = far_k;
+    src.far_v = far_v;
+    src.far_v_scale = far_v_scale;
+    src.far_v_zero = far_v_zero;
+    src.sz_dtype = sz_dtype;
+    int rc = fkv::attn_begin(h, B, Hkv, D, Na, F, fmt, src, spike_margin, st);
+    if (!rc) rc = fkv::attn_finish(fn, h, st);
     if (rc) {
         fkv_attn_destroy(h);
         return rc;
@@ -1868,7 +1690,6 @@ void fkv_attn_destroy(fkv_attn* h) {
     if (h->ws) (void)hipFree(h->ws);
     if (h->qbuf) (void)hipFree(h->qbuf);
     if (h->arrive) (void)hipFree(h->arrive);
-    if (h->tq.rot) (void)hipFree(h->tq.rot);
     if (h->order_ev) (void)hipEventDestroy(h->order_ev);
     delete h;
 }

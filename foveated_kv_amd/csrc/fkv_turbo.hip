@@ -1,5 +1,5 @@
-// TurboQuant far tier for gfx950: handle construction (blob packing), the
-// per-call query rotation / sketch, and the compression kernels.
+// TurboQuant far tier for gfx950: handle construction and the compression
+// kernels.
 //
 // Replaces the reference's TurboFoveatedHandle (csrc/foveated_attn.cpp:
 // 280-491) and its Python compression (src/foveated_kv/turbo_quantize.py:
@@ -14,120 +14,6 @@
 #include "fkv_common.h"
 
 namespace fkv {
-
-// ---------------------------------------------------------------------------
-// blob packing (csrc/foveated_attn.cpp:297-345 re-laid-out, fkv_attn.h)
-// ---------------------------------------------------------------------------
-
-__device__ inline uint8_t* tq_record(const BlobLayout& L, uint8_t* blob, int64_t bkv, int t) {
-    return blob + L.far + far_rec_index(L, bkv, t / kTile) * (int64_t)L.far_rec;
-}
-
-// One thread per (bkv, far token, 32-dim word k): the three complemented key
-// bit planes (index high bit, index low bit, QJL sign).
-__global__ void tq_pack_k_kernel(const uint8_t* __restrict__ idx, const uint8_t* __restrict__ sgn, BlobLayout L,
-                                 uint8_t* __restrict__ blob) {
-    const int D = L.D, NK = D / 32;
-    const int64_t n = (int64_t)L.B * L.Hkv * L.F_pad * NK;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int k = (int)(i % NK);
-        const int64_t r = i / NK;
-        const int t = (int)(r % L.F_pad);
-        const int64_t bkv = r / L.F_pad;
-        uint32_t wh = 0, wl = 0, ws = 0;
-        if (t < L.F) {
-            const uint8_t* ip = idx + (bkv * L.F + t) * (D / 4) + 8 * k;
-            const uint8_t* sp = sgn + (bkv * L.F + t) * (D / 8) + 4 * k;
-            for (int d = 0; d < 32; d++) {
-                const int c = (ip[d >> 2] >> (2 * (d & 3))) & 3;
-                const int sb = (sp[d >> 3] >> (d & 7)) & 1;
-                const int bit = 15 - (d >> 1) + 16 * (d & 1);
-                wh |= (uint32_t)((c >> 1) ^ 1) << bit;
-                wl |= (uint32_t)((c & 1) ^ 1) << bit;
-                ws |= (uint32_t)(sb ^ 1) << bit;
-            }
-        }
-        uint8_t* rec = tq_record(L, blob, bkv, t);
-        const int lt = t % kTile;
-        ((uint32_t*)(rec + 0 * 8 * D + lt * (D / 8)))[k] = wh;
-        ((uint32_t*)(rec + 1 * 8 * D + lt * (D / 8)))[k] = wl;
-        ((uint32_t*)(rec + 2 * 8 * D + lt * (D / 8)))[k] = ws;
-    }
-}
-
-// One thread per (bkv, tile, 64-dim half dh, lane l): the lane's four value
-// plane dwords for dim 64dh + l.
-__global__ void tq_pack_v_kernel(const uint8_t* __restrict__ vp, BlobLayout L, uint8_t* __restrict__ blob) {
-    const int D = L.D, NT = L.F_pad / kTile, NHALF = D / 64;
-    const int64_t n = (int64_t)L.B * L.Hkv * NT * NHALF * 64;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int l = (int)(i % 64);
-        int64_t r = i / 64;
-        const int dh = (int)(r % NHALF);
-        r /= NHALF;
-        const int tile = (int)(r % NT);
-        const int64_t bkv = r / NT;
-        const int d = 64 * dh + l, half = l >> 5;
-        uint32_t w[4] = {0u, 0u, 0u, 0u};  // hi own, hi other, lo own, lo other
-        for (int o = 0; o < 2; o++) {
-            const int base = 32 * (o ? 1 - half : half);
-            for (int jj = 0; jj < 32; jj++) {
-                const int t = tile * kTile + base + jj;
-                int c = 3;  // padding tokens: +1 bits (their weights are zero)
-                if (t < L.F) c = (vp[(bkv * L.F + t) * (D / 4) + d / 4] >> (2 * (d & 3))) & 3;
-                const int bit = 15 - (jj >> 1) + 16 * (jj & 1);
-                w[o] |= (uint32_t)((c >> 1) ^ 1) << bit;
-                w[2 + o] |= (uint32_t)((c & 1) ^ 1) << bit;
-            }
-        }
-        uint32_t* dst = (uint32_t*)(blob + L.far + far_rec_index(L, bkv, tile) * (int64_t)L.far_rec +
-                                    tq_vp_section(D) + dh * 1024 + l * 16);
-        dst[0] = w[0];
-        dst[1] = w[1];
-        dst[2] = w[2];
-        dst[3] = w[3];
-    }
-}
-
-// One thread per (bkv, far token): value group scales and norm | gamma.
-__global__ void tq_pack_sn_kernel(const void* __restrict__ vscale, const void* __restrict__ knorm,
-                                  const void* __restrict__ kgamma, int dtype, BlobLayout L,
-                                  uint8_t* __restrict__ blob) {
-    const int D = L.D, NG = D / 32;
-    const int64_t n = (int64_t)L.B * L.Hkv * L.F_pad;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int t = (int)(i % L.F_pad);
-        const int64_t bkv = i / L.F_pad;
-        uint8_t* rec = tq_record(L, blob, bkv, t);
-        const int lt = t % kTile;
-        uint16_t* sc = (uint16_t*)(rec + tq_sc_section(D));
-        const int64_t tok = bkv * L.F + t;
-        for (int g = 0; g < NG; g++)
-            sc[tq_sc_index(D, lt / 4, g % 2, lt % 4, g / 2)] = t < L.F ? load_as_f16(vscale, tok * NG + g, dtype)
-                                                                      : (uint16_t)0;
-        uint32_t w = 0;
-        if (t < L.F) w = (uint32_t)load_as_f16(knorm, tok, dtype) | ((uint32_t)load_as_f16(kgamma, tok, dtype) << 16);
-        ((uint32_t*)(rec + tq_ng_section(D)))[lt] = w;
-    }
-}
-
-// Pi and S -> the rotation MFMAs' fp16 operands (tq_rot_index).
-__global__ void rot_operand_kernel(const float* __restrict__ Pi, const float* __restrict__ S,
-                                   uint16_t* __restrict__ rot, int D) {
-    const int64_t n = 2 * (int64_t)D * D;
-    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int mat = (int)(e / ((int64_t)D * D)), i = (int)(e / D % D), j = (int)(e % D);
-        rot[tq_rot_index(D, mat, i, j)] = f2h((mat ? S : Pi)[(int64_t)i * D + j]);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// per-call query preparation (csrc/foveated_attn.cpp:415-421)
-// ---------------------------------------------------------------------------
 
 // ---------------------------------------------------------------------------
 // compression (src/foveated_kv/turbo_quantize.py:25-91, 139-178), fp32
@@ -579,28 +465,26 @@ int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t 
         return set_error("fkv_turbo_create: NULL array");
     hipStream_t st = (hipStream_t)stream;
     fkv_attn* h = new fkv_attn();
-    int rc = fkv::attn_begin(h, B, Hkv, D, Na, F, 1, near_k, near_v, near_dtype, near_valid, spike_margin, st);
-    if (!rc) rc = check_hip(hipMalloc(&h->tq.rot, (size_t)4 * D * D), "hipMalloc(rotation operands)");
+    fkv::PackSrc src{};
+    src.near_k = near_k;
+    src.near_v = near_v;
+    src.near_dtype = near_dtype;
+    src.near_valid = near_valid;
+    src.k_idx = k_idx;
+    src.k_signs = k_signs;
+    src.k_norm = k_norm;
+    src.k_gamma = k_gamma;
+    src.v_packed = v_packed;
+    src.v_scale = v_scale;
+    src.nz_dtype = nz_dtype;
+    src.Pi = Pi;
+    src.S = S;
+    int rc = fkv::attn_begin(h, B, Hkv, D, Na, F, 1, src, spike_margin, st);
     float cb[4] = {0.f, 0.f, 0.f, 0.f};
-    if (!rc) {
-        const int blk = 256;
-        const fkv::BlobLayout L = h->L;
-        hipLaunchKernelGGL(fkv::rot_operand_kernel, dim3(fkv::grid_for(2 * (int64_t)D * D, blk)), dim3(blk), 0, st,
-                           Pi, S, h->tq.rot, D);
-        if (F > 0) {
-            hipLaunchKernelGGL(fkv::tq_pack_k_kernel, dim3(fkv::grid_for((int64_t)B * Hkv * L.F_pad * (D / 32), blk)),
-                               dim3(blk), 0, st, k_idx, k_signs, L, h->blob);
-            hipLaunchKernelGGL(fkv::tq_pack_v_kernel,
-                               dim3(fkv::grid_for((int64_t)B * Hkv * (L.F_pad / fkv::kTile) * D, blk)), dim3(blk), 0,
-                               st, v_packed, L, h->blob);
-            hipLaunchKernelGGL(fkv::tq_pack_sn_kernel, dim3(fkv::grid_for((int64_t)B * Hkv * L.F_pad, blk)),
-                               dim3(blk), 0, st, v_scale, k_norm, k_gamma, nz_dtype, L, h->blob);
-        }
-        rc = check_hip(hipGetLastError(), "turbo pack kernels");
-    }
     if (!rc) rc = check_hip(hipMemcpyAsync(cb, centroids, sizeof(cb), hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
-    if (!rc) rc = fkv::attn_finish(h, st);
+    if (!rc) rc = fkv::attn_finish("fkv_turbo_create", h, st);
     if (!rc) {
+        h->tq.rot = (const uint16_t*)(h->blob + h->L.rot);
         // centroid(c) = alpha + beta*sh + gamma*sl + delta*sh*sl, sh/sl = +-1 bits of c
         const double c0 = cb[0], c1 = cb[1], c2 = cb[2], c3 = cb[3];
         h->tq.alpha = (float)((c0 + c1 + c2 + c3) / 4);

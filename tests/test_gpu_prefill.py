@@ -300,3 +300,68 @@ def test_turbo_values_edges(fkv, D, n, dt, offset):
     want = (codes.reshape(-1, 4) << np.array([0, 2, 4, 6], np.uint8)).sum(-1).astype(np.uint8)
     assert np.array_equal(packed.cpu().numpy(), want)
     assert np.array_equal(scale.cpu().numpy(), sc[:, 0].astype(np.float16))
+
+
+def _moved(t, offset):
+    """A contiguous copy of ``t`` whose storage starts ``offset`` elements in."""
+    flat = torch.empty(t.numel() + offset, dtype=t.dtype, device=t.device)[offset:]
+    flat.copy_(t.reshape(-1))
+    return flat.view(t.shape)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("fmt", ["fp8", "g32", "turbo"])
+@pytest.mark.parametrize("S", [700, 1000])
+def test_blob_from_any_alignment_and_type(fkv, orc, D, fmt, S):
+    """The blob packed from unaligned arrays, and from bf16 / fp32 near tiers,
+    gives the outputs of the aligned fp16 one bit for bit; the near tier
+    comes back as it went in (token counts off the tile edges)."""
+    from foveated_kv_amd import FoveatedKVCache, TierConfig, ext, turbo
+
+    B, H, G = 2, 3, 5
+    rng = np.random.default_rng(S + D)
+    # near values that every type holds exactly
+    k, v = (torch.from_numpy(rng.integers(-31, 32, (B, H, S, D)).astype(np.float16) / 16).cuda() for _ in range(2))
+    q = torch.from_numpy(rng.standard_normal((B, H * G, 1, D)).astype(np.float16)).cuda()
+    cache = FoveatedKVCache(TierConfig(compress_method="turbo" if fmt == "turbo" else "fp8",
+                                       v_group=32 if fmt == "g32" else 0))
+    cache.update(k, v, 0)
+    cache.compress()
+    lay = cache.layers[0]
+
+    def build(near=lambda t: t, other=lambda t: t):
+        if fmt == "turbo":
+            tc = lay._turbo_constants
+            return turbo.TurboFoveatedHandle(
+                near(lay.near_k), near(lay.near_v), *(other(t) for t in (
+                    lay.turbo_far_k_indices, lay.turbo_far_k_signs, lay.turbo_far_k_norm, lay.turbo_far_k_gamma,
+                    lay.turbo_far_v_packed, lay.turbo_far_v_scale)), lay.near_valid, tc.Pi, tc.S, tc.centroids, 10.0)
+        return ext.FoveatedHandle(near(lay.near_k), near(lay.near_v), *(other(t) for t in (
+            lay.far_k, lay.far_v, lay.far_v_scale, lay.far_v_zero)), lay.near_valid, 10.0)
+
+    flush(f"blob alignment and types D={D} {fmt} S={S} near={lay.near_k.shape[2]}")
+    want = build()(q)
+    for near, other in ((lambda t: _moved(t, 1), lambda t: _moved(t, 3)), (lambda t: t.bfloat16(), lambda t: t),
+                        (lambda t: _moved(t.float(), 1), lambda t: t), (lambda t: t.float(), lambda t: _moved(t, 1))):
+        h = build(near, other)
+        got = h(q)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        ek, ev = h.export_near()
+        assert torch.equal(ek, lay.near_k) and torch.equal(ev, lay.near_v)
+
+
+def test_far_nan_codes_refused(fkv):
+    """A NaN code anywhere in the far keys (first, last, inside a dword) is refused."""
+    from foveated_kv_amd import _lib, ext
+
+    k = torch.randn((1, 2, 300, 64), device="cuda").half()
+    cl = ext.CompressHandle(_cfg()).compress_layer(k, k)
+    flat = cl.far_k.view(-1)
+    for at in (0, 5, flat.numel() // 2 + 2, flat.numel() - 1):
+        for code in (0x7F, 0xFF):
+            old = flat[at].clone()
+            flat[at] = code
+            with pytest.raises(Exception, match="NaN codes"):
+                ext.FoveatedHandle(cl.near_k, cl.near_v, cl.far_k, cl.far_v, cl.far_v_scale, cl.far_v_zero, cl.near_valid)
+            flat[at] = old
+    ext.FoveatedHandle(cl.near_k, cl.near_v, cl.far_k, cl.far_v, cl.far_v_scale, cl.far_v_zero, cl.near_valid)
