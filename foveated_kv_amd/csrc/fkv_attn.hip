@@ -877,11 +877,16 @@ static int env_int(const char* name, int dflt) {
     return v && *v ? atoi(v) : dflt;
 }
 
-// Workgroups per (b, kv_head, head group): enough to fill 256 CUs, at least
-// two tiles per wave.
+// Workgroups per (b, kv_head, head group): as many as fit the target (the
+// CUs) in one round, at least two tiles per wave.  Rounded down: a workgroup
+// has a CU to itself, so the few past 256 of a launch rounded up start when
+// the others end and the chip runs two rounds for one (12 rows, 8,192-11,003
+// tokens: 22 splits = 264 workgroups 20.8-27.4 us, 21 = 252 14.9-19.3 us; 24
+// rows 21.6 against 14.8, 72 rows 38.1 against 26.3, 130 rows of 1 split
+// 46.8 us against 64.4 with 2; more rounds of shorter splits were slower too).
 static int plan_splits(const BlobLayout& L, int rows, int n_dec, int target, int waves = kWavesPerGroup) {
     const int tiles = (int)(cdiv(L.Na, kTile) + cdiv(L.F, kTile) + cdiv(n_dec, kTile));
-    int s = (int)cdiv(target, rows > 0 ? rows : 1);
+    int s = target / (rows > 0 ? rows : 1);
     const int cap = tiles / (2 * waves);
     if (s > cap) s = cap;
     if (s > kMaxSplits) s = kMaxSplits;

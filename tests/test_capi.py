@@ -227,3 +227,23 @@ def test_xcd_rule_fit_and_watch_words():
     assert viol([1] + [0] * 64) == 1                 # a merge saw another XCD's record
     assert viol([0, 0, 3, 0, 1]) == 2                # counters no merge re-armed
     assert viol([1, 2]) == 2
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+def test_launch_plan_is_one_round_of_the_chip(fmt):
+    """A launch never has a few workgroups more than the target (each has a CU
+    to itself: they would run as a second round): rows x splits stays within
+    it, unless there are more rows than that, which are not split."""
+    from foveated_kv_amd import _lib
+
+    lib = _lib.load()
+    out = (ctypes.c_int64 * 8)()
+    for B in (1, 2, 3, 5, 7, 12, 13, 24, 33, 70):
+        for Hkv in (1, 2, 3, 8, 10):
+            for G in (1, 4, 5, 8, 20):
+                for S in (600, 11003, 65536):
+                    assert lib.fkv_attn_plan(B, Hkv, 128, S // 7, S, Hkv * G, 0, 256, fmt, out) == _lib.FKV_OK
+                    rows, splits = out[1], out[2]
+                    assert splits >= 1 and (rows * splits <= 256 or splits == 1), (B, Hkv, G, S, rows, splits)
+                    # and no CU is left out that one more split per row would fill
+                    assert (splits + 1) * rows > 256 or splits == 64 or splits >= (S // 7 // 64 + S // 64) // 16
