@@ -32,10 +32,12 @@ namespace fkv {
 struct BlobLayout {
     int B, Hkv, D, Na, F, Na_pad, F_pad;
     int fmt;  // 0: fp8-E4M3 K / INT4 V far records, 1: TurboQuant, 2: fp8 K / group-32 INT4 V
-    size_t near_k, near_v, far, far_rec, near_valid, kscale, rot, total;
+    size_t near_k, near_v, far, far_rec, near_valid, kscale, total;
 };
 
 BlobLayout make_layout(int B, int Hkv, int D, int Na, int F, int fmt = 0);
+// Byte offset of the rotation operands of a fmt 1 blob: its last 4 * D * D bytes.
+__host__ __device__ inline size_t tq_rot_section(const BlobLayout& L) { return L.total - (size_t)4 * L.D * L.D; }
 
 // Far records are stored tile-major across (batch, kv head) rows: record
 // (bkv, tile) sits at index tile * B*Hkv + bkv, so workgroups of different

@@ -74,7 +74,7 @@ BlobLayout make_layout(int B, int Hkv, int D, int Na, int F, int fmt) {
     L.far = place(bkv * (L.F_pad / kTile) * L.far_rec);
     L.near_valid = place(((size_t)Hkv + 1) * 4);
     L.kscale = place(bkv * 4);
-    L.rot = place(fmt == 1 ? (size_t)4 * D * D : 0);
+    if (fmt == 1) place((size_t)4 * D * D);  // tq_rot_section
     L.total = off;
     return L;
 }

@@ -35,7 +35,7 @@ __global__ void pack_header_kernel(PackSrc s, BlobLayout L, uint8_t* __restrict_
     if (L.fmt == 1 && i < 2 * DD) {
         // Pi and S -> the query rotation's fp16 operands
         const int mat = (int)(i / DD), r = (int)(i / L.D % L.D), c = (int)(i % L.D);
-        ((uint16_t*)(blob + L.rot))[tq_rot_index(L.D, mat, r, c)] = f2h((mat ? s.S : s.Pi)[(int64_t)r * L.D + c]);
+        ((uint16_t*)(blob + tq_rot_section(L)))[tq_rot_index(L.D, mat, r, c)] = f2h((mat ? s.S : s.Pi)[(int64_t)r * L.D + c]);
     }
 }
 

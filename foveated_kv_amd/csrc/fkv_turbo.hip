@@ -484,7 +484,7 @@ int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t 
     if (!rc) rc = check_hip(hipMemcpyAsync(cb, centroids, sizeof(cb), hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
     if (!rc) rc = fkv::attn_finish("fkv_turbo_create", h, st);
     if (!rc) {
-        h->tq.rot = (const uint16_t*)(h->blob + h->L.rot);
+        h->tq.rot = (const uint16_t*)(h->blob + fkv::tq_rot_section(h->L));
         // centroid(c) = alpha + beta*sh + gamma*sl + delta*sh*sl, sh/sl = +-1 bits of c
         const double c0 = cb[0], c1 = cb[1], c2 = cb[2], c3 = cb[3];
         h->tq.alpha = (float)((c0 + c1 + c2 + c3) / 4);
