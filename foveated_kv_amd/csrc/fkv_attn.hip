@@ -856,7 +856,8 @@ namespace fkv {
 // unit (default instruction scheduling); the fp8 and group-32 ones come
 // from attn_kernel_one_quad / attn_kernel_quads.
 template <int D>
-static AttnKernel pick_attn_turbo(int nq) {
+static AttnKernel pick_attn_turbo(int nq, bool qc) {
+    if (qc) return nq == 1 ? attn_kernel<D, 1, 1, false, false, true> : attn_kernel<D, 2, 1, false, false, true>;
     switch (nq) {
         case 1: return attn_kernel<D, 1, 1>;
         case 2: return attn_kernel<D, 2, 1>;
@@ -1268,18 +1269,26 @@ int attn_call(const char* fn, fkv_attn* h, const void* query, int32_t q_dtype, i
     if (p.ws_floats > w.ws_floats || p.rows > (int)w.arrive_n)
         return set_error(name + ": launch plan exceeds the workspace (internal error)");
     const int hpg = p.hpg, head_groups = p.head_groups, ng_max = p.ng_max, rows = p.rows, splits = p.splits;
-    const uint16_t* q16 = (const uint16_t*)query;
+    // rows of one or two head quads round a bf16 or float32 query in the
+    // attention kernel's prologue (QC kernels; GQA groups of up to 8 heads); a
+    // cast launch remains for wider rows (rare: not worth their kernels), where
+    // the top-K selection reads the query as well, and for a query that the
+    // prologue's dword loads could not take
+    const bool qc = q_dtype != FKV_F16 && !topk && ng_max <= 8 && ((uintptr_t)query & 3) == 0;
+    const bool cast = q_dtype != FKV_F16 && !qc;
+    const void* qk = query;
     const int64_t qn = (int64_t)L.B * Hq * L.D;
-    if (q_dtype != FKV_F16) {
+    if (cast) {
         if ((size_t)qn > w.qbuf_n) return set_error(name + ": query exceeds the workspace (internal error)");
         hipLaunchKernelGGL(fkv::cast_to_f16_kernel, dim3(fkv::grid_for(qn, 256)), dim3(256), 0, st, query,
                            q_dtype, qn, w.qbuf);
-        q16 = w.qbuf;
+        qk = w.qbuf;
     }
     fkv::AttnArgs a;
     a.blob = h->blob;
     a.L = L;
-    a.q = q16;
+    a.q = (const uint16_t*)qk;
+    a.q_dtype = q_dtype;
     a.dec_k = (const uint16_t*)decode_k;
     a.dec_v = (const uint16_t*)decode_v;
     a.n_dec = n_dec_dev ? 0 : n_decode;
@@ -1358,9 +1367,9 @@ int attn_call(const char* fn, fkv_attn* h, const void* query, int32_t q_dtype, i
     a.tq_lvl = h->tq.lvl;
     const int nq = (ng_max + 3) / 4;
     const bool ext = topk || h->has_kscale;  // the kernels that carry the extensions
-    fkv::AttnKernel k = L.fmt == 1 ? (L.D == 128 ? fkv::pick_attn_turbo<128>(nq) : fkv::pick_attn_turbo<64>(nq))
-                        : nq == 1  ? fkv::attn_kernel_one_quad(L.D, L.fmt, ext, topk)
-                                   : fkv::attn_kernel_quads(L.D, L.fmt, nq, ext, topk);
+    fkv::AttnKernel k = L.fmt == 1 ? (L.D == 128 ? fkv::pick_attn_turbo<128>(nq, qc) : fkv::pick_attn_turbo<64>(nq, qc))
+                        : nq == 1  ? fkv::attn_kernel_one_quad(L.D, L.fmt, ext, topk, qc)
+                                   : fkv::attn_kernel_quads(L.D, L.fmt, nq, ext, topk, qc);
     hipLaunchKernelGGL(k, grid, block, 0, st, a);
     if (splits > 1 && !fused_merge) {
         const dim3 mgrid(rows, ng_max);
@@ -1371,7 +1380,7 @@ int attn_call(const char* fn, fkv_attn* h, const void* query, int32_t q_dtype, i
         fkv::SelectArgs sa;
         sa.blob = h->blob;
         sa.L = L;
-        sa.q = q16;
+        sa.q = (const uint16_t*)qk;  // fp16 (cast above)
         sa.Hq = Hq;
         sa.G = G;
         sa.K = h->spike_k;

@@ -70,7 +70,7 @@ __host__ __device__ constexpr int attn_waves(int D, int NQ, int fmt) {
 struct AttnArgs {
     const uint8_t* blob;
     BlobLayout L;
-    const uint16_t* q;      // (B, Hq, D) fp16
+    const uint16_t* q;      // (B, Hq, D) fp16 (QC kernels: q_dtype)
     const uint16_t* dec_k;  // (B, Hkv, dec_stride, D) fp16 rows, the first n_dec valid
     const uint16_t* dec_v;
     int n_dec;
@@ -115,6 +115,7 @@ struct AttnArgs {
     // per-head fp8 key scales, (B*Hkv) fp32 in the blob; NULL for a handle
     // whose keys are unscaled (no load then: the scale is 1)
     const float* kscale;
+    int q_dtype;  // QC kernels: FKV_BF16 or FKV_F32, rounded to fp16 in the prologue
 #ifdef FKV_PHASE_STAMPS
     unsigned long long* stamps;  // kStampSlots per workgroup (fkv_phase_stamps)
 #endif
@@ -276,6 +277,42 @@ __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_b
 // 32-bit LDS address of a pointer into a __shared__ array.
 __device__ inline uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(const FKV_LDS void*)p;
+}
+
+// A wave's query operand copy (QW dwords) rounded to fp16 in LDS: from bf16
+// in place, from float32 out of raw (2 QW dwords in the same order).  The
+// rounding of a separate cast launch: a captured step of eight 4K layers with
+// bf16 queries 101.6 -> 88.9 us, one call with float32 ones at 11,003 tokens
+// 24.9 -> 21.5.  Asm blocks that wait for their own LDS operations: the
+// compiler would drain the tile DMA in flight around ordinary ones.
+template <int QW>
+__device__ inline void query_to_f16(int dtype, uint8_t* qw, const uint8_t* raw, int lane) {
+#pragma unroll
+    for (int k = 0; k < QW / kWave; k += 2) {
+        const uint32_t dst = lds_addr(qw) + (k * kWave + lane) * 4;
+        uint32_t o0, o1;
+        if (dtype == FKV_BF16) {
+            uint32_t x, y;
+            asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %2 offset:256\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(x), "=&v"(y)
+                         : "v"(dst)
+                         : "memory");
+            o0 = (uint32_t)f2h(__uint_as_float(x << 16)) | ((uint32_t)f2h(__uint_as_float(x & 0xFFFF0000u)) << 16);
+            o1 = (uint32_t)f2h(__uint_as_float(y << 16)) | ((uint32_t)f2h(__uint_as_float(y & 0xFFFF0000u)) << 16);
+        } else {
+            const uint32_t src = lds_addr(raw) + (k * kWave + lane) * 8;
+            fkv_v2u x, y;
+            asm volatile("ds_read_b64 %0, %2\n\tds_read_b64 %1, %2 offset:512\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(x), "=&v"(y)
+                         : "v"(src)
+                         : "memory");
+            o0 = (uint32_t)f2h(__uint_as_float(x.x)) | ((uint32_t)f2h(__uint_as_float(x.y)) << 16);
+            o1 = (uint32_t)f2h(__uint_as_float(y.x)) | ((uint32_t)f2h(__uint_as_float(y.y)) << 16);
+        }
+        asm volatile("ds_write_b32 %0, %1\n\tds_write_b32 %0, %2 offset:256\n\ts_waitcnt lgkmcnt(0)" ::"v"(dst), "v"(o0),
+                     "v"(o1)
+                     : "memory");
+    }
 }
 
 // q as the B operand of the score MFMA, in LDS as [qd][s][j][4 halves].
@@ -2188,7 +2225,11 @@ __device__ inline void tq_rotate_query(const AttnArgs& a, const TqRotation<D>& r
 // its registers; each kernel has one far-tile body (a run-time choice
 // between two bodies in the stream loop had cost the extension kernels
 // ~1.2 us at C5 even where they took the plain one).
-template <int D, int NQ, int FMT, bool EXT = false, bool SPK = false>
+// QC: the query is bf16 or float32 (a.q_dtype) and rounded to fp16 in the
+// prologue instead of by a cast launch before this one; a template of its own,
+// because the run-time choice in the prologue of every kernel cost fp16
+// queries 0.5 us (C3-16K) to 1.1 us (C4).
+template <int D, int NQ, int FMT, bool EXT = false, bool SPK = false, bool QC = false>
 __global__ __launch_bounds__(64 * attn_waves(D, NQ, FMT)) void attn_kernel(AttnArgs a) {
     static_assert(EXT || !SPK, "the top-K kernels are extension kernels");
     constexpr int WPG = attn_waves(D, NQ, FMT);  // waves of the workgroup
@@ -2289,16 +2330,30 @@ __global__ __launch_bounds__(64 * attn_waves(D, NQ, FMT)) void attn_kernel(AttnA
     // Dword w = ((qd * NS + s) * 4 + j) * 2 + e holds dims 4s + 2e, +1 of
     // head 4qd + j; heads past the group read head 0's row (finite values
     // whose results are never written).  TurboQuant stages its own query.
+    // A bf16 query comes the same way, a float32 one (two dwords for one) to
+    // the ring's second slot, which no tile uses before the query has landed;
+    // both are rounded to fp16 in LDS then (query_to_f16).
+    constexpr int QW = NQ * NS * 8;  // fp16 operand dwords
     if constexpr (!TQ) {
-        constexpr int QW = NQ * NS * 8;
-        static_assert(QW % kWave == 0, "whole-wave query DMA");
+        static_assert(QW % (2 * kWave) == 0, "whole-wave query DMA");
+        static_assert(QW * 8 <= SLOT, "a float32 query fits a ring slot");
         uint8_t* qw = (uint8_t*)(qs + wave * QCOPY);  // this wave's copy (wave-uniform)
+        if (QC && a.q_dtype == FKV_F32) {
 #pragma unroll
-        for (int k = 0; k < QW / kWave; k++) {
-            const int wd = k * kWave + lane, e = wd & 1, jj = (wd >> 1) & 3, s = (wd >> 3) % NS;
-            const int h = 4 * ((wd >> 3) / NS) + jj;
-            const uint16_t* src = a.q + ((int64_t)b * a.Hq + head0 + (h < ng ? h : 0)) * D + 4 * s + 2 * e;
-            __builtin_amdgcn_global_load_lds((const void*)src, (FKV_LDS void*)(qw + k * kWave * 4), 4, 0, 0);
+            for (int k = 0; k < 2 * QW / kWave; k++) {
+                const int r = k * kWave + lane, e = r & 3, jj = (r >> 2) & 3, s = (r >> 4) % NS;
+                const int h = 4 * ((r >> 4) / NS) + jj;
+                const float* src = (const float*)a.q + ((int64_t)b * a.Hq + head0 + (h < ng ? h : 0)) * D + 4 * s + e;
+                __builtin_amdgcn_global_load_lds((const void*)src, (FKV_LDS void*)(ring + SLOT + k * kWave * 4), 4, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < QW / kWave; k++) {
+                const int wd = k * kWave + lane, e = wd & 1, jj = (wd >> 1) & 3, s = (wd >> 3) % NS;
+                const int h = 4 * ((wd >> 3) / NS) + jj;
+                const uint16_t* src = a.q + ((int64_t)b * a.Hq + head0 + (h < ng ? h : 0)) * D + 4 * s + 2 * e;
+                __builtin_amdgcn_global_load_lds((const void*)src, (FKV_LDS void*)(qw + k * kWave * 4), 4, 0, 0);
+            }
         }
     }
     // the wave's first two far tiles need no device state either.  Behind
@@ -2327,7 +2382,8 @@ __global__ __launch_bounds__(64 * attn_waves(D, NQ, FMT)) void attn_kernel(AttnA
             const int i = (threadIdx.x + NT * k) % (NQ * NS * 16);
             const int e = i & 3, jj = (i >> 2) & 3, sq = i >> 4;
             const int s = sq % NS, h = 4 * (sq / NS) + jj;
-            tq_q[k] = a.q[((int64_t)b * a.Hq + head0 + (h < ng ? h : 0)) * D + 4 * s + e];
+            const int64_t qi = ((int64_t)b * a.Hq + head0 + (h < ng ? h : 0)) * D + 4 * s + e;
+            tq_q[k] = QC ? load_as_f16(a.q, qi, a.q_dtype) : a.q[qi];
         }
     }
     // the second far tile follows the query wait below (TurboQuant: in the
@@ -2394,7 +2450,13 @@ __global__ __launch_bounds__(64 * attn_waves(D, NQ, FMT)) void attn_kernel(AttnA
         // the query DMA is this wave's oldest vector-memory op: wait for it
         // but not for the ring (the wave's own copy: no barrier), then issue
         // the second far tile (QFIRST rows: the first two)
-        if (QFIRST) {
+        if constexpr (QC) {
+            if (!QFIRST && un.nf > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FAR_OPS) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            query_to_f16<QW>(a.q_dtype, (uint8_t*)(qs + wave * QCOPY), ring + SLOT, lane);
+            if (QFIRST && un.nf > 0) issue(0);
+            if (early1) issue(1);
+        } else if (QFIRST) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (un.nf > 0) issue(0);
             if (early1) issue(1);
@@ -2698,7 +2760,7 @@ typedef void (*AttnKernel)(AttnArgs);
 // The fp8 and group-32 attention kernels (fmt 0, 2) of rows of one head
 // quad (fkv_attn_q1.hip; EXT: fkv_attn_q1x.hip) and of nq = 2..4 quads
 // (fkv_attn_qn.hip, fkv_attn_qnx.hip); spk picks the top-K kernels.
-AttnKernel attn_kernel_one_quad(int D, int fmt, bool ext, bool spk);
-AttnKernel attn_kernel_quads(int D, int fmt, int nq, bool ext, bool spk);
+AttnKernel attn_kernel_one_quad(int D, int fmt, bool ext, bool spk, bool qc);
+AttnKernel attn_kernel_quads(int D, int fmt, int nq, bool ext, bool spk, bool qc);  // qc: nq <= 2
 
 }  // namespace fkv

@@ -3,7 +3,8 @@
 // A translation unit of their own so that the Makefile can compile them
 // with the iterative-ilp instruction scheduling, which measured fastest for
 // them (C5 29.9 -> 29.0 us).  Their extension-carrying twins (per-head key
-// scales, top-K spikes) are in fkv_attn_qnx.hip.
+// scales, top-K spikes) and the ones for bf16 / float32 queries are in
+// fkv_attn_qnx.hip.
 #include "fkv_attn_kernel.h"
 
 namespace fkv {
@@ -21,10 +22,10 @@ AttnKernel pick(int nq) {
 
 }  // namespace
 
-AttnKernel attn_kernel_quads_ext(int D, int fmt, int nq, bool spk);
+AttnKernel attn_kernel_quads_ext(int D, int fmt, int nq, bool spk, bool qc);
 
-AttnKernel attn_kernel_quads(int D, int fmt, int nq, bool ext, bool spk) {
-    if (ext) return attn_kernel_quads_ext(D, fmt, nq, spk);
+AttnKernel attn_kernel_quads(int D, int fmt, int nq, bool ext, bool spk, bool qc) {
+    if (ext || qc) return attn_kernel_quads_ext(D, fmt, nq, spk, qc);
     if (D == 128) return fmt == 2 ? pick<128, 2>(nq) : pick<128, 0>(nq);
     return fmt == 2 ? pick<64, 2>(nq) : pick<64, 0>(nq);
 }
