@@ -290,10 +290,8 @@ __global__ __launch_bounds__(kWave) void kscale_finish_kernel(const float* __res
 // fp32 importance -> unsigned key with the same order; NaN ranks below
 // -inf, -0 equals +0.
 __device__ inline uint32_t order_key(float f) {
-    if (f != f) return 0u;
-    uint32_t b = __float_as_uint(f);
-    if (b == 0x80000000u) b = 0u;
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+    const uint32_t b = __float_as_uint(f + 0.0f);  // -0 + 0 = +0
+    return f != f ? 0u : b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
 }
 
 // Middle token i's rank key: importance, then position (the later token
@@ -316,24 +314,33 @@ __device__ inline void fixed_slots(int32_t* nrow, int S, const fkv_tiers& tb, in
     }
 }
 
+// No instruction: keeps what is computed from x after this point after it.
+// (Over R registers the compiler otherwise computes every lane mask of a loop
+// first, or keeps one loop's for the next, and spills them.)
+#define PART_PIN(x) asm volatile("" : "+v"(x))
+
 constexpr int kPartRegs = 64;  // most tokens per thread held in registers
 constexpr int kPartBits = 11, kPartBins = 1 << kPartBits, kPartCopies = 4;
 
 // Partition of a (batch, head) whose middle fits the workgroup's registers,
 // R tokens per thread (at most kPartThreads * R in all).  Bound by one CU's
-// chain of passes, not by memory, so the row is read once: wave w holds
-// order_key of the middle's tokens w * R * 64 .. in position order (register
-// r: 64 consecutive tokens).  A radix select of 11 + 11 + 10 bits over the
-// registers (LDS histograms, one per wave modulo kPartCopies; one per lane
-// modulo 16, free of bank conflicts, was no faster: the passes are bound by
-// their vector instructions) finds
-// the near_from_mid-th largest key v and how many tokens equal to it stay
-// near (the last ones in position order: the later token wins a tie, which
-// is what the 64-bit rank key orders by).  The compaction needs no block
-// step per chunk: a token's far row is its position less the near tokens
-// before it, and those follow from one scan of the waves' counts and
-// ballots.  64K tokens x 8 heads: 190 us with 8-bit passes that each re-read
-// the row and a block scan per 1,024 tokens, 53 us here.
+// vector instructions, not by memory, so the row is read once and as little
+// as possible is done per token: wave w holds order_key of the middle's
+// tokens w * R * 64 .. in position order (register r: 64 consecutive
+// tokens).  A radix select of 11 + 11 + 10 bits over the registers (LDS
+// histograms, one per wave modulo kPartCopies; one per lane modulo 16, free
+// of bank conflicts, was no faster) finds the near_from_mid-th largest key v
+// and how many tokens equal to it stay near (the last ones in position
+// order: the later token wins a tie, which is what the 64-bit rank key
+// orders by).  The compaction needs no block step per chunk: a token's far
+// row is its position less the near tokens before it, and those follow from
+// one scan of the waves' counts and ballots.  Registers past the middle hold
+// the lowest key: they come after every token in position order, so they
+// only take part in a tie at that key, where they are counted out, and their
+// places lie past the near and far rows (a range test per token and pass
+// made half of the instructions).  64K tokens x 8 heads: 190 us with 8-bit
+// passes that each re-read the row and a block scan per 1,024 tokens, 53 us
+// with the range tests (and their lane masks spilled), 40 us here.
 template <int R>
 __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const float* __restrict__ imp, int S,
                                                                      fkv_tiers tb, int32_t* __restrict__ near_idx,
@@ -346,116 +353,139 @@ __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const floa
     const int npad = tb.n_near_padded, F = tb.far_count, m0 = tb.mid_start;
     const int mlen = tb.mid_end > tb.mid_start ? tb.mid_end - tb.mid_start : 0;
     const int k = tb.near_from_mid;
-    const float* row = imp + (int64_t)bh * S + m0;
     int32_t* nrow = near_idx + (int64_t)bh * npad;
     int32_t* frow = far_idx + (int64_t)bh * F;
-    const int i0 = wave * R * kWave + lane;  // the lane's first token of the middle
-    const bool all = k >= mlen, none = k <= 0;
-    uint32_t key[R];
-    uint32_t v = 0, equal_far = 0;  // near <=> key > v, or key == v and not among the first equal_far such
-    if (!all && !none) {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int i = i0 + r * kWave;
-            key[r] = order_key(i < mlen ? row[i] : 0.f);
+    fixed_slots(nrow, S, tb, tid);
+    if (k >= mlen || k <= 0) {  // the whole middle is near, or far
+        for (int i = tid; i < mlen; i += kPartThreads) {
+            if (k > 0) nrow[tb.n_sinks + i] = m0 + i;
+            else if (i < F) frow[i] = m0 + i;
         }
-        fixed_slots(nrow, S, tb, tid);
-        uint32_t rem = k;
-        constexpr int shift[3] = {32 - kPartBits, 32 - 2 * kPartBits, 0};
-        constexpr int bits[3] = {kPartBits, kPartBits, 32 - 2 * kPartBits};
+        return;
+    }
+    const int i0 = wave * R * kWave + lane;  // the lane's first token of the middle
+    const float* row = imp + (int64_t)bh * S + m0;
+    uint32_t key[R];
+    {
+        float f[R];
 #pragma unroll
-        for (int p = 0; p < 3; p++) {
-            for (int i = tid; i < kPartCopies * kPartBins; i += kPartThreads) (&hist[0][0])[i] = 0;
-            __syncthreads();
-            const uint32_t high = p == 0 ? 0u : ~0u << (shift[p] + bits[p]);  // digits already known
+        for (int r = 0; r < R; r++) f[r] = row[min(i0 + r * kWave, mlen - 1)];
+#pragma unroll
+        for (int r = 0; r < R; r++) key[r] = order_key(f[r]);
+        if ((wave + 1) * R * kWave > mlen)
 #pragma unroll
             for (int r = 0; r < R; r++)
-                if (i0 + r * kWave < mlen && ((key[r] ^ v) & high) == 0)
-                    atomicAdd(&hist[wave % kPartCopies][(key[r] >> shift[p]) & ((1u << bits[p]) - 1)], 1u);
-            __syncthreads();
-            // thread t takes bins top - 2t and top - 2t - 1: an inclusive scan
-            // over the threads counts the keys from the top bin down
-            const int hi = kPartBins - 1 - 2 * tid;
-            uint32_t c1 = 0, c0 = 0;
+                if (i0 + r * kWave >= mlen) key[r] = 0;
+    }
+    uint32_t v = 0, rem = k;
+    constexpr int shift[3] = {32 - kPartBits, 32 - 2 * kPartBits, 0};
+    constexpr int bits[3] = {kPartBits, kPartBits, 32 - 2 * kPartBits};
 #pragma unroll
-            for (int q = 0; q < kPartCopies; q++) {
-                c1 += hist[q][hi];
-                c0 += hist[q][hi - 1];
-            }
-            uint32_t inc = c1 + c0;
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) {
-                const uint32_t t = __shfl_up(inc, d, kWave);
-                if (lane >= d) inc += t;
-            }
-            if (lane == kWave - 1) wtot[wave] = inc;
-            __syncthreads();
-            uint32_t above = inc - c1 - c0;
-#pragma unroll
-            for (int w = 0; w < kPartWaves; w++)
-                if (w < wave) above += wtot[w];
-            if (above < rem && above + c1 >= rem) {
-                s_bin = hi;
-                s_rem = rem - above;
-                s_cnt = c1;
-            } else if (above + c1 < rem && above + c1 + c0 >= rem) {
-                s_bin = hi - 1;
-                s_rem = rem - above - c1;
-                s_cnt = c0;
-            }
-            __syncthreads();
-            v |= s_bin << shift[p];
-            rem = s_rem;
-        }
-        equal_far = s_cnt - rem;
-        uint32_t gt = 0, eq = 0;  // the wave's tokens above and at v
+    for (int p = 0; p < 3; p++) {
+        for (int i = tid; i < kPartCopies * kPartBins; i += kPartThreads) (&hist[0][0])[i] = 0;
+        __syncthreads();
+        uint32_t* const h = hist[wave % kPartCopies];
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const bool in = i0 + r * kWave < mlen;
-            gt += __popcll(__ballot(in && key[r] > v));
-            eq += __popcll(__ballot(in && key[r] == v));
-        }
-        if (lane == 0) {
-            wgt[wave] = gt;
-            weq[wave] = eq;
+            PART_PIN(key[r]);
+            if (p == 0 || (key[r] ^ v) >> (shift[p] + bits[p]) == 0)  // the digits already known
+                atomicAdd(&h[(key[r] >> shift[p]) & ((1u << bits[p]) - 1)], 1u);
         }
         __syncthreads();
-    } else {
-        fixed_slots(nrow, S, tb, tid);
-    }
-    uint32_t near_before = 0, eq_before = 0;  // in the waves before this one
-    if (!all && !none) {
+        // thread t takes bins top - 2t and top - 2t - 1: an inclusive scan
+        // over the threads counts the keys from the top bin down
+        const int hi = kPartBins - 1 - 2 * tid;
+        uint32_t c1 = 0, c0 = 0;
+#pragma unroll
+        for (int q = 0; q < kPartCopies; q++) {
+            c1 += hist[q][hi];
+            c0 += hist[q][hi - 1];
+        }
+        uint32_t inc = c1 + c0;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const uint32_t t = __shfl_up(inc, d, kWave);
+            if (lane >= d) inc += t;
+        }
+        if (lane == kWave - 1) wtot[wave] = inc;
+        __syncthreads();
+        uint32_t above = inc - c1 - c0;
 #pragma unroll
         for (int w = 0; w < kPartWaves; w++)
-            if (w < wave) {
-                near_before += wgt[w];
-                eq_before += weq[w];
-            }
-        near_before += eq_before > equal_far ? eq_before - equal_far : 0u;
-    } else if (all) {
-        near_before = min(wave * R * kWave, mlen);
+            if (w < wave) above += wtot[w];
+        if (above < rem && above + c1 >= rem) {
+            s_bin = hi;
+            s_rem = rem - above;
+            s_cnt = c1;
+        } else if (above + c1 < rem && above + c1 + c0 >= rem) {
+            s_bin = hi - 1;
+            s_rem = rem - above - c1;
+            s_cnt = c0;
+        }
+        __syncthreads();
+        v |= (uint32_t)__builtin_amdgcn_readfirstlane((int)s_bin) << shift[p];
+        rem = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_rem);
     }
+    // tokens equal to v that stay far (the registers past the middle are not tokens)
+    const uint32_t equal_far = s_cnt - (v == 0 ? (uint32_t)(kPartThreads * R - mlen) : 0u) - rem;
+    // lane r: which of register r's tokens lie above v (near) and at v
+    static_assert(R <= kWave, "a lane per register");
+    uint32_t nlo = 0, nhi = 0, elo = 0, ehi = 0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const int i = i0 + r * kWave;
-        const bool in = i < mlen;
-        bool nf = in && all;
-        if (!all && !none) {
-            const uint64_t em = __ballot(in && key[r] == v);
-            const uint32_t rank = eq_before + __builtin_amdgcn_mbcnt_hi((uint32_t)(em >> 32),
-                                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)em, 0u));
-            nf = in && (key[r] > v || (key[r] == v && rank >= equal_far));
-            eq_before += __popcll(em);
+        PART_PIN(key[r]);
+        const uint64_t g = __ballot(key[r] > v), e = __ballot(key[r] == v);
+        // (a select per lane would need R lane masks; the wait states are those
+        // of a scalar register written by a compare and read here)
+        asm volatile("s_nop 1\n\tv_writelane_b32 %0, %4, %8\n\tv_writelane_b32 %1, %5, %8\n\t"
+                     "v_writelane_b32 %2, %6, %8\n\tv_writelane_b32 %3, %7, %8"
+                     : "+v"(nlo), "+v"(nhi), "+v"(elo), "+v"(ehi)
+                     : "s"((uint32_t)g), "s"((uint32_t)(g >> 32)), "s"((uint32_t)e), "s"((uint32_t)(e >> 32)), "n"(r));
+    }
+    // inclusive sums over the wave's registers
+    auto lane_scan = [&](uint32_t x) {
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const uint32_t t = __shfl_up(x, d, kWave);
+            if (lane >= d) x += t;
         }
-        const uint64_t nm = __ballot(nf);
-        const int before = (int)(near_before + __builtin_amdgcn_mbcnt_hi((uint32_t)(nm >> 32),
-                                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)nm, 0u)));
-        if (nf) {
-            if (before < k) nrow[tb.n_sinks + before] = m0 + i;
-        } else if (in && i - before < F) {
+        return x;
+    };
+    uint64_t near = ((uint64_t)nhi << 32) | nlo, at_v = ((uint64_t)ehi << 32) | elo;
+    const uint32_t eq = __popcll(at_v), eq_upto = lane_scan(eq);
+    const uint32_t gt_all = lane_scan(__popcll(near));
+    if (lane == kWave - 1) {
+        wgt[wave] = gt_all;
+        weq[wave] = eq_upto;
+    }
+    __syncthreads();
+    uint32_t near_before = 0, eq_before = 0;  // in the waves before this one
+#pragma unroll
+    for (int w = 0; w < kPartWaves; w++)
+        if (w < wave) {
+            near_before += wgt[w];
+            eq_before += weq[w];
+        }
+    near_before += eq_before > equal_far ? eq_before - equal_far : 0u;
+    // the first equal_far tokens at v are far: this register's share of them
+    const uint32_t eq_first = eq_before + eq_upto - eq;
+    for (uint32_t n = min(equal_far > eq_first ? equal_far - eq_first : 0u, eq); n > 0; n--) at_v &= at_v - 1;
+    near |= at_v;
+    nlo = (uint32_t)near;
+    nhi = (uint32_t)(near >> 32);
+    const uint32_t upto = near_before + lane_scan(__popcll(near)), first = upto - __popcll(near);
+    nrow += tb.n_sinks;
+#pragma unroll 4
+    for (int r = 0; r < R; r++) {
+        const uint32_t lo = __builtin_amdgcn_readlane(nlo, r), hi = __builtin_amdgcn_readlane(nhi, r);
+        const int before = (int)__builtin_amdgcn_readlane(first, r) +
+                           (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+        const int i = i0 + r * kWave;
+        if (((((uint64_t)hi << 32) | lo) >> lane) & 1) {
+            if (before < k) nrow[before] = m0 + i;
+        } else if (i - before < F) {
             frow[i - before] = m0 + i;
         }
-        near_before += __popcll(nm);
     }
 }
 
