@@ -222,20 +222,50 @@ __host__ __device__ inline int kscale_parts(int F, int D, int BH) {
     return p < 1 ? 1 : (int)p;
 }
 
+// The largest magnitude among elements that are finite as fp16, over packed
+// or single elements: a magnitude's bits order as integers, and adding BIAS
+// makes those that fp16 does not hold as finite numbers negative, which a
+// signed maximum passes over.  Three instructions per dword instead of a
+// conversion, a test and a maximum per element.
+template <int DT>
+struct FiniteMax {
+    // the smallest magnitude that fp16 rounds to infinity (or holds as one)
+    static constexpr uint32_t kTop = DT == FKV_F16 ? 0x7C00u : DT == FKV_BF16 ? 0x4780u : 0x477FF000u;
+    static constexpr uint32_t kBias = DT == FKV_F32 ? 0x80000000u - kTop : 0x8000u - kTop;
+    uint32_t m = DT == FKV_F32 ? kBias : kBias | (kBias << 16);
+    __device__ inline void add(uint32_t w) {
+        if constexpr (DT == FKV_F32) {
+            m = (uint32_t)max((int32_t)m, (int32_t)((w & 0x7FFFFFFFu) + kBias));
+        } else {
+            const fkv_us2 bias = {(uint16_t)kBias, (uint16_t)kBias};
+            const fkv_s2 x = __builtin_bit_cast(fkv_s2, as_us2(w & 0x7FFF7FFFu) + bias);
+            m = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(fkv_s2, m), x));
+        }
+    }
+    // as the fp16 value it is encoded from (rounding keeps the order)
+    __device__ inline float value() const {
+        if constexpr (DT == FKV_F32) return h2f(f2h(__uint_as_float(m - kBias)));
+        const uint32_t lo = (m & 0xFFFFu) - kBias, hi = (m >> 16) - kBias, x = lo > hi ? lo : hi;
+        return DT == FKV_F16 ? h2f((uint16_t)x) : h2f(f2h(bf2f((uint16_t)x)));
+    }
+};
+
 // Bound by the one read of the far keys.  A maximum does not depend on the
 // order, so the rows of a (batch, head) are dealt over as many workgroups as
 // fill the chip (one workgroup per head read 121 MB of keys at 8 heads x 59K
-// rows in 3,690 us: eight CUs; the whole call went from 4,070 to 414 us), and
-// each lane group has kScaleRows rows in flight.  Far rows are positions mid_start.. (far_idx NULL) or
-// far_idx[bh][f]; out-of-range indices are zero rows.
-template <int D>
+// rows in 3,690 us: eight CUs), and each lane group has kScaleRows rows in
+// flight; 41 us with a conversion and a test per element, 36 us here (8 or
+// 16 rows in flight: no faster).
+// Far rows are positions mid_start.. (far_idx NULL) or far_idx[bh][f];
+// out-of-range indices are zero rows.
+template <int D, int DT>
 __global__ __launch_bounds__(kScaleThreads) void kscale_kernel(CompressArgs a, const int32_t* __restrict__ far_idx,
                                                                float* __restrict__ part_max) {
-    constexpr int LPR = D / 8, RPB = kScaleThreads / LPR;
+    constexpr int LPR = D / 8, RPB = kScaleThreads / LPR, NQ = DT == FKV_F32 ? 2 : 1;  // 16-byte loads per lane and row
     __shared__ float red[kScaleThreads / kWave];
     const int bh = blockIdx.y, sub = threadIdx.x % LPR, parts = gridDim.x;
     const int F = a.tb.far_count;
-    float amax = 0.f;
+    FiniteMax<DT> amax;
     for (int64_t f0 = (int64_t)blockIdx.x * kScaleRows * RPB + threadIdx.x / LPR; f0 < F;
          f0 += (int64_t)parts * kScaleRows * RPB) {
         int t[kScaleRows];
@@ -244,26 +274,28 @@ __global__ __launch_bounds__(kScaleThreads) void kscale_kernel(CompressArgs a, c
             const int64_t f = f0 + u * RPB;
             t[u] = f >= F ? -1 : far_idx ? far_idx[(int64_t)bh * F + f] : a.tb.mid_start + (int)f;
         }
-        uint4 kx[kScaleRows];
+        uint4 kx[kScaleRows][NQ];
 #pragma unroll
         for (int u = 0; u < kScaleRows; u++) {
-            const bool in = t[u] >= 0 && t[u] < a.S;
             // a row outside the sequence reads row 0 and is left out below
-            kx[u] = load8(a.k, a.dtype, ((int64_t)bh * a.S + (in ? t[u] : 0)) * D + sub * 8);
+            const bool in = t[u] >= 0 && t[u] < a.S;
+            const uint4* p = (const uint4*)a.k + (((int64_t)bh * a.S + (in ? t[u] : 0)) * LPR + sub) * NQ;
+#pragma unroll
+            for (int q = 0; q < NQ; q++) kx[u][q] = p[q];
         }
 #pragma unroll
         for (int u = 0; u < kScaleRows; u++)
-            if (t[u] >= 0 && t[u] < a.S) {
-                const uint32_t w[4] = {kx[u].x, kx[u].y, kx[u].z, kx[u].w};
+            if (t[u] >= 0 && t[u] < a.S)
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const uint16_t h = (uint16_t)(w[i / 2] >> (16 * (i & 1)));
-                    if (((h >> 10) & 0x1f) != 0x1f) amax = fmaxf(amax, fabsf(h2f(h)));
+                for (int q = 0; q < NQ; q++) {
+                    amax.add(kx[u][q].x);
+                    amax.add(kx[u][q].y);
+                    amax.add(kx[u][q].z);
+                    amax.add(kx[u][q].w);
                 }
-            }
     }
-    amax = wave_max(amax);
-    if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = amax;
+    const float m0 = wave_max(amax.value());
+    if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = m0;
     __syncthreads();
     if (threadIdx.x == 0) {
         float m = 0.f;
@@ -688,10 +720,13 @@ int compress_launch(const char* fn, const fkv_tier_config* cfg, fkv::CompressArg
         // reduced (the compress launch then writes the codes over them); with
         // no far rows there is no buffer: the scales are 1
         float* part_max = a.tb.far_count > 0 ? (float*)a.far_k : nullptr;
-        if (part_max)
-            hipLaunchKernelGGL(D == 128 ? fkv::kscale_kernel<128> : fkv::kscale_kernel<64>,
-                               dim3((unsigned)parts, (unsigned)(B * H)), dim3(fkv::kScaleThreads), 0, st, a,
+        if (part_max) {
+            auto* kern = a.dtype == FKV_F16    ? (D == 128 ? fkv::kscale_kernel<128, FKV_F16> : fkv::kscale_kernel<64, FKV_F16>)
+                         : a.dtype == FKV_BF16 ? (D == 128 ? fkv::kscale_kernel<128, FKV_BF16> : fkv::kscale_kernel<64, FKV_BF16>)
+                                               : (D == 128 ? fkv::kscale_kernel<128, FKV_F32> : fkv::kscale_kernel<64, FKV_F32>);
+            hipLaunchKernelGGL(kern, dim3((unsigned)parts, (unsigned)(B * H)), dim3(fkv::kScaleThreads), 0, st, a,
                                near_idx ? far_idx : nullptr, part_max);
+        }
         hipLaunchKernelGGL(fkv::kscale_finish_kernel, dim3((unsigned)(B * H)), dim3(fkv::kWave), 0, st, part_max,
                            part_max ? parts : 0, far_k_scale);
         a.kscale = far_k_scale;

@@ -58,6 +58,24 @@ def test_k_scale_reduction_edges(fkv, B, H, D, S, near_pct):
         assert np.array_equal(cl.far_k_scale.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("top", [65504.0, 65519.0, 65520.0, 65280.0, 65536.0, float("inf"), float("nan"), 6e-8, 2e-8, 0.0])
+def test_k_scale_finite_in_fp16(fkv, dt, top):
+    """The maximum is over the keys as fp16: one that overflows there is left
+    out, as infinities and NaN are, whatever type it came in."""
+    from foveated_kv_amd import ext
+
+    flush(f"k_scale of {top} from {dt}")
+    k = torch.full((1, 2, 300, 64), 1e-8 if 0 < top < 1e-3 or top == 0 else 3.0)
+    k[0, 0, 150, 5], k[0, 0, 151, 6] = top, -top
+    k = k.to(dt).cuda()
+    cl = ext.CompressHandle(_cfg(k_scale=1)).compress_layer(k, k)
+    far = cl.archive_k.float()
+    far = torch.where(torch.isfinite(far), far.abs(), torch.zeros_like(far)).amax((2, 3)).cpu().numpy()
+    want = np.where(far > 0, far / np.float32(240), np.float32(1)).astype(np.float32)
+    assert np.array_equal(cl.far_k_scale.cpu().numpy(), want)
+
+
 # the edges of the tokens a thread holds (4, 16, 64 per thread of 1,024),
 # the first middle past them, and one whose last wave is partly empty
 @pytest.mark.parametrize("mid", [1, 63, 65, 4096, 4097, 16384, 16385, 50001, 65536, 65537])
