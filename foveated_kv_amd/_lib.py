@@ -93,6 +93,12 @@ SIGNATURES = {
                                            I32, P, F32, P]),
     "fkv_turbo_create": (ctypes.c_int, [ctypes.POINTER(P), I32, I32, I32, I32, I32, P, P, I32, P, P, P, P, P,
                                         P, I32, P, P, P, P, F32, P]),
+    "fkv_attn_blob_bytes": (ctypes.c_int64, [I32, I32, I32, I32, I32, I32]),
+    "fkv_attn_create_at": (ctypes.c_int, [ctypes.POINTER(P), I32, I32, I32, I32, I32, I32, P, P, I32, P, P, P, P,
+                                          I32, P, F32, P, ctypes.c_int64, P]),
+    "fkv_turbo_create_at": (ctypes.c_int, [ctypes.POINTER(P), I32, I32, I32, I32, I32, P, P, I32, P, P, P, P, P,
+                                           P, I32, P, P, P, P, F32, P, ctypes.c_int64, P]),
+    "fkv_tier_index_rows": (ctypes.c_int, [ctypes.POINTER(TiersC), I32, I32, I32, P, P, P]),
     "fkv_turbo_compress_keys": (ctypes.c_int, [P, I32, ctypes.c_int64, I32, P, P, P, P, P, P, P, P, P]),
     "fkv_turbo_compress_values": (ctypes.c_int, [P, I32, ctypes.c_int64, I32, P, P, P]),
     "fkv_attn_call": (ctypes.c_int, [P, P, I32, I32, P, P, I32, P, P, P, P]),

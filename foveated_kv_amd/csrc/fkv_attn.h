@@ -140,6 +140,7 @@ __host__ __device__ inline int64_t tq_rot_index(int D, int mat, int i, int j) {
 struct fkv_attn_impl {
     fkv::BlobLayout L;
     uint8_t* blob = nullptr;
+    bool own_blob = true;   // allocated here, or the caller's (fkv_attn_create_at)
     float margin = 0.f;
     // Call workspace, allocated once by the handle's first call for that
     // call's query-head count and never re-allocated (a captured HIP graph
@@ -147,7 +148,7 @@ struct fkv_attn_impl {
     // decode length can produce, the per-row arrival counters, an fp16 copy
     // of bf16 / f32 queries.
     int ws_hq = 0;          // query heads the workspace is sized for (0: none yet)
-    float* ws = nullptr;    // split partials
+    float* ws = nullptr;    // split partials; arrive and qbuf lie behind them in one allocation
     size_t ws_floats = 0;
     uint16_t* qbuf = nullptr;
     int* arrive = nullptr;  // per-row split arrival counters (zero between calls)
@@ -229,10 +230,10 @@ struct PackSrc {
 };
 // The whole blob from its sources (stream-ordered; every tile, padding included).
 int pack_blob(const PackSrc& s, const BlobLayout& L, uint8_t* blob, hipStream_t st);
-// Handle construction shared by the formats: allocates the blob and packs it
-// (stream-ordered).
-int attn_begin(fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const PackSrc& s, float margin,
-               hipStream_t st);
+// Handle construction shared by the formats: allocates the blob, or takes the
+// caller's (blob_bytes of it), and packs it (stream-ordered).
+int attn_begin(const char* fn, fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const PackSrc& s,
+               float margin, void* blob, int64_t blob_bytes, hipStream_t st);
 // Synchronous end of construction: reads near_valid back for the split plan
 // and whether the far codes held one the reference never emits (FKV_EDATA).
 int attn_finish(const char* fn, fkv_attn_impl* h, hipStream_t st);

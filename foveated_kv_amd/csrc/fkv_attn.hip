@@ -997,16 +997,21 @@ int xcd_rule(int dev, hipStream_t st, int* mod) {
     return FKV_OK;
 }
 
-int attn_begin(fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const PackSrc& s, float margin,
-               hipStream_t st) {
+int attn_begin(const char* fn, fkv_attn_impl* h, int B, int Hkv, int D, int Na, int F, int fmt, const PackSrc& s,
+               float margin, void* blob, int64_t blob_bytes, hipStream_t st) {
     h->L = make_layout(B, Hkv, D, Na, F, fmt);
+    if (blob && (blob_bytes < (int64_t)h->L.total || ((uintptr_t)blob & 255) != 0))
+        return set_error(std::string(fn) + ": the blob must be 256-byte aligned and hold " +
+                         std::to_string(h->L.total) + " bytes");
     h->margin = margin;
     // tuning knobs are read once here, never on the call path
     h->target_wgs = env_int("FKV_TARGET_WGS", 256);
     if (h->target_wgs < 1) h->target_wgs = 1;
     h->fused_merge = env_int("FKV_FUSED_MERGE", 1) != 0;
     int rc = check_hip(hipGetDevice(&h->device), "hipGetDevice");
-    if (!rc) rc = check_hip(hipMalloc(&h->blob, h->L.total), "hipMalloc(blob)");
+    h->own_blob = !blob;
+    h->blob = (uint8_t*)blob;
+    if (!rc && !blob) rc = check_hip(hipMalloc(&h->blob, h->L.total), "hipMalloc(blob)");
     return rc ? rc : pack_blob(s, h->L, h->blob, st);
 }
 
@@ -1036,7 +1041,7 @@ namespace {
 int create_fp8(const char* fn, int fmt, fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
                const void* near_k, const void* near_v, int32_t near_dtype, const uint8_t* far_k,
                const uint8_t* far_v, const void* far_v_scale, const void* far_v_zero, int32_t sz_dtype,
-               const int32_t* near_valid, float spike_margin, void* stream) {
+               const int32_t* near_valid, float spike_margin, void* blob, int64_t blob_bytes, void* stream) {
     const std::string name(fn);
     if (!out) return set_error(name + ": out is NULL");
     *out = nullptr;
@@ -1061,7 +1066,7 @@ int create_fp8(const char* fn, int fmt, fkv_attn** out, int32_t B, int32_t Hkv, 
     src.far_v_scale = far_v_scale;
     src.far_v_zero = far_v_zero;
     src.sz_dtype = sz_dtype;
-    int rc = fkv::attn_begin(h, B, Hkv, D, Na, F, fmt, src, spike_margin, st);
+    int rc = fkv::attn_begin(fn, h, B, Hkv, D, Na, F, fmt, src, spike_margin, blob, blob_bytes, st);
     if (!rc) rc = fkv::attn_finish(fn, h, st);
     if (rc) {
         fkv_attn_destroy(h);
@@ -1081,7 +1086,7 @@ int fkv_attn_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t N
                     const void* far_v_zero, int32_t sz_dtype, const int32_t* near_valid,
                     float spike_margin, void* stream) {
     return create_fp8("fkv_attn_create", 0, out, B, Hkv, D, Na, F, near_k, near_v, near_dtype, far_k, far_v,
-                      far_v_scale, far_v_zero, sz_dtype, near_valid, spike_margin, stream);
+                      far_v_scale, far_v_zero, sz_dtype, near_valid, spike_margin, nullptr, 0, stream);
 }
 
 int fkv_attn_create_g32(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
@@ -1090,7 +1095,23 @@ int fkv_attn_create_g32(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32
                         const void* far_v_zero, int32_t sz_dtype, const int32_t* near_valid,
                         float spike_margin, void* stream) {
     return create_fp8("fkv_attn_create_g32", 2, out, B, Hkv, D, Na, F, near_k, near_v, near_dtype, far_k, far_v,
-                      far_v_scale, far_v_zero, sz_dtype, near_valid, spike_margin, stream);
+                      far_v_scale, far_v_zero, sz_dtype, near_valid, spike_margin, nullptr, 0, stream);
+}
+
+int64_t fkv_attn_blob_bytes(int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F, int32_t fmt) {
+    if (B <= 0 || Hkv <= 0 || Na < 0 || F < 0 || (D != 64 && D != 128) || fmt < 0 || fmt > 2)
+        return set_error("fkv_attn_blob_bytes: bad shape or format (head dim must be 64 or 128)");
+    return (int64_t)fkv::make_layout(B, Hkv, D, Na, F, fmt).total;
+}
+
+int fkv_attn_create_at(fkv_attn** out, int32_t fmt, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
+                       const void* near_k, const void* near_v, int32_t near_dtype, const uint8_t* far_k,
+                       const uint8_t* far_v, const void* far_v_scale, const void* far_v_zero, int32_t sz_dtype,
+                       const int32_t* near_valid, float spike_margin, void* blob, int64_t blob_bytes, void* stream) {
+    if (fmt != 0 && fmt != 2) return set_error("fkv_attn_create_at: format must be 0 or 2");
+    if (!blob) return set_error("fkv_attn_create_at: NULL blob");
+    return create_fp8("fkv_attn_create_at", fmt, out, B, Hkv, D, Na, F, near_k, near_v, near_dtype, far_k, far_v,
+                      far_v_scale, far_v_zero, sz_dtype, near_valid, spike_margin, blob, blob_bytes, stream);
 }
 
 }  // extern "C"
@@ -1189,19 +1210,15 @@ int ensure_workspace(const std::string& name, fkv_attn* h, int Hq, hipStream_t s
     const size_t wsf = fkv::workspace_floats(L, Hq);
     const int rows = fkv::workspace_rows(L, Hq);
     const size_t qn = (size_t)L.B * Hq * L.D;
-    int rc = check_hip(hipMalloc(&h->ws, wsf * sizeof(float)), "hipMalloc(ws)");
-    // arrival counters [rows], then the XCD watch words [1 + rows]
-    if (!rc) rc = check_hip(hipMalloc(&h->arrive, (2 * (size_t)rows + 1) * sizeof(int)), "hipMalloc(arrive)");
-    if (!rc) rc = check_hip(hipMalloc(&h->qbuf, qn * 2), "hipMalloc(qbuf)");
-    if (rc) {
-        if (h->ws) (void)hipFree(h->ws);
-        if (h->arrive) (void)hipFree(h->arrive);
-        if (h->qbuf) (void)hipFree(h->qbuf);
-        h->ws = nullptr;
-        h->arrive = nullptr;
-        h->qbuf = nullptr;
-        return rc;
-    }
+    // one allocation: split records, arrival counters [rows] and XCD watch
+    // words [1 + rows], the fp16 query copy
+    const size_t wsb = ((wsf * sizeof(float) + 255) & ~(size_t)255),
+                 arb = (((2 * (size_t)rows + 1) * sizeof(int) + 255) & ~(size_t)255);
+    uint8_t* mem = nullptr;
+    if (int rc = check_hip(hipMalloc(&mem, wsb + arb + qn * 2), "hipMalloc(workspace)")) return rc;
+    h->ws = (float*)mem;
+    h->arrive = (int*)(mem + wsb);
+    h->qbuf = (uint16_t*)(mem + wsb + arb);
     h->ws_floats = wsf;
     h->arrive_n = rows;
     h->ws_hq = Hq;
@@ -1699,11 +1716,17 @@ int fkv_attn_set_k_scale(fkv_attn* h, const float* k_scale, void* stream) {
 
 void fkv_attn_destroy(fkv_attn* h) {
     if (!h) return;
-    if (h->blob) (void)hipFree(h->blob);
+    // hipFree waits for the device; a caller's blob must be as free of work
+    // when this returns as one freed here
+    if (h->blob && !h->own_blob) {
+        int dev = -1;
+        if (hipGetDevice(&dev) == hipSuccess && dev != h->device) (void)hipSetDevice(h->device);
+        (void)hipDeviceSynchronize();
+        if (dev >= 0 && dev != h->device) (void)hipSetDevice(dev);
+    }
+    if (h->blob && h->own_blob) (void)hipFree(h->blob);
     free_spike_buffers(h);
     if (h->ws) (void)hipFree(h->ws);
-    if (h->qbuf) (void)hipFree(h->qbuf);
-    if (h->arrive) (void)hipFree(h->arrive);
     if (h->order_ev) (void)hipEventDestroy(h->order_ev);
     delete h;
 }

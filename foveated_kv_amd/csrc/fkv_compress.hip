@@ -663,6 +663,22 @@ __global__ __launch_bounds__(256) void compress_gather_kernel(CompressArgs a, co
     far_row<D, VG>(a, bh, (int64_t)bh * F + (r - npad), sub, kw, vw);
 }
 
+// The recency partition's index sets, one element per thread (an
+// importance partition of position-valued importance gives the same).
+__global__ void tier_index_kernel(fkv_tiers tb, int S, int64_t bh_n, int32_t* __restrict__ near_idx,
+                                  int32_t* __restrict__ far_idx) {
+    const int npad = tb.n_near_padded, F = tb.far_count, row = npad + F;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < bh_n * row; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t bh = i / row;
+        const int e = (int)(i % row), mid = e - tb.n_sinks, win = mid - tb.near_from_mid;
+        if (e >= npad) far_idx[bh * F + e - npad] = tb.mid_start + e - npad;
+        else near_idx[bh * npad + e] = mid < 0           ? e
+                                       : win < 0         ? tb.near_mid_start + mid
+                                       : win < tb.window ? S - tb.window + win
+                                                         : -1;
+    }
+}
+
 }  // namespace fkv
 
 namespace {
@@ -783,6 +799,23 @@ extern "C" int fkv_partition_importance(const fkv_tier_config* cfg, const float*
     hipLaunchKernelGGL(kern, dim3((unsigned)(B * H)), dim3(fkv::kPartThreads), 0, (hipStream_t)stream, importance, S,
                        tb, near_idx, far_idx);
     return fkv::check_hip(hipGetLastError(), "partition_kernel launch");
+}
+
+extern "C" int fkv_tier_index_rows(const fkv_tiers* tiers, int32_t B, int32_t H, int32_t S, int32_t* near_idx,
+                                   int32_t* far_idx, void* stream) {
+    using fkv::set_error;
+    if (!tiers) return set_error("fkv_tier_index_rows: tiers is NULL");
+    const fkv_tiers tb = *tiers;
+    if (B <= 0 || H <= 0 || S < 0 || tb.n_near_padded < 0 || tb.far_count < 0)
+        return set_error("fkv_tier_index_rows: bad shape");
+    if ((tb.n_near_padded > 0 && !near_idx) || (tb.far_count > 0 && !far_idx))
+        return set_error("fkv_tier_index_rows: NULL argument");
+    const int64_t n = (int64_t)B * H * ((int64_t)tb.n_near_padded + tb.far_count);
+    if (n == 0) return FKV_OK;
+    const int64_t blocks = fkv::cdiv(n, 256);
+    hipLaunchKernelGGL(fkv::tier_index_kernel, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0,
+                       (hipStream_t)stream, tb, S, (int64_t)B * H, near_idx, far_idx);
+    return fkv::check_hip(hipGetLastError(), "tier_index_kernel launch");
 }
 
 extern "C" int fkv_compress_layer_indexed(const fkv_tier_config* cfg, const void* keys, const void* values,

@@ -444,25 +444,27 @@ __global__ __launch_bounds__(256) void tq_compress_values_kernel(const void* __r
 using fkv::check_hip;
 using fkv::set_error;
 
-extern "C" {
+namespace {
 
-int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
+int turbo_create(const char* fn, fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
                      const void* near_k, const void* near_v, int32_t near_dtype, const uint8_t* k_idx,
                      const uint8_t* k_signs, const void* k_norm, const void* k_gamma, const uint8_t* v_packed,
                      const void* v_scale, int32_t nz_dtype, const int32_t* near_valid, const float* Pi,
-                     const float* S, const float* centroids, float spike_margin, void* stream) {
-    if (!out) return set_error("fkv_turbo_create: out is NULL");
+                     const float* S, const float* centroids, float spike_margin, void* blob, int64_t blob_bytes,
+                 void* stream) {
+    const std::string name(fn);
+    if (!out) return set_error(name + ": out is NULL");
     *out = nullptr;
     if (B <= 0 || Hkv <= 0 || Na < 0 || F < 0)
-        return set_error("fkv_turbo_create: bad shape B=" + std::to_string(B) + " Hkv=" + std::to_string(Hkv) +
+        return set_error(name + ": bad shape B=" + std::to_string(B) + " Hkv=" + std::to_string(Hkv) +
                          " Na=" + std::to_string(Na) + " F=" + std::to_string(F));
-    if (D != 64 && D != 128) return set_error("fkv_turbo_create: head dim must be 64 or 128, got " + std::to_string(D));
+    if (D != 64 && D != 128) return set_error(name + ": head dim must be 64 or 128, got " + std::to_string(D));
     if (near_dtype < FKV_F16 || near_dtype > FKV_F32 || nz_dtype < FKV_F16 || nz_dtype > FKV_F32)
-        return set_error("fkv_turbo_create: unsupported dtype");
+        return set_error(name + ": unsupported dtype");
     if ((Na > 0 && (!near_k || !near_v)) ||
         (F > 0 && (!k_idx || !k_signs || !k_norm || !k_gamma || !v_packed || !v_scale)) || !near_valid || !Pi ||
         !S || !centroids)
-        return set_error("fkv_turbo_create: NULL array");
+        return set_error(name + ": NULL array");
     hipStream_t st = (hipStream_t)stream;
     fkv_attn* h = new fkv_attn();
     fkv::PackSrc src{};
@@ -479,10 +481,10 @@ int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t 
     src.nz_dtype = nz_dtype;
     src.Pi = Pi;
     src.S = S;
-    int rc = fkv::attn_begin(h, B, Hkv, D, Na, F, 1, src, spike_margin, st);
+    int rc = fkv::attn_begin(fn, h, B, Hkv, D, Na, F, 1, src, spike_margin, blob, blob_bytes, st);
     float cb[4] = {0.f, 0.f, 0.f, 0.f};
     if (!rc) rc = check_hip(hipMemcpyAsync(cb, centroids, sizeof(cb), hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
-    if (!rc) rc = fkv::attn_finish("fkv_turbo_create", h, st);
+    if (!rc) rc = fkv::attn_finish(fn, h, st);
     if (!rc) {
         h->tq.rot = (const uint16_t*)(h->blob + fkv::tq_rot_section(h->L));
         // centroid(c) = alpha + beta*sh + gamma*sl + delta*sh*sl, sh/sl = +-1 bits of c
@@ -498,7 +500,7 @@ int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t 
         // the kernel expands the high-bit value plane to +-2 against
         // weights scaled by lvl (one weight for both planes)
         if (std::fabs(h->tq.lvh - 2.0 * h->tq.lvl) > 2e-6 * h->tq.lvh)
-            rc = fkv::set_error("fkv_turbo_create: value levels with lvh != 2 lvl (internal error)");
+            rc = fkv::set_error(name + ": value levels with lvh != 2 lvl (internal error)");
     }
     if (rc) {
         fkv_attn_destroy(h);
@@ -506,6 +508,32 @@ int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t 
     }
     *out = h;
     return FKV_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
+                     const void* near_k, const void* near_v, int32_t near_dtype, const uint8_t* k_idx,
+                     const uint8_t* k_signs, const void* k_norm, const void* k_gamma, const uint8_t* v_packed,
+                     const void* v_scale, int32_t nz_dtype, const int32_t* near_valid, const float* Pi,
+                     const float* S, const float* centroids, float spike_margin, void* stream) {
+    return turbo_create("fkv_turbo_create", out, B, Hkv, D, Na, F, near_k, near_v, near_dtype, k_idx, k_signs, k_norm,
+                        k_gamma, v_packed, v_scale, nz_dtype, near_valid, Pi, S, centroids, spike_margin, nullptr, 0,
+                        stream);
+}
+
+int fkv_turbo_create_at(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
+                        const void* near_k, const void* near_v, int32_t near_dtype, const uint8_t* k_idx,
+                        const uint8_t* k_signs, const void* k_norm, const void* k_gamma, const uint8_t* v_packed,
+                        const void* v_scale, int32_t nz_dtype, const int32_t* near_valid, const float* Pi,
+                        const float* S, const float* centroids, float spike_margin, void* blob, int64_t blob_bytes,
+                        void* stream) {
+    if (!blob) return set_error("fkv_turbo_create_at: NULL blob");
+    return turbo_create("fkv_turbo_create_at", out, B, Hkv, D, Na, F, near_k, near_v, near_dtype, k_idx, k_signs,
+                        k_norm, k_gamma, v_packed, v_scale, nz_dtype, near_valid, Pi, S, centroids, spike_margin, blob,
+                        blob_bytes, stream);
 }
 
 int fkv_turbo_compress_keys(const void* keys, int32_t dtype, int64_t n_tokens, int32_t D, const float* Pi,

@@ -168,6 +168,20 @@ class CompressHandle:
         return [self.compress_layer(k, v, with_archive) for k, v in zip(all_keys, all_values)]
 
 
+def tier_index_rows(tb, S, B, H, device):
+    """fkv_tier_index_rows: near_idx (B,H,Npad) and far_idx (B,H,F) int32 of
+    the recency partition with tier boundaries ``tb``, on the GPU ``device``."""
+    c = _lib.TiersC(tb["n_sinks"], tb["window"], tb["near_from_mid"], tb["far_count"], tb["R_actual"],
+                    tb["N_near_padded"], tb["mid_start"], tb["mid_end"], tb["near_mid_start"],
+                    tb["N_near_padded"] - tb["R_actual"])
+    near_idx = torch.empty((B, H, tb["N_near_padded"]), dtype=torch.int32, device=device)
+    far_idx = torch.empty((B, H, tb["far_count"]), dtype=torch.int32, device=device)
+    with torch.cuda.device(device):
+        check(_lib.load().fkv_tier_index_rows(ctypes.byref(c), B, H, S, ptr(near_idx), ptr(far_idx),
+                                              _lib.stream_ptr(device)), "fkv_tier_index_rows")
+    return near_idx, far_idx
+
+
 def partition_importance(cfg, importance, B, H, S):
     """fkv_partition_importance: importance (fp32, broadcastable to (B,H,S),
     on the device) -> near_idx (B,H,Npad) int32 (sinks, chosen middle,
@@ -251,11 +265,11 @@ class FoveatedHandle:
         lib = _lib.load()
         h = ctypes.c_void_p()
         with torch.cuda.device(self.device):
-            create = lib.fkv_attn_create_g32 if grouped else lib.fkv_attn_create
-            check(create(ctypes.byref(h), B, H, D, Na, F, ptr(nk), ptr(nv), dtype_code(nk.dtype),
-                         ptr(fk), ptr(fv), ptr(fvs), ptr(fvz), dtype_code(fvs.dtype), ptr(valid),
-                         self.spike_margin, _lib.stream_ptr(self.device)),
-                  "fkv_attn_create_g32" if grouped else "fkv_attn_create")
+            blob = self._new_blob(lib, 2 if grouped else 0)
+            check(lib.fkv_attn_create_at(ctypes.byref(h), 2 if grouped else 0, B, H, D, Na, F, ptr(nk), ptr(nv),
+                                         dtype_code(nk.dtype), ptr(fk), ptr(fv), ptr(fvs), ptr(fvz),
+                                         dtype_code(fvs.dtype), ptr(valid), self.spike_margin, ptr(blob),
+                                         blob.numel(), _lib.stream_ptr(self.device)), "fkv_attn_create_at")
         self._h = h
         self._lib = lib
         self.spike_k = 1
@@ -267,6 +281,18 @@ class FoveatedHandle:
                 check(lib.fkv_attn_set_k_scale(h, ptr(ks), _lib.stream_ptr(self.device)), "fkv_attn_set_k_scale")
         self.set_spike_k(spike_k)
 
+    def _new_blob(self, lib, fmt):
+        """The handle's device blob, from torch's caching allocator (a
+        hipMalloc and hipFree of 84 MB took about 400 us of every handle).
+        Destroying the handle waits for the device before the tensor goes
+        back to the allocator, so work on any stream -- calls, promotions,
+        graph replays -- is done with it by then."""
+        n = lib.fkv_attn_blob_bytes(self.B, self.H_kv, self.D, self.N_near, self.N_far, fmt)
+        if n < 0:
+            check(int(n), "fkv_attn_blob_bytes")
+        self._blob = torch.empty(n, dtype=torch.uint8, device=self.device)
+        return self._blob
+
     def set_spike_k(self, spike_k):
         """Spiking far tokens per query head reported by later calls."""
         check(self._lib.fkv_attn_set_spike_k(self._h, int(spike_k)), "fkv_attn_set_spike_k")
@@ -275,8 +301,9 @@ class FoveatedHandle:
     def __del__(self):
         h = getattr(self, "_h", None)
         if h is not None and h.value:
-            self._lib.fkv_attn_destroy(h)
+            self._lib.fkv_attn_destroy(h)  # waits for the device: the blob is idle
             self._h = None
+        self._blob = None
 
     def __call__(self, query, decode_k=None, decode_v=None, n_decode=None, out=None):
         """-> [out (B,Hq,1,D) fp16, spike_flags (B,Hq) int32, spike_tokens (B,Hq) int32]

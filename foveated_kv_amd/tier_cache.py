@@ -201,13 +201,18 @@ class FoveatedLayer:
     _turbo_constants: Optional[object] = None
     far_k_scale: Optional[torch.Tensor] = None  # (B,H) fp32: per-head-scaled fp8 keys
     spike_k: int = 1  # spiking far tokens per query head the fused kernel reports
+    # position of the next token (None: one past the largest index, which
+    # reads both index tensors back)
+    next_position: Optional[int] = field(default=None, repr=False)
 
     def __post_init__(self):
-        max_pos = -1
-        for t in (self.near_idx, self.far_idx):
-            if t.numel() > 0:
-                max_pos = max(max_pos, int(t.max().item()))
-        self._next_pos = max_pos + 1
+        if self.next_position is None:
+            max_pos = -1
+            for t in (self.near_idx, self.far_idx):
+                if t.numel() > 0:
+                    max_pos = max(max_pos, int(t.max().item()))
+            self.next_position = max_pos + 1
+        self._next_pos = self.next_position
         self._decode = _DecodeBuffer()
         if self.near_valid is None:
             self.near_valid = torch.full((self.near_k.shape[1],), self.near_k.shape[2],
@@ -292,7 +297,7 @@ class FoveatedLayer:
         if self.compress_method == "turbo":
             from .turbo import TurboFoveatedHandle
 
-            tc = self._turbo_constants
+            tc = self._turbo_constants.on(self.near_k.device)
             handle = TurboFoveatedHandle(
                 self.near_k, self.near_v, self.turbo_far_k_indices, self.turbo_far_k_signs,
                 self.turbo_far_k_norm, self.turbo_far_k_gamma, self.turbo_far_v_packed,
@@ -382,6 +387,8 @@ class FoveatedLayer:
 def tier_index_tensors(tb: dict, S: int, B: int, H: int, device):
     """near_idx (B,H,Npad) with -1 headroom and far_idx (B,H,F), int32
     (mlx_foveated.py:719-752)."""
+    if torch.device(device).type == "cuda":
+        return ext.tier_index_rows(tb, S, B, H, torch.device(device))
     parts = []
     if tb["n_sinks"] > 0:
         parts.append(torch.arange(tb["n_sinks"], device=device))
@@ -471,7 +478,7 @@ class FoveatedKVCache:
                              far_v=cl.far_v, far_v_scale=cl.far_v_scale, far_v_zero=cl.far_v_zero,
                              far_idx=far_idx, archive_k=cl.archive_k, archive_v=cl.archive_v,
                              archive_idx=far_idx, near_valid=cl.near_valid, far_k_scale=cl.far_k_scale,
-                             spike_k=int(self.cfg.spike_k))
+                             spike_k=int(self.cfg.spike_k), next_position=S)
 
     def attend(self, layer_idx: int, query):
         layer = self.layers[layer_idx]

@@ -282,10 +282,11 @@ class TurboFoveatedHandle(ext.FoveatedHandle):
         lib = _lib.load()
         h = ctypes.c_void_p()
         with torch.cuda.device(self.device):
-            check(lib.fkv_turbo_create(ctypes.byref(h), B, H, D, Na, F, ptr(nk), ptr(nv), dtype_code(nk.dtype),
-                                       ptr(ki), ptr(ks), ptr(kn), ptr(kg), ptr(vp), ptr(vs), dtype_code(nz),
-                                       ptr(valid), ptr(pi), ptr(sm), ptr(cb), self.spike_margin,
-                                       _lib.stream_ptr(self.device)), "fkv_turbo_create")
+            blob = self._new_blob(lib, 1)
+            check(lib.fkv_turbo_create_at(ctypes.byref(h), B, H, D, Na, F, ptr(nk), ptr(nv), dtype_code(nk.dtype),
+                                          ptr(ki), ptr(ks), ptr(kn), ptr(kg), ptr(vp), ptr(vs), dtype_code(nz),
+                                          ptr(valid), ptr(pi), ptr(sm), ptr(cb), self.spike_margin, ptr(blob),
+                                          blob.numel(), _lib.stream_ptr(self.device)), "fkv_turbo_create_at")
         self._h = h
         self._lib = lib
 
@@ -314,4 +315,4 @@ def build_turbo_layer(cfg, keys, values, importance=None):
                          far_idx=far_idx, archive_k=cl.archive_k, archive_v=cl.archive_v, archive_idx=far_idx,
                          near_valid=cl.near_valid, compress_method="turbo", turbo_far_k_indices=ki,
                          turbo_far_k_signs=ks, turbo_far_k_norm=kn, turbo_far_k_gamma=kg, turbo_far_v_packed=vp,
-                         turbo_far_v_scale=vs, _turbo_constants=tc)
+                         turbo_far_v_scale=vs, _turbo_constants=tc, next_position=S)

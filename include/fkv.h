@@ -108,6 +108,12 @@ int fkv_compress_layer(const fkv_tier_config* cfg, const void* keys, const void*
 int fkv_partition_importance(const fkv_tier_config* cfg, const float* importance, int32_t B, int32_t H,
                              int32_t S, int32_t* near_idx, int32_t* far_idx, void* stream);
 
+/* The recency partition's index sets (mlx_foveated.py:719-752) for tiers as
+ * fkv_tier_boundaries gives them: near_idx (B,H,Npad) int32 (sinks, near
+ * middle, window, -1 headroom) and far_idx (B,H,F) int32.  Asynchronous. */
+int fkv_tier_index_rows(const fkv_tiers* tiers, int32_t B, int32_t H, int32_t S, int32_t* near_idx,
+                        int32_t* far_idx, void* stream);
+
 /* fkv_compress_layer from explicit index sets (as fkv_partition_importance
  * writes them): near slot s < R_actual is the row near_idx[b,h,s], far row
  * f is far_idx[b,h,f]; the archive holds the far rows in far_idx order.
@@ -189,6 +195,25 @@ int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t 
                      const uint8_t* k_signs, const void* k_norm, const void* k_gamma, const uint8_t* v_packed,
                      const void* v_scale, int32_t nz_dtype, const int32_t* near_valid, const float* Pi,
                      const float* S, const float* centroids, float spike_margin, void* stream);
+
+/* Handle construction into a caller's blob: fkv_attn_create (fmt 0),
+ * fkv_attn_create_g32 (fmt 2) and fkv_turbo_create with the blob's device
+ * memory given instead of allocated -- 256-byte aligned, at least
+ * fkv_attn_blob_bytes of the same shape and format, and the caller's until
+ * fkv_attn_destroy, which returns only when no work on the device uses it.
+ * For programs that keep device memory in a caching allocator: allocating and
+ * freeing an 84 MB blob took about 400 us.  Synchronous, as those. */
+int64_t fkv_attn_blob_bytes(int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F, int32_t fmt);
+int fkv_attn_create_at(fkv_attn** out, int32_t fmt, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
+                       const void* near_k, const void* near_v, int32_t near_dtype, const uint8_t* far_k,
+                       const uint8_t* far_v, const void* far_v_scale, const void* far_v_zero, int32_t sz_dtype,
+                       const int32_t* near_valid, float spike_margin, void* blob, int64_t blob_bytes, void* stream);
+int fkv_turbo_create_at(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F,
+                        const void* near_k, const void* near_v, int32_t near_dtype, const uint8_t* k_idx,
+                        const uint8_t* k_signs, const void* k_norm, const void* k_gamma, const uint8_t* v_packed,
+                        const void* v_scale, int32_t nz_dtype, const int32_t* near_valid, const float* Pi,
+                        const float* S, const float* centroids, float spike_margin, void* blob, int64_t blob_bytes,
+                        void* stream);
 
 /* TurboQuant compression on the GPU (src/foveated_kv/turbo_quantize.py:
  * 25-91): keys (n_tokens, D) in dtype -> out_idx (n_tokens, D/4) u8,

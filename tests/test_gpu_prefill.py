@@ -383,3 +383,93 @@ def test_far_nan_codes_refused(fkv):
                 ext.FoveatedHandle(cl.near_k, cl.near_v, cl.far_k, cl.far_v, cl.far_v_scale, cl.far_v_zero, cl.near_valid)
             flat[at] = old
     ext.FoveatedHandle(cl.near_k, cl.near_v, cl.far_k, cl.far_v, cl.far_v_scale, cl.far_v_zero, cl.near_valid)
+
+
+def test_tier_index_rows_match_host(fkv):
+    """The index kernel against the torch construction, over tier configs and
+    lengths down to empty tiers."""
+    from foveated_kv_amd.tier_cache import TierConfig, tier_index_tensors
+
+    for kw in ({}, dict(n_sinks=0, window_size=0), dict(near_pct=0.5), dict(near_pct=1.0),
+               dict(promo_headroom_pct=0.0, promo_headroom_min=0)):
+        for S in (0, 1, 3, 36, 37, 500, 4097):
+            tb = TierConfig(**kw).tier_boundaries(S)
+            flush(f"tier index rows {kw} S={S}")
+            for a, b in zip(tier_index_tensors(tb, S, 2, 3, "cuda"), tier_index_tensors(tb, S, 2, 3, "cpu")):
+                assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a.cpu(), b)
+
+
+def test_layer_next_position(fkv):
+    """The position after the prompt, as counted from the index tensors."""
+    from foveated_kv_amd import FoveatedKVCache, FoveatedLayer, TierConfig
+
+    for kw in ({}, dict(compress_method="turbo"), dict(window_size=0, n_sinks=0)):
+        for S in (40, 333):
+            k = torch.randn((1, 2, S, 64), device="cuda").half()
+            cache = FoveatedKVCache(TierConfig(**kw))
+            cache.update(k, k, 0)
+            cache.compress(importance=torch.rand(S, device="cuda") if S == 333 else None)
+            lay = cache.layers[0]
+            want = max(int(lay.near_idx.max()), int(lay.far_idx.max()) if lay.far_idx.numel() else -1) + 1
+            assert lay._next_pos == want == S
+
+
+def test_blob_memory_outlives_calls_in_flight(fkv):
+    """A handle dropped right after calls on another stream and a graph replay:
+    its blob's memory is not handed out again while they run."""
+    from foveated_kv_amd import FoveatedKVCache, TierConfig
+
+    k, v = (torch.randn((2, 4, 6000, 128), device="cuda").half() for _ in range(2))
+    q = torch.randn((2, 16, 1, 128), device="cuda").half()
+    cache = FoveatedKVCache(TierConfig())
+    cache.update(k, v, 0)
+    cache.compress()
+    lay = cache.layers[0]
+    want = [t.clone() for t in lay.attend_fused_with_spikes(q)]
+    side = torch.cuda.Stream()
+    for _ in range(5):
+        lay._kcache = None
+        lay._ensure_kcache()
+        h = lay._kcache["cpp_handle"]
+        outs = [torch.empty_like(t) for t in want]
+        h(q, out=outs)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            h(q, out=outs)
+        nbytes = h._blob.numel()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(20):
+                got = h(q)
+            g.replay()
+        lay._kcache = None
+        del h
+        junk = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")  # likely the same memory
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want)) and all(torch.equal(a, b) for a, b in zip(outs, want))
+        del junk, g
+
+
+def test_create_at_checks_the_blob(fkv):
+    """A blob that is too small or not aligned is refused before any use."""
+    import ctypes
+
+    from foveated_kv_amd import _lib, ext
+
+    k = torch.randn((1, 2, 300, 64), device="cuda").half()
+    cl = ext.CompressHandle(_cfg()).compress_layer(k, k)
+    lib = _lib.load()
+    Na, F = cl.near_k.shape[2], cl.far_k.shape[2]
+    n = lib.fkv_attn_blob_bytes(1, 2, 64, Na, F, 0)
+    mem = torch.empty(n + 512, dtype=torch.uint8, device="cuda")
+    for off, size, ok in ((0, n, True), (0, n - 1, False), (16, n, False), (256, n, True)):
+        h = ctypes.c_void_p()
+        rc = lib.fkv_attn_create_at(
+            ctypes.byref(h), 0, 1, 2, 64, Na, F, _lib.ptr(cl.near_k), _lib.ptr(cl.near_v), 0, _lib.ptr(cl.far_k),
+            _lib.ptr(cl.far_v), _lib.ptr(cl.far_v_scale), _lib.ptr(cl.far_v_zero), 0, _lib.ptr(cl.near_valid), 10.0,
+            ctypes.c_void_p(mem.data_ptr() + off), size, _lib.stream_ptr(torch.device("cuda")))
+        assert (rc == 0) == ok
+        if ok:
+            lib.fkv_attn_destroy(h)
+    assert lib.fkv_attn_blob_bytes(1, 2, 96, Na, F, 0) < 0 and lib.fkv_attn_blob_bytes(1, 2, 64, Na, F, 3) < 0
