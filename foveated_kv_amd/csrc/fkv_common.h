@@ -70,18 +70,39 @@ __device__ inline float wave_min(float v) {
     return v;
 }
 
-// 8 consecutive elements as packed fp16 bits (astype(float16) semantics: RNE)
+// 16-byte accesses that leave the caches to others (non-temporal).
+typedef uint32_t fkv_u2 __attribute__((ext_vector_type(2)));
+typedef uint32_t fkv_u4 __attribute__((ext_vector_type(4)));
+__device__ inline uint4 load16_nt(const void* p) {
+    const fkv_u4 v = __builtin_nontemporal_load((const fkv_u4*)p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <bool NT>
+__device__ inline void store16(void* p, uint4 v) {
+    const fkv_u4 x = {v.x, v.y, v.z, v.w};
+    if (NT) __builtin_nontemporal_store(x, (fkv_u4*)p);
+    else *(fkv_u4*)p = x;
+}
+template <bool NT>
+__device__ inline void store8(void* p, uint32_t lo, uint32_t hi) {
+    const fkv_u2 x = {lo, hi};
+    if (NT) __builtin_nontemporal_store(x, (fkv_u2*)p);
+    else *(fkv_u2*)p = x;
+}
+
+// 8 consecutive elements, read once (non-temporal), as packed fp16 bits
+// (astype(float16) semantics: RNE)
 __device__ inline uint4 load8(const void* base, int dtype, int64_t elem) {
-    if (dtype == FKV_F16) return *(const uint4*)((const uint16_t*)base + elem);
+    if (dtype == FKV_F16) return load16_nt((const uint16_t*)base + elem);
     auto pk = [](float a, float b) { return (uint32_t)f2h(a) | ((uint32_t)f2h(b) << 16); };
     if (dtype == FKV_BF16) {
-        const uint4 w = *(const uint4*)((const uint16_t*)base + elem);
+        const uint4 w = load16_nt((const uint16_t*)base + elem);
         auto two = [&](uint32_t u) { return pk(__uint_as_float(u << 16), __uint_as_float(u & 0xFFFF0000u)); };
         return make_uint4(two(w.x), two(w.y), two(w.z), two(w.w));
     }
-    const float4* p = (const float4*)((const float*)base + elem);
-    const float4 a = p[0], b = p[1];
-    return make_uint4(pk(a.x, a.y), pk(a.z, a.w), pk(b.x, b.y), pk(b.z, b.w));
+    const uint4 a = load16_nt((const float*)base + elem), b = load16_nt((const float*)base + elem + 4);
+    auto two = [&](uint32_t x, uint32_t y) { return pk(__uint_as_float(x), __uint_as_float(y)); };
+    return make_uint4(two(a.x, a.y), two(a.z, a.w), two(b.x, b.y), two(b.z, b.w));
 }
 
 // a / b rounded to nearest even, from y = 1.0f / b (so rounded itself):

@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <type_traits>
 
 #include "fkv_common.h"
 #include "../../include/fkv.h"
@@ -113,18 +114,18 @@ __device__ inline void row_minmax(float& mn, float& mx) {
 // permutes): the 64K x 8 head layer from bf16 with key scales and group-32
 // values took 191 us without (3.4 TB/s), 124 us now (5.3 TB/s); the 8 x 8 x
 // 16K fp16 layer was at the memory's rate before (219 us) and still is (218).
-template <int D, int VG>
+template <int D, int VG, bool NT>
 __device__ inline void far_row(const CompressArgs& a, int bh, int64_t fr, int sub, uint4 kw, uint4 vw) {
     constexpr int LPR = D / 8;
-    if (a.arc_k) *(uint4*)(a.arc_k + fr * D + sub * 8) = kw;
-    if (a.arc_v) *(uint4*)(a.arc_v + fr * D + sub * 8) = vw;
+    if (a.arc_k) store16<true>(a.arc_k + fr * D + sub * 8, kw);
+    if (a.arc_v) store16<true>(a.arc_v + fr * D + sub * 8, vw);
     // far K: E4M3 codes
     if (a.kscale) {
         const float scale = a.kscale[bh], rscale = 1.0f / scale;
         kw = make_uint4(scaled_keys(kw.x, scale, rscale), scaled_keys(kw.y, scale, rscale),
                         scaled_keys(kw.z, scale, rscale), scaled_keys(kw.w, scale, rscale));
     }
-    *(uint2*)(a.far_k + fr * D + sub * 8) = make_uint2(encode_e4m3x4(kw.x, kw.y), encode_e4m3x4(kw.z, kw.w));
+    store8<NT>(a.far_k + fr * D + sub * 8, encode_e4m3x4(kw.x, kw.y), encode_e4m3x4(kw.z, kw.w));
     // far V: INT4 per token (VG = 0) or per 32-dim group
     constexpr int RL = VG ? VG / 8 : LPR;  // lanes of one quantisation row
     const uint32_t vs[4] = {vw.x, vw.y, vw.z, vw.w};
@@ -147,7 +148,9 @@ __device__ inline void far_row(const CompressArgs& a, int bh, int64_t fr, int su
         c += q - (float)c >= 0.5f ? 1u : 0u;
         packed |= min(c, 15u) << (4 * i);
     }
-    *(uint32_t*)(a.far_v + fr * (D / 2) + sub * 4) = packed;
+    uint32_t* const pv = (uint32_t*)(a.far_v + fr * (D / 2) + sub * 4);
+    if (NT) __builtin_nontemporal_store(packed, pv);
+    else *pv = packed;
     if (sub % RL == 0) {
         const int64_t si = VG ? fr * (D / VG) + sub / RL : fr;
         a.fvs[si] = f2h(scale);
@@ -157,7 +160,7 @@ __device__ inline void far_row(const CompressArgs& a, int bh, int64_t fr, int su
 
 // VG = 0: one INT4 scale / zero per token (the reference); VG = 32: one per
 // 32-dim group (4 lanes), the same quantiser applied to every group.
-template <int D, int VG>
+template <int D, int VG, bool NT>
 __global__ __launch_bounds__(256) void compress_kernel(CompressArgs a) {
     constexpr int LPR = D / 8;       // lanes per row
     constexpr int RPB = 256 / LPR;   // rows per block
@@ -172,8 +175,8 @@ __global__ __launch_bounds__(256) void compress_kernel(CompressArgs a) {
     const uint4 zero4 = make_uint4(0, 0, 0, 0);
     if (r >= a.S) {  // headroom slot: zeros
         const int64_t o = ((int64_t)bh * npad + tb.r_actual + (r - a.S)) * D + sub * 8;
-        *(uint4*)(a.near_k + o) = zero4;
-        *(uint4*)(a.near_v + o) = zero4;
+        store16<NT>(a.near_k + o, zero4);
+        store16<NT>(a.near_v + o, zero4);
         return;
     }
     const int t = r;
@@ -187,12 +190,12 @@ __global__ __launch_bounds__(256) void compress_kernel(CompressArgs a) {
     const uint4 kw = load8(a.k, a.dtype, src), vw = load8(a.v, a.dtype, src);
     if (slot >= 0) {
         const int64_t o = ((int64_t)bh * npad + slot) * D + sub * 8;
-        *(uint4*)(a.near_k + o) = kw;
-        *(uint4*)(a.near_v + o) = vw;
+        store16<NT>(a.near_k + o, kw);
+        store16<NT>(a.near_v + o, vw);
         return;
     }
     if (f < 0) return;  // unreachable: every position is near or far
-    far_row<D, VG>(a, bh, (int64_t)bh * F + f, sub, kw, vw);
+    far_row<D, VG, NT>(a, bh, (int64_t)bh * F + f, sub, kw, vw);
 }
 
 
@@ -631,7 +634,7 @@ __global__ __launch_bounds__(kPartThreads) void partition_kernel(const float* __
 // (source near_idx, zeros for headroom / -1 / out-of-range indices), row
 // Npad + f is far row f (source far_idx; an out-of-range index encodes a
 // zero row).
-template <int D, int VG>
+template <int D, int VG, bool NT>
 __global__ __launch_bounds__(256) void compress_gather_kernel(CompressArgs a, const int32_t* __restrict__ near_idx,
                                                               const int32_t* __restrict__ far_idx) {
     constexpr int LPR = D / 8;
@@ -656,11 +659,11 @@ __global__ __launch_bounds__(256) void compress_gather_kernel(CompressArgs a, co
     }
     if (near) {
         const int64_t o = ((int64_t)bh * npad + r) * D + sub * 8;
-        *(uint4*)(a.near_k + o) = kw;
-        *(uint4*)(a.near_v + o) = vw;
+        store16<NT>(a.near_k + o, kw);
+        store16<NT>(a.near_v + o, vw);
         return;
     }
-    far_row<D, VG>(a, bh, (int64_t)bh * F + (r - npad), sub, kw, vw);
+    far_row<D, VG, NT>(a, bh, (int64_t)bh * F + (r - npad), sub, kw, vw);
 }
 
 // The recency partition's index sets, one element per thread (an
@@ -748,20 +751,33 @@ int compress_launch(const char* fn, const fkv_tier_config* cfg, fkv::CompressArg
         a.kscale = far_k_scale;
     }
     const int rpb = 256 / (D / 8);
+    // K and V are read once and the archive is written for later: both pass
+    // the caches by, which leaves the tiers in the 256 MB last-level cache for
+    // the blob packing that follows (4 x 8 heads x 8,192 tokens: compress 62 ->
+    // 58 us, packing 32 -> 25). Tiers that would not stay there pass it by as
+    // well (8 x 8 x 16K, 262 MB: 215 us with plain stores, 211 with the first
+    // rule alone, 204 with both; 132 MB of tiers 121 with the first, 125 with
+    // both): from three quarters of the cache on.
+    const size_t tiers = (size_t)B * H * ((size_t)a.tb.n_near_padded * D * 4 + (size_t)a.tb.far_count * (D + D / 2));
+    const bool nt = tiers > ((size_t)192 << 20);
     if (!near_idx) {
         const int rows = a.S + a.tb.headroom;
         dim3 grid((unsigned)fkv::cdiv(rows > 0 ? rows : 1, rpb), (unsigned)(B * H));
-        void (*kern)(fkv::CompressArgs) = D == 128 ? (g32 ? fkv::compress_kernel<128, 32> : fkv::compress_kernel<128, 0>)
-                                                   : (g32 ? fkv::compress_kernel<64, 32> : fkv::compress_kernel<64, 0>);
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a);
+        auto pick = [&](auto NT) {
+            return D == 128 ? (g32 ? fkv::compress_kernel<128, 32, NT.value> : fkv::compress_kernel<128, 0, NT.value>)
+                            : (g32 ? fkv::compress_kernel<64, 32, NT.value> : fkv::compress_kernel<64, 0, NT.value>);
+        };
+        hipLaunchKernelGGL(nt ? pick(std::true_type{}) : pick(std::false_type{}), grid, dim3(256), 0, st, a);
         return fkv::check_hip(hipGetLastError(), "compress_kernel launch");
     }
     const int rows = a.tb.n_near_padded + a.tb.far_count;
     dim3 grid((unsigned)fkv::cdiv(rows > 0 ? rows : 1, rpb), (unsigned)(B * H));
-    void (*kern)(fkv::CompressArgs, const int32_t*, const int32_t*) =
-        D == 128 ? (g32 ? fkv::compress_gather_kernel<128, 32> : fkv::compress_gather_kernel<128, 0>)
-                 : (g32 ? fkv::compress_gather_kernel<64, 32> : fkv::compress_gather_kernel<64, 0>);
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a, near_idx, far_idx);
+    auto pick = [&](auto NT) {
+        return D == 128 ? (g32 ? fkv::compress_gather_kernel<128, 32, NT.value> : fkv::compress_gather_kernel<128, 0, NT.value>)
+                        : (g32 ? fkv::compress_gather_kernel<64, 32, NT.value> : fkv::compress_gather_kernel<64, 0, NT.value>);
+    };
+    hipLaunchKernelGGL(nt ? pick(std::true_type{}) : pick(std::false_type{}), grid, dim3(256), 0, st, a, near_idx,
+                       far_idx);
     return fkv::check_hip(hipGetLastError(), "compress_gather_kernel launch");
 }
 

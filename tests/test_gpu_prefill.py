@@ -473,3 +473,24 @@ def test_create_at_checks_the_blob(fkv):
         if ok:
             lib.fkv_attn_destroy(h)
     assert lib.fkv_attn_blob_bytes(1, 2, 96, Na, F, 0) < 0 and lib.fkv_attn_blob_bytes(1, 2, 64, Na, F, 3) < 0
+
+
+@pytest.mark.parametrize("importance", [False, True])
+def test_compress_past_the_cache(fkv, importance):
+    """Large tiers (stores that pass the caches by) hold the bytes that
+    the same heads compressed a few at a time do."""
+    from foveated_kv_amd import ext
+
+    B, H, S, D = 8, 8, 17000, 128
+    g = torch.Generator(device="cuda").manual_seed(3)
+    k, v = (torch.randn((B, H, S, D), generator=g, device="cuda", dtype=torch.float16) for _ in range(2))
+    imp = torch.rand((B, H, S), generator=g, device="cuda") if importance else None
+    h = ext.CompressHandle(_cfg())
+    flush(f"compress past the cache importance={importance}")
+    big = h.compress_layer(k, v, importance=imp)
+    nbytes = sum(getattr(big, n).numel() * getattr(big, n).element_size() for n in ("near_k", "near_v", "far_k", "far_v"))
+    assert nbytes > 192 << 20
+    for b in range(0, B, 4):
+        part = h.compress_layer(k[b:b + 4], v[b:b + 4], importance=None if imp is None else imp[b:b + 4])
+        for n in ("near_k", "near_v", "far_k", "far_v", "far_v_scale", "far_v_zero", "archive_k", "archive_v"):
+            assert torch.equal(getattr(big, n)[b:b + 4], getattr(part, n)), n
