@@ -87,6 +87,8 @@ SIGNATURES = {
                                                   P, P, P, P, P, P, P, P, P, P, P, P]),
     "fkv_compress_layer_ex": (ctypes.c_int, [ctypes.POINTER(TierConfigC), P, P, I32, I32, I32, I32, I32,
                                              P, P, P, P, P, P, P, P, P, P, P, P, P]),
+    "fkv_archive_layer": (ctypes.c_int, [ctypes.POINTER(TierConfigC), P, P, I32, I32, I32, I32, I32,
+                                         P, P, P, P, P, P, P, P]),
     "fkv_attn_create": (ctypes.c_int, [ctypes.POINTER(P), I32, I32, I32, I32, I32, P, P, I32, P, P, P, P,
                                        I32, P, F32, P]),
     "fkv_attn_create_g32": (ctypes.c_int, [ctypes.POINTER(P), I32, I32, I32, I32, I32, P, P, I32, P, P, P, P,

@@ -117,6 +117,11 @@ __device__ inline void row_minmax(float& mn, float& mx) {
 template <int D, int VG, bool NT>
 __device__ inline void far_row(const CompressArgs& a, int bh, int64_t fr, int sub, uint4 kw, uint4 vw) {
     constexpr int LPR = D / 8;
+    if (!a.far_k) {  // near tier and archive only (the archive is read next)
+        store16<false>(a.arc_k + fr * D + sub * 8, kw);
+        store16<false>(a.arc_v + fr * D + sub * 8, vw);
+        return;
+    }
     if (a.arc_k) store16<true>(a.arc_k + fr * D + sub * 8, kw);
     if (a.arc_v) store16<true>(a.arc_v + fr * D + sub * 8, vw);
     // far K: E4M3 codes
@@ -690,7 +695,7 @@ namespace {
 int compress_setup(const char* fn, const fkv_tier_config* cfg, const void* keys, const void* values,
                    int32_t in_dtype, int32_t B, int32_t H, int32_t S, int32_t D, void* near_k, void* near_v,
                    uint8_t* far_k, uint8_t* far_v, void* far_v_scale, void* far_v_zero, int32_t* near_valid,
-                   void* archive_k, void* archive_v, fkv::CompressArgs& a) {
+                   void* archive_k, void* archive_v, fkv::CompressArgs& a, bool archive_only = false) {
     using fkv::set_error;
     const std::string name(fn);
     if (!cfg) return set_error(name + ": cfg is NULL");
@@ -704,7 +709,7 @@ int compress_setup(const char* fn, const fkv_tier_config* cfg, const void* keys,
     fkv_tiers tb;
     if (int rc = fkv_tier_boundaries(cfg, S, &tb)) return rc;
     if ((S > 0 && (!keys || !values)) || !near_k || !near_v || !near_valid ||
-        (tb.far_count > 0 && (!far_k || !far_v || !far_v_scale || !far_v_zero)))
+        (tb.far_count > 0 && (archive_only ? !archive_k || !archive_v : !far_k || !far_v || !far_v_scale || !far_v_zero)))
         return set_error(name + ": NULL output/input");
     a.k = keys;
     a.v = values;
@@ -864,5 +869,20 @@ extern "C" int fkv_compress_layer_ex(const fkv_tier_config* cfg, const void* key
     if (!near_idx != !far_idx && a.tb.far_count > 0)
         return fkv::set_error("fkv_compress_layer_ex: near_idx and far_idx are both given or both NULL");
     return compress_launch("fkv_compress_layer_ex", cfg, a, D, near_idx, near_idx ? far_idx : nullptr, far_k_scale,
+                           (hipStream_t)stream);
+}
+
+extern "C" int fkv_archive_layer(const fkv_tier_config* cfg, const void* keys, const void* values, int32_t in_dtype,
+                                 int32_t B, int32_t H, int32_t S, int32_t D, const int32_t* near_idx,
+                                 const int32_t* far_idx, void* near_k, void* near_v, int32_t* near_valid,
+                                 void* archive_k, void* archive_v, void* stream) {
+    fkv::CompressArgs a;
+    if (int rc = compress_setup("fkv_archive_layer", cfg, keys, values, in_dtype, B, H, S, D, near_k, near_v, nullptr,
+                                nullptr, nullptr, nullptr, near_valid, archive_k, archive_v, a, true))
+        return rc;
+    if (!near_idx != !far_idx && a.tb.far_count > 0)
+        return fkv::set_error("fkv_archive_layer: near_idx and far_idx are both given or both NULL");
+    if (cfg->k_scale) return fkv::set_error("fkv_archive_layer: there are no far keys to scale");
+    return compress_launch("fkv_archive_layer", cfg, a, D, near_idx, near_idx ? far_idx : nullptr, nullptr,
                            (hipStream_t)stream);
 }

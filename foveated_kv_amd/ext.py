@@ -125,6 +125,14 @@ class CompressHandle:
         (batch, head), ties to the later token (importance = position gives
         the reference's recency partition); the index sets are returned as
         ``near_idx`` / ``far_idx``."""
+        return self._compress(keys, values, with_archive, importance, far=True)
+
+    def archive_layer(self, keys, values, importance=None):
+        """The near tier and the fp16 archive alone (the far fields stay
+        None): what a TurboQuant layer takes."""
+        return self._compress(keys, values, True, importance, far=False)
+
+    def _compress(self, keys, values, with_archive, importance, far):
         _require_device(keys, values, importance)
         if keys.shape != values.shape or keys.dim() != 4:
             raise ValueError(f"keys/values must be (B,H,S,D) with equal shapes, got {tuple(keys.shape)} / {tuple(values.shape)}")
@@ -142,21 +150,30 @@ class CompressHandle:
         npad = tb["N_near_padded"]
         near_k = torch.empty((B, H, npad, D), dtype=torch.float16, device=dev)
         near_v = torch.empty_like(near_k)
-        far_k = torch.empty((B, H, F, D), dtype=torch.uint8, device=dev)
-        far_v = torch.empty((B, H, F, D // 2), dtype=torch.uint8, device=dev)
-        vg = int(self.cfg.v_group)
-        fvs = torch.empty((B, H, F, D // vg) if vg else (B, H, F), dtype=torch.float16, device=dev)
-        fvz = torch.empty_like(fvs)
+        far_k = far_v = fvs = fvz = None
+        if far:
+            far_k = torch.empty((B, H, F, D), dtype=torch.uint8, device=dev)
+            far_v = torch.empty((B, H, F, D // 2), dtype=torch.uint8, device=dev)
+            vg = int(self.cfg.v_group)
+            fvs = torch.empty((B, H, F, D // vg) if vg else (B, H, F), dtype=torch.float16, device=dev)
+            fvz = torch.empty_like(fvs)
         near_valid = torch.empty((H,), dtype=torch.int32, device=dev)
         arc_k = torch.empty((B, H, F, D), dtype=torch.float16, device=dev) if with_archive else None
         arc_v = torch.empty_like(arc_k) if with_archive else None
-        ks = torch.empty((B, H), dtype=torch.float32, device=dev) if int(self.cfg.k_scale) else None
+        ks = torch.empty((B, H), dtype=torch.float32, device=dev) if far and int(self.cfg.k_scale) else None
         lib = _lib.load()
         c = self.cfg.to_c()
         near_idx = far_idx = None
         with torch.cuda.device(dev):
             if importance is not None:
                 near_idx, far_idx = partition_importance(self.cfg, importance, B, H, S)
+            if not far:
+                check(lib.fkv_archive_layer(
+                    ctypes.byref(c), ptr(k), ptr(v), dtype_code(k.dtype), B, H, S, D, ptr(near_idx), ptr(far_idx),
+                    ptr(near_k), ptr(near_v), ptr(near_valid), ptr(arc_k), ptr(arc_v), _lib.stream_ptr(dev)),
+                    "fkv_archive_layer")
+                return CompressedLayer(near_k, near_v, None, None, None, None, near_valid, tb["R_actual"],
+                                       arc_k, arc_v, near_idx, far_idx)
             check(lib.fkv_compress_layer_ex(
                 ctypes.byref(c), ptr(k), ptr(v), dtype_code(k.dtype), B, H, S, D, ptr(near_idx), ptr(far_idx),
                 ptr(near_k), ptr(near_v), ptr(far_k), ptr(far_v), ptr(fvs), ptr(fvz), ptr(ks), ptr(near_valid),

@@ -293,12 +293,12 @@ class TurboFoveatedHandle(ext.FoveatedHandle):
 
 def build_turbo_layer(cfg, keys, values, importance=None):
     """The turbo branch of _assign_and_build_layer (mlx_foveated.py:799-944):
-    near tier, archive and indices from the fused compress kernel, the far
+    near tier, archive and indices from the compress kernel, the far
     rows (fp16) compressed with TurboQuant; the fp8 far fields stay empty."""
     from .tier_cache import FoveatedLayer, tier_index_tensors
 
     B, H, S, D = keys.shape
-    cl = ext.CompressHandle(cfg.to_native()).compress_layer(keys, values, importance=importance)
+    cl = ext.CompressHandle(cfg.to_native()).archive_layer(keys, values, importance=importance)
     if cl.near_idx is not None:
         near_idx, far_idx = cl.near_idx, cl.far_idx
     else:

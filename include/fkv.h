@@ -145,6 +145,14 @@ int fkv_compress_layer_ex(const fkv_tier_config* cfg, const void* keys, const vo
                           void* far_v_scale, void* far_v_zero, float* far_k_scale, int32_t* near_valid,
                           void* archive_k, void* archive_v, void* stream);
 
+/* The near tier and the fp16 archive of far rows alone (fkv_compress_layer_ex
+ * without the fp8 / INT4 far tier): what a TurboQuant layer takes, whose far
+ * tier is compressed from the archive.  cfg->k_scale must be 0. */
+int fkv_archive_layer(const fkv_tier_config* cfg, const void* keys, const void* values, int32_t in_dtype,
+                      int32_t B, int32_t H, int32_t S, int32_t D, const int32_t* near_idx,
+                      const int32_t* far_idx, void* near_k, void* near_v, int32_t* near_valid,
+                      void* archive_k, void* archive_v, void* stream);
+
 /* ---------------------------------------------------------------------- */
 /* fused attention handle (FoveatedHandle, csrc/foveated_attn.cpp:135-254)  */
 /* ---------------------------------------------------------------------- */

@@ -494,3 +494,21 @@ def test_compress_past_the_cache(fkv, importance):
         part = h.compress_layer(k[b:b + 4], v[b:b + 4], importance=None if imp is None else imp[b:b + 4])
         for n in ("near_k", "near_v", "far_k", "far_v", "far_v_scale", "far_v_zero", "archive_k", "archive_v"):
             assert torch.equal(getattr(big, n)[b:b + 4], getattr(part, n)), n
+
+
+@pytest.mark.parametrize("importance", [False, True])
+@pytest.mark.parametrize("dt,S,D", [(torch.float16, 700, 128), (torch.bfloat16, 37, 64), (torch.float32, 2100, 64),
+                                    (torch.float16, 20, 128)])
+def test_archive_layer_is_the_compress_layer_without_far_codes(fkv, importance, dt, S, D):
+    from foveated_kv_amd import ext
+
+    g = torch.Generator(device="cuda").manual_seed(S)
+    k, v = (torch.randn((2, 3, S, D), generator=g, device="cuda").to(dt) for _ in range(2))
+    imp = torch.rand((2, 3, S), generator=g, device="cuda") if importance else None
+    flush(f"archive layer S={S} D={D} {dt} importance={importance}")
+    h = ext.CompressHandle(_cfg())
+    a, b = h.archive_layer(k, v, importance=imp), h.compress_layer(k, v, importance=imp)
+    for n in ("near_k", "near_v", "near_valid", "archive_k", "archive_v", "near_idx", "far_idx"):
+        x, y = getattr(a, n), getattr(b, n)
+        assert (x is None) == (y is None) and (x is None or torch.equal(x, y)), n
+    assert a.far_k is None and a.n_near_actual == b.n_near_actual
