@@ -24,14 +24,14 @@ namespace fkv {
 //
 // Three D x D products per token, all on the matrix cores
 // (v_mfma_f32_32x32x16_f16) at fp32 precision: every fp32 operand is split
-// into fp16 hi + lo / 2048 after a power-of-two scale that puts its row's
-// (token's) largest value near 1, the keys are fp16 already, products of
-// fp16 values are exact and summed in fp32, and the lo products run first
-// in the same accumulators, which are scaled by 1 / 2048 before the hi ones
-// (lo x lo, below 2^-24, is left out).  Against 64 bits over N(0, 1) keys
-// with outlier channels, 60 x 262,112 tokens: 99 codes and 201 signs off of
-// 2.0e9 at D = 128 (207 and 338 with fp32 FMA chains), 42 and 104 of 1.0e9
-// at D = 64 (70 and 125).
+// into fp16 hi + lo after a power-of-two scale that puts its row's (token's)
+// largest value near 1,024 (256), so that lo keeps its 11 bits above fp16's
+// subnormals; the keys are fp16 already, products of fp16 values are exact
+// and summed in fp32, and the lo products run first, while the sums are
+// small (lo x lo, below 2^-24, is left out).  Against 64 bits over N(0, 1) keys
+// with outlier channels, 40 x 262,112 tokens: 56 codes and 117 signs off of
+// 1.3e9 at D = 128 (123 and 235 with fp32 FMA chains), 23 and 71 of 6.7e8
+// at D = 64 (42 and 89).
 // The matrix is the A operand (rows = output dims) and the tokens are the B
 // operand (columns), so a lane's accumulators hold its own token's output
 // dims 32 rb + 8 a + 4 (lane / 32) + b; every product's K slots are numbered
@@ -42,12 +42,13 @@ typedef _Float16 fkv_h8 __attribute__((ext_vector_type(8)));
 typedef float fkv_f16v __attribute__((ext_vector_type(16)));
 
 constexpr int kTqTok = 128;  // tokens per workgroup of the key compressor (32 per wave)
-constexpr float kTqLo = 2048.0f;
+constexpr float kTqRow = 1024.0f, kTqTokn = 256.0f;  // the largest value of a matrix row / of a token's operand
 
 // The key compressor's prepared constants: per product (Pi, Pi^T, S) the lo
 // and the hi operand, [part][row block][K step][lane][8 halves]; the inverse
 // row scales of the first two products (the second times the centroids'
-// inverse scale); the boundaries ascending; the codes' centroids as hi | lo << 16.
+// inverse scale); the boundaries ascending; the four centroids' hi, then
+// their lo halves as byte tables (code c at bytes 2 c, 2 c + 1).
 __host__ __device__ constexpr size_t tq_op_bytes(int D) { return (size_t)4 * D * D; }
 __host__ __device__ constexpr size_t tq_scale_section(int D) { return 3 * tq_op_bytes(D); }
 __host__ __device__ constexpr size_t tq_const_section(int D) { return tq_scale_section(D) + (size_t)8 * D; }
@@ -61,7 +62,7 @@ __device__ inline float pow2_scale(float m, float& inv) {
 }
 __device__ inline void split_half(float x, uint16_t& hi, uint16_t& lo) {
     hi = f2h(x);
-    lo = f2h((x - h2f(hi)) * kTqLo);
+    lo = f2h(x - h2f(hi));
 }
 
 // Blocks 0 .. 3 D - 1: one output row of one product (64 threads); the last
@@ -87,11 +88,7 @@ __global__ __launch_bounds__(kWave) void tq_prep_kernel(const float* __restrict_
             }
         float* const c = (float*)(prep + tq_const_section(D));
         for (int i = 0; i < 3; i++) c[i] = b[i];
-        for (int i = 0; i < 4; i++) {
-            uint16_t hi, lo;
-            split_half(cb[i] * cscale, hi, lo);
-            ((uint32_t*)c)[4 + i] = (uint32_t)hi | ((uint32_t)lo << 16);
-        }
+        for (int i = 0; i < 4; i++) split_half(cb[i] * cscale * kTqTokn, ((uint16_t*)(c + 4))[i], ((uint16_t*)(c + 6))[i]);
         return;
     }
     const int op = blockIdx.x / D, i = blockIdx.x % D;
@@ -101,11 +98,11 @@ __global__ __launch_bounds__(kWave) void tq_prep_kernel(const float* __restrict_
     m = wave_max(m);
     float inv;
     const float scale = pow2_scale(m, inv);
-    if (op < 2 && lane == 0) scales[op * D + i] = op == 1 ? inv * cinv : inv;
+    if (op < 2 && lane == 0) scales[op * D + i] = (op == 1 ? inv * cinv / kTqTokn : inv) / kTqRow;
     uint16_t* const out = (uint16_t*)(prep + op * tq_op_bytes(D));
     for (int j = lane; j < D; j += kWave) {
         uint16_t hi, lo;
-        split_half(at(j) * scale, hi, lo);
+        split_half(at(j) * scale * kTqRow, hi, lo);
         // K step j / 16, lane half (j % 8) / 4, slot 4 ((j % 16) / 8) + j % 4
         const int64_t o = ((int64_t)((i / 32) * (D / 16) + j / 16) * 64 + (i % 32) + 32 * ((j % 8) / 4)) * 8 +
                           4 * ((j % 16) / 8) + j % 4;
@@ -149,18 +146,11 @@ struct TqGemm {
             for (int rb = 0; rb < NB; rb++) cur[rb] = nxt[rb];
         }
     }
-    __device__ inline void lo_done() {
-#pragma unroll
-        for (int rb = 0; rb < NB; rb++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[rb][i] *= 1.0f / kTqLo;
-    }
-    // fp32-precision product with the split operand hi + lo / kTqLo
+    // fp32-precision product with the split operand hi + lo
     __device__ inline void split(const fkv_h8 (&hi)[NS], const fkv_h8 (&lo)[NS]) {
         clear();
         add(0, hi);
         add(1, lo);
-        lo_done();
         add(1, hi);
     }
 };
@@ -177,9 +167,10 @@ __device__ inline float tq_half_sum(const float (&p)[8]) {
 // is done with them, while its results are turned into codes, residuals or
 // signs.  WIDE: keys and code buffers 16-byte aligned (else element loads
 // and byte stores).  Bound by issue: per 32 tokens of a wave 256 MFMAs (27 us
-// over 262K tokens at D = 128) and 2,300 vector instructions (31 us), and the
+// over 262K tokens at D = 128) and 2,000 vector instructions (27 us), and the
 // LDS reads of the operands (27 us).  4 x 8 heads x 8,191 tokens: 869 us with
-// fp32 FMA chains (30 TFLOP/s), 84 us now.
+// fp32 FMA chains (30 TFLOP/s), 78 us now (84 while the lo sums were scaled
+// before the hi ones and centroids were selected code by code).
 template <int D, bool WIDE>
 __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __restrict__ keys, int dtype, int64_t n_tok,
                                                                   const uint8_t* __restrict__ prep,
@@ -212,9 +203,8 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
     for (int i = tid; i < 2 * D; i += 256) sc_s[i] = ((const float*)(prep + tq_scale_section(D)))[i];
     const float* const cst = (const float*)(prep + tq_const_section(D));
     float b0 = cst[0], b1 = cst[1], b2 = cst[2];
-    uint32_t cw[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) cw[i] = ((const uint32_t*)cst)[4 + i];
+    const uint32_t* const tab = (const uint32_t*)cst + 4;
+    const uint32_t hi01 = tab[0], hi23 = tab[1], lo01 = tab[2], lo23 = tab[3];
     // the token's keys as the B operand: slots 0..3 of step s are dims 16 s +
     // 4 h .., slots 4..7 dims 16 s + 8 + 4 h ..
     fkv_h8 kb[NS];
@@ -276,7 +266,6 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
     ready();
     g.clear();
     g.add(0, kb);
-    g.lo_done();
     g.add(1, kb);
     __syncthreads();  // every wave is done with the operands
     fetch(1);
@@ -289,17 +278,25 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
         for (int a = 0; a < 4; a++) {
             const float4 sc = *(const float4*)&sc_s[32 * rb + 8 * a + 4 * h];
             const float f[4] = {sc.x, sc.y, sc.z, sc.w};
+            uint32_t c[4];
 #pragma unroll
             for (int b = 0; b < 4; b++) {
                 const float y = g.acc[rb][4 * a + b] * f[b];
-                const bool p0 = y >= b0, p1 = y >= b1, p2 = y >= b2;
-                uint32_t code = p2 ? 3u : p1 ? 2u : p0 ? 1u : 0u;
-                uint32_t c = p2 ? cw[3] : p1 ? cw[2] : p0 ? cw[1] : cw[0];
-                asm volatile("" : "+v"(code), "+v"(c));  // here, so that the masks end (they were spilled)
-                w[rb] |= code << (8 * a + 2 * b);
+                c[b] = (uint32_t)(y >= b0) + (uint32_t)(y >= b1) + (uint32_t)(y >= b2);
+                asm volatile("" : "+v"(c[b]));  // here, so that the lane masks end (they were spilled)
+                w[rb] |= c[b] << (8 * a + 2 * b);
+            }
+            // the centroids of two codes from the byte tables
+#pragma unroll
+            for (int b = 0; b < 4; b += 2) {
+                const uint32_t t = c[b] | (c[b + 1] << 16), sel = ((t << 1) | (t << 9)) + 0x01000100u;
+                const fkv_h2 ch = as_h2(__builtin_amdgcn_perm(hi23, hi01, sel)),
+                             cl = as_h2(__builtin_amdgcn_perm(lo23, lo01, sel));
                 const int s = 2 * rb + a / 2, e = 4 * (a % 2) + b;
-                hi[s][e] = __builtin_bit_cast(_Float16, (uint16_t)c);
-                lo[s][e] = __builtin_bit_cast(_Float16, (uint16_t)(c >> 16));
+                hi[s][e] = ch[0];
+                hi[s][e + 1] = ch[1];
+                lo[s][e] = cl[0];
+                lo[s][e + 1] = cl[1];
             }
         }
     }
@@ -350,10 +347,10 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
         out_norm[t] = f2h(nrm);
         out_gamma[t] = f2h(gamma);
     }
-    // the residual scaled so that its largest value is at most 2 (only the
+    // the residual scaled so that its largest value is at most 512 (only the
     // sign of its projections is kept); a non-finite one gives no sign
     const int ge = (int)((__float_as_uint(gamma) >> 23) & 0xFF);
-    const float rs = gamma < INFINITY ? __uint_as_float((uint32_t)(254 - min(ge, 253)) << 23) : 0.f;
+    const float rs = gamma < INFINITY ? __uint_as_float((uint32_t)(254 - min(ge, 253)) << 23) * (ge ? kTqTokn : 1.0f) : 0.f;
 #pragma unroll
     for (int rb = 0; rb < NB; rb++)
 #pragma unroll
