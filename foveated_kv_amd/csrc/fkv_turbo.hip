@@ -28,10 +28,11 @@ namespace fkv {
 // largest value near 1,024 (256), so that lo keeps its 11 bits above fp16's
 // subnormals; the keys are fp16 already, products of fp16 values are exact
 // and summed in fp32, and the lo products run first, while the sums are
-// small (lo x lo, below 2^-24, is left out).  Against 64 bits over N(0, 1) keys
-// with outlier channels, 40 x 262,112 tokens: 56 codes and 117 signs off of
-// 1.3e9 at D = 128 (123 and 235 with fp32 FMA chains), 23 and 71 of 6.7e8
-// at D = 64 (42 and 89).
+// small (lo x lo, below 2^-24, is left out).  A token with a rotated
+// coordinate that close to a boundary (1 in 6,000) takes its codes from
+// 64-bit sums.  Against 64 bits over N(0, 1) keys with outlier channels, 20 x
+// 262,112 tokens: no code and 62 signs off of 6.7e8 at D = 128 (59 and 121
+// with fp32 FMA chains), none and 36 of 3.4e8 at D = 64 (18 and 48).
 // The matrix is the A operand (rows = output dims) and the tokens are the B
 // operand (columns), so a lane's accumulators hold its own token's output
 // dims 32 rb + 8 a + 4 (lane / 32) + b; every product's K slots are numbered
@@ -48,7 +49,7 @@ constexpr float kTqRow = 1024.0f, kTqTokn = 256.0f;  // the largest value of a m
 // and the hi operand, [part][row block][K step][lane][8 halves]; the inverse
 // row scales of the first two products (the second times the centroids'
 // inverse scale); the boundaries ascending; the four centroids' hi, then
-// their lo halves as byte tables (code c at bytes 2 c, 2 c + 1).
+// their lo halves as byte tables (code c at bytes 2 (3 - c), 2 (3 - c) + 1).
 __host__ __device__ constexpr size_t tq_op_bytes(int D) { return (size_t)4 * D * D; }
 __host__ __device__ constexpr size_t tq_scale_section(int D) { return 3 * tq_op_bytes(D); }
 __host__ __device__ constexpr size_t tq_const_section(int D) { return tq_scale_section(D) + (size_t)8 * D; }
@@ -88,7 +89,8 @@ __global__ __launch_bounds__(kWave) void tq_prep_kernel(const float* __restrict_
             }
         float* const c = (float*)(prep + tq_const_section(D));
         for (int i = 0; i < 3; i++) c[i] = b[i];
-        for (int i = 0; i < 4; i++) split_half(cb[i] * cscale * kTqTokn, ((uint16_t*)(c + 4))[i], ((uint16_t*)(c + 6))[i]);
+        for (int i = 0; i < 4; i++)  // entry 3 - code
+            split_half(cb[3 - i] * cscale * kTqTokn, ((uint16_t*)(c + 4))[i], ((uint16_t*)(c + 6))[i]);
         return;
     }
     const int op = blockIdx.x / D, i = blockIdx.x % D;
@@ -161,19 +163,95 @@ __device__ inline float tq_half_sum(const float (&p)[8]) {
     return s + __shfl_xor(s, 32);
 }
 
+// fp16 bits of the centroids of two codes (given as 3 - code in the halves of
+// c01, c23) from the byte tables: two per dword.
+__device__ inline void centroids4(uint32_t t01, uint32_t t23, uint32_t c01, uint32_t c23, uint32_t& o01, uint32_t& o23) {
+    o01 = __builtin_amdgcn_perm(t23, t01, ((c01 << 1) | (c01 << 9)) + 0x01000100u);
+    o23 = __builtin_amdgcn_perm(t23, t01, ((c23 << 1) | (c23 << 9)) + 0x01000100u);
+}
+
+// Slots 4 u .. 4 u + 3 of an operand.
+__device__ inline void put4(fkv_h8& o, int u, uint32_t w01, uint32_t w23) {
+    const fkv_h2 x = as_h2(w01), y = as_h2(w23);
+    o[4 * u] = x[0];
+    o[4 * u + 1] = x[1];
+    o[4 * u + 2] = y[0];
+    o[4 * u + 3] = y[1];
+}
+
+// The codes of one token in 64 bits, by the whole wave: dim i's code from
+// lane i % 64, returned as masks of the codes' low and high bits per 64 dims.
+// For tokens with a rotated coordinate so near a boundary that the fp32-precision
+// sums may fall on the wrong side of it (one token in 6,000).
+template <int D, bool WIDE>
+__device__ inline void exact_codes(const void* keys, int dtype, int64_t t, const float* __restrict__ Pi, const float* bd,
+                                   int lane, uint64_t (&m0)[D / 64], uint64_t (&m1)[D / 64]) {
+    float k[D / 64];
+    double ss = 0.0, y[D / 64];
+#pragma unroll
+    for (int i = 0; i < D / 64; i++) {
+        k[i] = h2f(load_as_f16(keys, t * D + 64 * i + lane, dtype));
+        ss += (double)k[i] * (double)k[i];
+        y[i] = 0.0;
+    }
+    for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
+    const double nc = fmax(sqrt(ss), (double)1e-8f);
+    // matrix elements in flight per row (a lane reads along its own rows): the
+    // wave waits for D / U of these round trips, and its workgroup for it
+    constexpr int U = WIDE ? 32 : 8;
+#pragma unroll
+    for (int jj = 0; jj < D / 64; jj++)
+#pragma unroll 1
+        for (int j0 = 0; j0 < 64; j0 += U) {
+            float m[D / 64][U];
+#pragma unroll
+            for (int i = 0; i < D / 64; i++) {
+                const float* p = Pi + (int64_t)(64 * i + lane) * D + 64 * jj + j0;
+#pragma unroll
+                for (int u = 0; u < U; u += 4) {
+                    if (WIDE) {
+                        const float4 v = *(const float4*)(p + u);
+                        m[i][u] = v.x;
+                        m[i][u + 1] = v.y;
+                        m[i][u + 2] = v.z;
+                        m[i][u + 3] = v.w;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) m[i][u + e] = p[u + e];
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const double kj = (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(k[jj]), j0 + u));
+#pragma unroll
+                for (int i = 0; i < D / 64; i++) y[i] = fma(kj, (double)m[i][u], y[i]);
+            }
+        }
+#pragma unroll
+    for (int i = 0; i < D / 64; i++) {
+        const double v = y[i] / nc;
+        const int c = (v >= (double)bd[0]) + (v >= (double)bd[1]) + (v >= (double)bd[2]);
+        m0[i] = __ballot(c & 1);
+        m1[i] = __ballot(c & 2);
+    }
+}
+
 // One workgroup of four waves per 128 tokens, two workgroups per CU (64 KB of
 // LDS each at D = 128): one's vector work overlaps the other's matrix work.
 // Each product's operands come to LDS by LDS DMA once the previous product
 // is done with them, while its results are turned into codes, residuals or
-// signs.  WIDE: keys and code buffers 16-byte aligned (else element loads
+// signs.  WIDE: keys, Pi and code buffers 16-byte aligned (else element loads
 // and byte stores).  Bound by issue: per 32 tokens of a wave 256 MFMAs (27 us
-// over 262K tokens at D = 128) and 2,000 vector instructions (27 us), and the
+// over 262K tokens at D = 128) and 2,200 vector instructions (29 us), and the
 // LDS reads of the operands (27 us).  4 x 8 heads x 8,191 tokens: 869 us with
-// fp32 FMA chains (30 TFLOP/s), 78 us now (84 while the lo sums were scaled
-// before the hi ones and centroids were selected code by code).
+// fp32 FMA chains (30 TFLOP/s), 84 us now: 78 without the test for close
+// coordinates, 81 without the few 64-bit ones, whose wave its workgroup and
+// at the end the launch wait for.
 template <int D, bool WIDE>
 __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __restrict__ keys, int dtype, int64_t n_tok,
                                                                   const uint8_t* __restrict__ prep,
+                                                                  const float* __restrict__ Pi,
                                                                   uint8_t* __restrict__ out_idx,
                                                                   uint8_t* __restrict__ out_sgn,
                                                                   uint16_t* __restrict__ out_norm,
@@ -255,11 +333,11 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
         for (int e = 0; e < 8; e++) ss[e] = fmaf((float)kb[s][e], (float)kb[s][e], ss[e]);
     const float nrm = sqrtf(tq_half_sum(ss));
     {
-        // y >= b  <=>  k Pi^T >= b max(n, 1e-8); no code of a non-finite norm
-        const float nc = fmaxf(nrm, 1e-8f), nan = __uint_as_float(0x7FC00000u);
-        b0 = nc < INFINITY ? b0 * nc : nan;
-        b1 = nc < INFINITY ? b1 * nc : nan;
-        b2 = nc < INFINITY ? b2 * nc : nan;
+        // y >= b  <=>  k Pi^T >= b max(n, 1e-8)
+        const float nc = fmaxf(nrm, 1e-8f);
+        b0 *= nc;
+        b1 *= nc;
+        b2 *= nc;
     }
     TqGemm<D> g{op_s, lane, {}};
     // ---- codes ----
@@ -271,6 +349,7 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
     fetch(1);
     fkv_h8 hi[NS], lo[NS];
     uint32_t w[NB];
+    float gap = INFINITY;  // the least distance of a coordinate from a boundary
 #pragma unroll
     for (int rb = 0; rb < NB; rb++) {
         w[rb] = 0;
@@ -281,22 +360,65 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
             uint32_t c[4];
 #pragma unroll
             for (int b = 0; b < 4; b++) {
-                const float y = g.acc[rb][4 * a + b] * f[b];
-                c[b] = (uint32_t)(y >= b0) + (uint32_t)(y >= b1) + (uint32_t)(y >= b2);
-                asm volatile("" : "+v"(c[b]));  // here, so that the lane masks end (they were spilled)
+                // the boundaries above the coordinate: 3 - code.  The signs of
+                // the differences are exact (f is a power of two), and a zero
+                // one is positive; compares would leave lane masks to spill
+                const float y = g.acc[rb][4 * a + b];
+                const float d0 = fmaf(y, f[b], -b0), d1 = fmaf(y, f[b], -b1), d2 = fmaf(y, f[b], -b2);
+                c[b] = (__float_as_uint(d0) >> 31) + (__float_as_uint(d1) >> 31) + (__float_as_uint(d2) >> 31);
+                gap = fminf(fminf(fminf(fabsf(d0), fabsf(d1)), fabsf(d2)), gap);
                 w[rb] |= c[b] << (8 * a + 2 * b);
             }
-            // the centroids of two codes from the byte tables
+            // the centroids' halves, two codes at a time
+            uint32_t h01, h23, l01, l23;
+            centroids4(hi01, hi23, c[0] | (c[1] << 16), c[2] | (c[3] << 16), h01, h23);
+            centroids4(lo01, lo23, c[0] | (c[1] << 16), c[2] | (c[3] << 16), l01, l23);
+            put4(hi[2 * rb + a / 2], a % 2, h01, h23);
+            put4(lo[2 * rb + a / 2], a % 2, l01, l23);
+        }
+        w[rb] = ~w[rb];  // the codes
+    }
+    // tokens with a coordinate within twelve standard deviations of the sums'
+    // error (5e-9 of the norm) take their codes from 64-bit sums
+    const uint64_t close = __ballot(live && nrm > 0.f && nrm < INFINITY && gap < 6e-8f * nrm);
+    const bool odd_norm = !(nrm < INFINITY);
+    uint32_t redo = (uint32_t)close | (uint32_t)(close >> 32);
+    if (redo || __ballot(odd_norm)) {
+        while (redo) {
+            const int tl = __builtin_ctz(redo);
+            redo &= redo - 1;
+            uint64_t m0[D / 64], m1[D / 64];
+            exact_codes<D, WIDE>(keys, dtype, (int64_t)blockIdx.x * kTqTok + wave * 32 + tl, Pi, cst, lane, m0, m1);
+            if ((lane & 31) == tl) {
 #pragma unroll
-            for (int b = 0; b < 4; b += 2) {
-                const uint32_t t = c[b] | (c[b + 1] << 16), sel = ((t << 1) | (t << 9)) + 0x01000100u;
-                const fkv_h2 ch = as_h2(__builtin_amdgcn_perm(hi23, hi01, sel)),
-                             cl = as_h2(__builtin_amdgcn_perm(lo23, lo01, sel));
-                const int s = 2 * rb + a / 2, e = 4 * (a % 2) + b;
-                hi[s][e] = ch[0];
-                hi[s][e + 1] = ch[1];
-                lo[s][e] = cl[0];
-                lo[s][e + 1] = cl[1];
+                for (int rb = 0; rb < NB; rb++) {
+                    w[rb] = 0;
+#pragma unroll
+                    for (int a = 0; a < 4; a++) {
+                        // four low and four high bits interleaved
+                        const int at = (32 * rb + 8 * a) % 64 + 4 * h;
+                        uint32_t x = (uint32_t)(m0[rb / 2] >> at) & 15u, z = (uint32_t)(m1[rb / 2] >> at) & 15u;
+                        x = (x | (x << 2)) & 0x33u;
+                        x = (x | (x << 1)) & 0x55u;
+                        z = (z | (z << 2)) & 0x33u;
+                        z = (z | (z << 1)) & 0x55u;
+                        w[rb] |= (x | (z << 1)) << (8 * a);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int rb = 0; rb < NB; rb++) {
+            if (odd_norm) w[rb] = 0;  // no code of a non-finite norm
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                const uint32_t q = ~w[rb] >> (8 * a);
+                const uint32_t c01 = (q & 3u) | ((q & 12u) << 14), c23 = ((q >> 4) & 3u) | ((q & 192u) << 10);
+                uint32_t h01, h23, l01, l23;
+                centroids4(hi01, hi23, c01, c23, h01, h23);
+                centroids4(lo01, lo23, c01, c23, l01, l23);
+                put4(hi[2 * rb + a / 2], a % 2, h01, h23);
+                put4(lo[2 * rb + a / 2], a % 2, l01, l23);
             }
         }
     }
@@ -550,11 +672,11 @@ int fkv_turbo_compress_keys(const void* keys, int32_t dtype, int64_t n_tokens, i
                        boundaries, D, prep);
     // vector loads and stores where the caller's arrays are 16-byte aligned
     // (a token's rows then are too)
-    const bool wide = (((uintptr_t)keys | (uintptr_t)out_idx | (uintptr_t)out_signs) & 15) == 0;
+    const bool wide = (((uintptr_t)keys | (uintptr_t)Pi | (uintptr_t)out_idx | (uintptr_t)out_signs) & 15) == 0;
     auto* kern = D == 128 ? (wide ? fkv::tq_compress_keys_kernel<128, true> : fkv::tq_compress_keys_kernel<128, false>)
                           : (wide ? fkv::tq_compress_keys_kernel<64, true> : fkv::tq_compress_keys_kernel<64, false>);
     hipLaunchKernelGGL(kern, dim3((unsigned)fkv::cdiv(n_tokens, fkv::kTqTok)), dim3(256), 0, st, keys, dtype, n_tokens,
-                       prep, out_idx, out_signs, (uint16_t*)out_norm, (uint16_t*)out_gamma);
+                       prep, Pi, out_idx, out_signs, (uint16_t*)out_norm, (uint16_t*)out_gamma);
     rc = check_hip(hipGetLastError(), "tq_compress_keys_kernel launch");
     (void)hipFreeAsync(prep, st);
     return rc;

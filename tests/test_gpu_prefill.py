@@ -512,3 +512,26 @@ def test_archive_layer_is_the_compress_layer_without_far_codes(fkv, importance, 
         x, y = getattr(a, n), getattr(b, n)
         assert (x is None) == (y is None) and (x is None or torch.equal(x, y)), n
     assert a.far_k is None and a.n_near_actual == b.n_near_actual
+
+
+@pytest.mark.parametrize("D,dt", [(64, torch.float16), (128, torch.float16), (128, torch.float32)])
+def test_turbo_codes_are_the_64_bit_ones(fkv, D, dt):
+    """Coordinates near a boundary are decided by 64-bit sums: over 200,000
+    tokens (about 30 of them near one; with zero and padded ones) every code
+    is the one that fp64 gives."""
+    from foveated_kv_amd.turbo import get_turbo_constants, turbo_compress_keys
+
+    g = torch.Generator(device="cuda").manual_seed(D)
+    n = 200_003
+    k = torch.randn((1, 1, n, D), generator=g, device="cuda")
+    k[..., :4] *= 8
+    k[0, 0, 5] = 0
+    k = k.to(dt)
+    tc = get_turbo_constants(D)
+    flush(f"turbo codes against fp64 D={D} {dt} n={n}")
+    idx = turbo_compress_keys(k, tc)[0]
+    got = ((idx.unsqueeze(-1) >> torch.tensor([0, 2, 4, 6], device="cuda", dtype=torch.uint8)) & 3).flatten(-2)
+    kd = k.half().double()
+    y = (kd @ tc.Pi.cuda().double().T.contiguous()) / kd.norm(dim=-1, keepdim=True).clamp_min(np.float32(1e-8))
+    want = torch.bucketize(y, tc.boundaries.cuda().double(), right=True)
+    assert int((got != want).sum()) == 0
