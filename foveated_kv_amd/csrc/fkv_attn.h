@@ -95,20 +95,11 @@ __host__ __device__ constexpr int tq_sc_index(int D, int blk, int half, int e, i
 __host__ __device__ constexpr int64_t g32_sz_section(int D) { return (int64_t)96 * D; }
 __host__ __device__ constexpr int64_t g32_record_bytes(int D) { return (int64_t)104 * D; }
 
-// Byte of the E4M3 code of (token t, dim d) inside its tile's K section.
-__host__ __device__ inline int64_t far_k_index(int t, int d) {
-    return (int64_t)(d >> 4) * 1024 + (t & 63) * 16 + (d & 15);
-}
-// Far V nibble of (token t, dim d) inside its tile's V section: dword index
-// and bit position.  Dword u of a lane holds 4-token groups 2(u%8) (bits
-// 0-7, 16-23) and 2(u%8)+1 (bits 8-15, 24-31) of dim half u/8; token e of a
-// group sits at bit 16(e&1) + 4(e>>1) of its byte pair.
-__host__ __device__ inline void far_v_pos(int t, int d, int64_t& dword, int& bit) {
-    const int sp = (t & 63) >> 2, e = t & 3;
-    const int u = (d >> 6) * 8 + (sp >> 1);
-    dword = (int64_t)(u >> 2) * 256 + (d & 63) * 4 + (u & 3);
-    bit = (sp & 1) * 8 + (e & 1) * 16 + (e >> 1) * 4;
-}
+// Far K: the E4M3 code of (token t, dim d) is byte (d >> 4) * 1024 + (t & 63)
+// * 16 + (d & 15) of its tile's K section.  Far V: dword u of a lane holds
+// 4-token groups 2(u%8) (bits 0-7, 16-23) and 2(u%8)+1 (bits 8-15, 24-31) of
+// dim half u/8; token e of a group sits at bit 16(e&1) + 4(e>>1) of its byte
+// pair, dword (u >> 2) * 256 + lane * 4 + (u & 3) of the V section.
 
 // Element i of an fp16 / bf16 / fp32 array as fp16 bits (round to nearest even).
 __device__ inline uint16_t load_as_f16(const void* p, int64_t i, int dtype) {

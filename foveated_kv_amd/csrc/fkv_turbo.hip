@@ -43,7 +43,7 @@ typedef _Float16 fkv_h8 __attribute__((ext_vector_type(8)));
 typedef float fkv_f16v __attribute__((ext_vector_type(16)));
 
 constexpr int kTqTok = 128;  // tokens per workgroup of the key compressor (32 per wave)
-constexpr float kTqRow = 1024.0f, kTqTokn = 256.0f;  // the largest value of a matrix row / of a token's operand
+constexpr float kTqRow = 1024.0f, kTqVec = 256.0f;  // the largest value of a matrix row / of a token's operand
 
 // The key compressor's prepared constants: per product (Pi, Pi^T, S) the lo
 // and the hi operand, [part][row block][K step][lane][8 halves]; the inverse
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(kWave) void tq_prep_kernel(const float* __restrict_
         float* const c = (float*)(prep + tq_const_section(D));
         for (int i = 0; i < 3; i++) c[i] = b[i];
         for (int i = 0; i < 4; i++)  // entry 3 - code
-            split_half(cb[3 - i] * cscale * kTqTokn, ((uint16_t*)(c + 4))[i], ((uint16_t*)(c + 6))[i]);
+            split_half(cb[3 - i] * cscale * kTqVec, ((uint16_t*)(c + 4))[i], ((uint16_t*)(c + 6))[i]);
         return;
     }
     const int op = blockIdx.x / D, i = blockIdx.x % D;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kWave) void tq_prep_kernel(const float* __restrict_
     m = wave_max(m);
     float inv;
     const float scale = pow2_scale(m, inv);
-    if (op < 2 && lane == 0) scales[op * D + i] = (op == 1 ? inv * cinv / kTqTokn : inv) / kTqRow;
+    if (op < 2 && lane == 0) scales[op * D + i] = (op == 1 ? inv * cinv / kTqVec : inv) / kTqRow;
     uint16_t* const out = (uint16_t*)(prep + op * tq_op_bytes(D));
     for (int j = lane; j < D; j += kWave) {
         uint16_t hi, lo;
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
     // the residual scaled so that its largest value is at most 512 (only the
     // sign of its projections is kept); a non-finite one gives no sign
     const int ge = (int)((__float_as_uint(gamma) >> 23) & 0xFF);
-    const float rs = gamma < INFINITY ? __uint_as_float((uint32_t)(254 - min(ge, 253)) << 23) * (ge ? kTqTokn : 1.0f) : 0.f;
+    const float rs = gamma < INFINITY ? __uint_as_float((uint32_t)(254 - min(ge, 253)) << 23) * (ge ? kTqVec : 1.0f) : 0.f;
 #pragma unroll
     for (int rb = 0; rb < NB; rb++)
 #pragma unroll
@@ -665,6 +665,11 @@ int fkv_turbo_compress_keys(const void* keys, int32_t dtype, int64_t n_tokens, i
     if (!keys || !Pi || !S || !centroids || !boundaries || !out_idx || !out_signs || !out_norm || !out_gamma)
         return set_error("fkv_turbo_compress_keys: NULL argument");
     hipStream_t st = (hipStream_t)stream;
+    // the constants' workspace is allocated and freed by each call, which a
+    // captured graph could not replay
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (int rc = check_hip(hipStreamIsCapturing(st, &cs), "hipStreamIsCapturing")) return rc;
+    if (cs != hipStreamCaptureStatusNone) return set_error("fkv_turbo_compress_keys: not under graph capture");
     uint8_t* prep = nullptr;
     int rc = check_hip(hipMallocAsync((void**)&prep, fkv::tq_prep_bytes(D), st), "hipMallocAsync");
     if (rc) return rc;

@@ -535,3 +535,18 @@ def test_turbo_codes_are_the_64_bit_ones(fkv, D, dt):
     y = (kd @ tc.Pi.cuda().double().T.contiguous()) / kd.norm(dim=-1, keepdim=True).clamp_min(np.float32(1e-8))
     want = torch.bucketize(y, tc.boundaries.cuda().double(), right=True)
     assert int((got != want).sum()) == 0
+
+
+def test_turbo_keys_refused_under_capture(fkv):
+    from foveated_kv_amd.turbo import get_turbo_constants, turbo_compress_keys
+
+    k = torch.randn((1, 1, 64, 64), device="cuda").half()
+    tc = get_turbo_constants(64)
+    turbo_compress_keys(k, tc)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        with pytest.raises(Exception, match="graph capture"):
+            turbo_compress_keys(k, tc)
+    want = turbo_compress_keys(k, tc)
+    assert all(torch.equal(a, b) for a, b in zip(turbo_compress_keys(k, tc), want))
