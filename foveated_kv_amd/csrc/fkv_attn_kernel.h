@@ -83,6 +83,11 @@ struct AttnArgs {
     int num_splits;
     float spike_margin;
     float inv_sqrt_d;
+    // QC kernels: FKV_BF16 or FKV_F32, rounded to fp16 in the prologue. Held
+    // here, where alignment leaves a gap: at the end of the struct it makes the
+    // argument block 568 bytes in place of 560, and a call measured 6.22 us
+    // against 6.16 (512 tokens) and 10.27 against 10.21 (4096 tokens)
+    int q_dtype;
     uint16_t* out;  // (B, Hq, D) fp16
     int32_t* flags;
     int32_t* tokens;
@@ -115,7 +120,6 @@ struct AttnArgs {
     // per-head fp8 key scales, (B*Hkv) fp32 in the blob; NULL for a handle
     // whose keys are unscaled (no load then: the scale is 1)
     const float* kscale;
-    int q_dtype;  // QC kernels: FKV_BF16 or FKV_F32, rounded to fp16 in the prologue
 #ifdef FKV_PHASE_STAMPS
     unsigned long long* stamps;  // kStampSlots per workgroup (fkv_phase_stamps)
 #endif
