@@ -295,9 +295,11 @@ class FoveatedLayer:
         if self._kcache is not None:
             return
         if self.compress_method == "turbo":
-            from .turbo import TurboFoveatedHandle
+            from .turbo import TurboConstants, TurboFoveatedHandle
 
-            tc = self._turbo_constants.on(self.near_k.device)
+            tc = self._turbo_constants
+            if isinstance(tc, TurboConstants):
+                tc = tc.on(self.near_k.device)
             handle = TurboFoveatedHandle(
                 self.near_k, self.near_v, self.turbo_far_k_indices, self.turbo_far_k_signs,
                 self.turbo_far_k_norm, self.turbo_far_k_gamma, self.turbo_far_v_packed,

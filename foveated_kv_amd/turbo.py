@@ -36,8 +36,9 @@ from ._lib import check, dtype_code, ptr
 @dataclass(frozen=True)
 class TurboConstants:
     """Pi (D,D) rotation, S (D,D) QJL matrix, Lloyd-Max centroids (4,) and
-    boundaries (3,), fp32 CPU tensors; ``on(device)`` returns device copies
-    (cached)."""
+    boundaries (3,), fp32 CPU tensors; ``on(device)`` returns device copies,
+    kept on this object (never by its id, which a later object can have) and
+    made anew when a tensor was written to."""
 
     Pi: torch.Tensor
     S: torch.Tensor
@@ -45,19 +46,22 @@ class TurboConstants:
     boundaries: torch.Tensor
 
     def on(self, device):
-        return _constants_on(self, torch.device(device))
+        device = torch.device(device)
+        if device.type == "cuda" and device.index is None:
+            device = torch.device("cuda", torch.cuda.current_device())
+        src = (self.Pi, self.S, self.centroids, self.boundaries)
+        if any(not isinstance(t, torch.Tensor) or t.is_inference() for t in src):
+            # nothing says whether these were written to: copied on each call
+            return TurboConstants(*(torch.as_tensor(t).to(device) for t in src))
+        versions = tuple(t._version for t in src)
+        copies = self.__dict__.setdefault("_device_copies", {})
+        hit = copies.get(device)
+        if hit is None or hit[0] != versions:
+            hit = copies[device] = (versions, TurboConstants(*(t.to(device) for t in src)))
+        return hit[1]
 
-
-_device_cache = {}
-
-
-def _constants_on(tc, device):
-    key = (id(tc), str(device))
-    hit = _device_cache.get(key)
-    if hit is None:
-        hit = TurboConstants(tc.Pi.to(device), tc.S.to(device), tc.centroids.to(device), tc.boundaries.to(device))
-        _device_cache[key] = hit
-    return hit
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_device_copies"}
 
 
 def _rotation_matrix(d, seed):
@@ -114,9 +118,10 @@ def _lloyd_max(d, bits=2, n_iters=200):
 @lru_cache(maxsize=4)
 def get_turbo_constants(d: int, pi_seed: int = 42, s_seed: int = 137) -> TurboConstants:
     c, b = _lloyd_max(d)
-    return TurboConstants(Pi=torch.from_numpy(_rotation_matrix(d, pi_seed)),
-                          S=torch.from_numpy(_qjl_matrix(d, s_seed)),
-                          centroids=torch.from_numpy(c), boundaries=torch.from_numpy(b))
+    with torch.inference_mode(False):  # kept: ordinary tensors whoever asks first
+        return TurboConstants(Pi=torch.from_numpy(_rotation_matrix(d, pi_seed)),
+                              S=torch.from_numpy(_qjl_matrix(d, s_seed)),
+                              centroids=torch.from_numpy(c), boundaries=torch.from_numpy(b))
 
 
 # ---------------------------------------------------------------------------
