@@ -148,6 +148,10 @@ def turbo_compress_keys(keys: torch.Tensor, tc: TurboConstants):
     if k.numel() == 0:
         return idx, sgn, nrm, gam
     c = tc.on(dev)
+    # the kernel reads D * D, 4 and 3 elements whatever the constants hold
+    for name, n in (("Pi", D * D), ("S", D * D), ("centroids", 4), ("boundaries", 3)):
+        if getattr(c, name).numel() != n:
+            raise ValueError(f"{name} has {getattr(c, name).numel()} elements, keys of {D} dims need {n}")
     lib = _lib.load()
     with torch.cuda.device(dev):
         check(lib.fkv_turbo_compress_keys(ptr(k), dtype_code(k.dtype), B * H * N, D, ptr(_f32(c.Pi, dev)),

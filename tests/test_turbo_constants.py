@@ -62,6 +62,29 @@ def test_built_in_constants_are_ordinary_tensors_in_inference_mode():
         assert not tc.Pi.is_inference() and tc.on("meta") is tc.on("meta")
 
 
+@pytest.mark.parametrize("name,shape", [("Pi", (8, 8)), ("S", (8, 8)), ("S", (32, 16)), ("centroids", (3,)),
+                                        ("boundaries", (2,))])
+def test_constants_of_another_head_dim_are_refused(monkeypatch, name, shape):
+    """Before the library is called: its kernel would read past their end."""
+    import dataclasses
+
+    from foveated_kv_amd import _lib, ext, turbo
+
+    class Reached(Exception):
+        pass
+
+    def load():
+        raise Reached
+
+    monkeypatch.setattr(ext, "_require_device", lambda *a: None)
+    monkeypatch.setattr(_lib, "load", load)
+    keys = torch.zeros((1, 1, 3, 16), dtype=torch.float16)
+    with pytest.raises(Reached):
+        turbo.turbo_compress_keys(keys, _constants(3))
+    with pytest.raises(ValueError, match=name):
+        turbo.turbo_compress_keys(keys, dataclasses.replace(_constants(3), **{name: torch.zeros(shape)}))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
 def test_fused_attention_takes_the_layers_own_constants(D):
