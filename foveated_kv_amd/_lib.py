@@ -117,6 +117,7 @@ SIGNATURES = {
     "fkv_phase_stamps": (ctypes.c_int, [P, I32, I32]),
     "fkv_xcd_watch_violations": (ctypes.c_int32, [P, I32]),
     "fkv_attn_destroy": (None, [P]),
+    "fkv_attn_try_destroy": (ctypes.c_int, [P]),
     "fkv_attn_set_k_scale": (ctypes.c_int, [P, P, P]),
     "fkv_attn_set_spike_k": (ctypes.c_int, [P, I32]),
     "fkv_e4m3_decode": (ctypes.c_int, [P, P, ctypes.c_int64, P]),

@@ -1189,6 +1189,28 @@ void free_spike_buffers(fkv_attn* h) {
     h->spk_cand_n = h->spk_arrive = h->spk_cand_t = nullptr;
 }
 
+// Waits until no work on the handle's device can use its memory.  Fails,
+// without having waited, while a stream captures; the error is reported here
+// and not left for the next launch's hipGetLastError.
+int wait_for_device(const fkv_attn* h) {
+    int dev = -1;
+    int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
+    if (!rc && dev != h->device) rc = check_hip(hipSetDevice(h->device), "hipSetDevice");
+    if (!rc) rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
+    if (dev >= 0 && dev != h->device) (void)hipSetDevice(dev);
+    if (rc) (void)hipGetLastError();
+    return rc;
+}
+
+// The handle and all memory that is its own.
+void release(fkv_attn* h) {
+    if (h->blob && h->own_blob) (void)hipFree(h->blob);
+    free_spike_buffers(h);
+    if (h->ws) (void)hipFree(h->ws);
+    if (h->order_ev) (void)hipEventDestroy(h->order_ev);
+    delete h;
+}
+
 // The top-K spike selection's buffers for Hq query heads (spike_k > 1).
 int ensure_spike_buffers(fkv_attn* h, int Hq) {
     if (h->spike_k <= 1 || h->spk_hq == Hq) return FKV_OK;
@@ -1733,21 +1755,19 @@ int fkv_attn_set_k_scale(fkv_attn* h, const float* k_scale, void* stream) {
     return rc;
 }
 
+int fkv_attn_try_destroy(fkv_attn* h) {
+    if (!h) return FKV_OK;
+    if (int rc = wait_for_device(h)) return rc;
+    release(h);
+    return FKV_OK;
+}
+
 void fkv_attn_destroy(fkv_attn* h) {
     if (!h) return;
     // hipFree waits for the device; a caller's blob must be as free of work
     // when this returns as one freed here
-    if (h->blob && !h->own_blob) {
-        int dev = -1;
-        if (hipGetDevice(&dev) == hipSuccess && dev != h->device) (void)hipSetDevice(h->device);
-        (void)hipDeviceSynchronize();
-        if (dev >= 0 && dev != h->device) (void)hipSetDevice(dev);
-    }
-    if (h->blob && h->own_blob) (void)hipFree(h->blob);
-    free_spike_buffers(h);
-    if (h->ws) (void)hipFree(h->ws);
-    if (h->order_ev) (void)hipEventDestroy(h->order_ev);
-    delete h;
+    if (h->blob && !h->own_blob) (void)wait_for_device(h);
+    release(h);
 }
 
 }  // extern "C"

@@ -10,6 +10,7 @@ Tensors are torch tensors on a ROCm device instead of mx.array.  Every call
 is enqueued on torch's current stream of the tensors' device.
 """
 
+import collections
 import ctypes
 
 import torch
@@ -235,6 +236,33 @@ class BlobWriteInfo:
         self.D = c.D
 
 
+# Handles dropped while the device could not be waited for (a stream was
+# capturing), with their blobs: calls of theirs may still run, so both stay
+# until a later handle is made or dropped.
+_undestroyed = collections.deque()
+
+
+def _destroy(lib, h, blob):
+    """Destroys handle ``h``, after which ``blob`` is idle, or keeps both."""
+    done = False
+    try:
+        done = not torch.cuda.is_current_stream_capturing() and lib.fkv_attn_try_destroy(h) == _lib.FKV_OK
+    finally:
+        if not done:
+            _undestroyed.append((lib, h, blob))
+    return done
+
+
+def _destroy_kept():
+    for _ in range(len(_undestroyed)):
+        try:
+            kept = _undestroyed.popleft()
+        except IndexError:  # another thread took it
+            return
+        if not _destroy(*kept):
+            return
+
+
 class FoveatedHandle:
     """FoveatedHandle (csrc/foveated_attn.cpp:135-254): copies the static tier
     arrays into a private device blob; calling it launches the fused kernel.
@@ -303,7 +331,8 @@ class FoveatedHandle:
         hipMalloc and hipFree of 84 MB took about 400 us of every handle).
         Destroying the handle waits for the device before the tensor goes
         back to the allocator, so work on any stream -- calls, promotions,
-        graph replays -- is done with it by then."""
+        graph replays -- is done with it by then (_destroy)."""
+        _destroy_kept()
         n = lib.fkv_attn_blob_bytes(self.B, self.H_kv, self.D, self.N_near, self.N_far, fmt)
         if n < 0:
             check(int(n), "fkv_attn_blob_bytes")
@@ -318,8 +347,9 @@ class FoveatedHandle:
     def __del__(self):
         h = getattr(self, "_h", None)
         if h is not None and h.value:
-            self._lib.fkv_attn_destroy(h)  # waits for the device: the blob is idle
             self._h = None
+            if _destroy(self._lib, h, self._blob) and _undestroyed:
+                _destroy_kept()
         self._blob = None
 
     def __call__(self, query, decode_k=None, decode_v=None, n_decode=None, out=None):

@@ -208,7 +208,8 @@ int fkv_turbo_create(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32_t 
  * fkv_attn_create_g32 (fmt 2) and fkv_turbo_create with the blob's device
  * memory given instead of allocated -- 256-byte aligned, at least
  * fkv_attn_blob_bytes of the same shape and format, and the caller's until
- * fkv_attn_destroy, which returns only when no work on the device uses it.
+ * fkv_attn_try_destroy returns FKV_OK: then no work on the device uses it
+ * (fkv_attn_destroy waits as well, but cannot while a stream captures).
  * For programs that keep device memory in a caching allocator: allocating and
  * freeing an 84 MB blob took about 400 us.  Synchronous, as those. */
 int64_t fkv_attn_blob_bytes(int32_t B, int32_t Hkv, int32_t D, int32_t Na, int32_t F, int32_t fmt);
@@ -415,6 +416,11 @@ int fkv_attn_blob_info(const fkv_attn* h, fkv_blob_info* out);
 int fkv_attn_read_near_valid(const fkv_attn* h, uint32_t* host_out, void* stream);
 
 void fkv_attn_destroy(fkv_attn* h);
+
+/* fkv_attn_destroy that says whether the device could be waited for: anything
+ * but FKV_OK (FKV_EHIP while a stream captures) leaves the handle and a
+ * caller's blob as they are, in use, for a later try. */
+int fkv_attn_try_destroy(fkv_attn* h);
 
 /* Decodes n (multiple of 4) E4M3 codes to fp16 with the converter the fused
  * kernel uses (gfx950 v_cvt_scalef32_pk_f16_fp8).  Replaces the reference's
