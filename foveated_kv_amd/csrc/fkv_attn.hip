@@ -897,20 +897,44 @@ static int env_int(const char* name, int dflt) {
     return v && *v ? atoi(v) : dflt;
 }
 
+static int plan_tiles(const BlobLayout& L, int n_dec) {
+    return (int)(cdiv(L.Na, kTile) + cdiv(L.F, kTile) + cdiv(n_dec, kTile));
+}
+
 // Workgroups per (b, kv_head, head group): as many as fit the target (the
-// CUs) in one round, at least two tiles per wave.  Rounded down: a workgroup
-// has a CU to itself, so the few past 256 of a launch rounded up start when
-// the others end and the chip runs two rounds for one (12 rows, 8,192-11,003
-// tokens: 22 splits = 264 workgroups 20.8-27.4 us, 21 = 252 14.9-19.3 us; 24
-// rows 21.6 against 14.8, 72 rows 38.1 against 26.3, 130 rows of 1 split
-// 46.8 us against 64.4 with 2; more rounds of shorter splits were slower too).
+// CUs) in one round, at least two tiles per wave.  Rounded down: where a
+// workgroup has a CU to itself, the few past 256 of a launch rounded up start
+// when the others end and the chip runs two rounds for one (D = 128, 12 rows,
+// 8,192-11,003 tokens: 22 splits = 264 workgroups 20.8-27.4 us, 21 = 252
+// 14.9-19.3 us; 24 rows 21.6 against 14.8, 72 rows 38.1 against 26.3, 130 rows
+// of 1 split 46.8 us against 64.4 with 2; never slower over 12-248 rows x
+// 1,024-16,384 tokens x every far format x 4 and 7 heads).
 static int plan_splits(const BlobLayout& L, int rows, int n_dec, int target, int waves = kWavesPerGroup) {
-    const int tiles = (int)(cdiv(L.Na, kTile) + cdiv(L.F, kTile) + cdiv(n_dec, kTile));
     int s = target / (rows > 0 ? rows : 1);
-    const int cap = tiles / (2 * waves);
+    const int cap = plan_tiles(L, n_dec) / (2 * waves);
     if (s > cap) s = cap;
     if (s > kMaxSplits) s = kMaxSplits;
     return s < 1 ? 1 : s;
+}
+
+// Whether a round is two workgroups per CU.  Two fit at D = 64 with one or
+// two head quads (137-183 VGPRs, 72-80 KB of LDS; nothing else does), and
+// the second one overlaps the first's chains: worth it for TurboQuant from
+// 20 rows on (below, a row's merge of more records outweighs it) and for two
+// quads that 256 workgroups split into at most 3; one quad of fp8 keys is
+// bound by memory, so there only where more than a fifth of the CUs would
+// stay idle.  Contexts under 32 tiles: one.  Measured with one / two per CU,
+// 16,384 tokens unless said, us: TurboQuant 7 heads, 172 rows 157.8 / 115.6,
+// 24 rows of 4 heads 22.0 / 15.8; fp8 7 heads, 132 rows 89.5 / 52.4, 72 rows
+// 37.0 / 30.4, 36 rows 22.5 / 21.0 (8,192: 16.2 / 16.4); fp8 4 heads, 132 rows
+// 62.8 / 47.3, 64 rows 23.6 / 24.5, 16 rows 12.5 / 14.7, 200 rows of 1,024
+// tokens 8.8 / 9.9.
+static bool two_workgroups_per_cu(const BlobLayout& L, int rows, int quads, int n_dec, int target) {
+    if (L.D != 64 || quads > 2) return false;
+    const int one = target / (rows > 0 ? rows : 1);
+    if (L.fmt == 1) return one <= 12;
+    if (plan_tiles(L, n_dec) < 32) return false;
+    return quads == 2 ? one <= 3 : one * rows * 5 < target * 4;
 }
 
 static size_t partial_floats(int rows, int splits, int ng_max, int D) {
@@ -931,8 +955,10 @@ LaunchPlan plan_launch(const BlobLayout& L, int Hq, int n_decode, int target_wgs
     p.head_groups = (int)cdiv(G, hpg);
     p.ng_max = G < hpg ? G : hpg;
     p.rows = L.B * L.Hkv * p.head_groups;
-    p.waves = attn_waves(L.D, (int)cdiv(p.ng_max, 4), L.fmt);
-    p.splits = plan_splits(L, p.rows, n_decode, target_wgs, p.waves);
+    const int quads = (int)cdiv(p.ng_max, 4);
+    p.waves = attn_waves(L.D, quads, L.fmt);
+    const int round = two_workgroups_per_cu(L, p.rows, quads, n_decode, target_wgs) ? 2 * target_wgs : target_wgs;
+    p.splits = plan_splits(L, p.rows, n_decode, round, p.waves);
     // rows of 2..4 splits keep one record per wave (their merge reads at most
     // 16 records, 32 for 8-wave TurboQuant rows: within kMaxSplits); rows of
     // more splits merge their waves in LDS first (C4's 8 splits: 32 wave

@@ -247,3 +247,30 @@ def test_launch_plan_is_one_round_of_the_chip(fmt):
                     assert splits >= 1 and (rows * splits <= 256 or splits == 1), (B, Hkv, G, S, rows, splits)
                     # and no CU is left out that one more split per row would fill
                     assert (splits + 1) * rows > 256 or splits == 64 or splits >= (S // 7 // 64 + S // 64) // 16
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+def test_launch_plan_where_two_workgroups_share_a_cu(fmt):
+    """At D = 64 the kernels of one or two head quads (G <= 8) fit a CU twice:
+    rows that leave CUs idle with a workgroup each are split for two, within
+    one round of those; wider rows and short contexts keep one."""
+    from foveated_kv_amd import _lib
+
+    lib = _lib.load()
+    out = (ctypes.c_int64 * 8)()
+
+    def splits(B, Hkv, G, S):
+        assert lib.fkv_attn_plan(B, Hkv, 64, S // 7, S, Hkv * G, 0, 256, fmt, out) == _lib.FKV_OK
+        return int(out[1]), int(out[2])
+
+    for B, Hkv in ((33, 4), (43, 4), (25, 8), (31, 8), (12, 2), (9, 4), (18, 4), (64, 8), (65, 8)):
+        for G in (1, 4, 5, 8, 12, 16):
+            for S in (600, 2048, 11003, 65536):
+                rows, s = splits(B, Hkv, G, S)
+                assert s >= 1 and (rows * s <= (512 if G <= 8 else 256) or s == 1), (B, Hkv, G, S, rows, s)
+    assert splits(33, 4, 7, 16384) == (132, 3) and splits(43, 4, 4, 16384) == (172, 2)  # not one split of 256
+    assert splits(33, 4, 12, 16384) == (132, 1)                                         # three quads: one per CU
+    assert splits(31, 8, 4, 16384) == (248, 2 if fmt == 1 else 1)                       # one quad, few CUs idle
+    assert splits(31, 8, 7, 16384) == (248, 2) and splits(32, 8, 4, 16384) == (256, 2 if fmt == 1 else 1)
+    assert splits(33, 4, 4, 1024) == (132, 2 if fmt == 1 else 1)                        # short
+    assert splits(18, 4, 7, 16384) == (72, 7) and splits(8, 2, 4, 16384) == (16, 16)
