@@ -192,7 +192,7 @@ struct LaunchPlan {
     int wave_recs;  // split records per split (waves: one per wave, 1: merged in LDS)
     size_t ws_floats;
 };
-LaunchPlan plan_launch(const BlobLayout& L, int Hq, int n_decode, int target_wgs);
+LaunchPlan plan_launch(const BlobLayout& L, int Hq, int n_decode, int target_wgs, bool round_up = false);
 // The workspace a handle's first call allocates for Hq query heads: enough
 // for every launch plan of that head count (any decode length).
 size_t workspace_floats(const BlobLayout& L, int Hq);

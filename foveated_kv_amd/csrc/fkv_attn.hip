@@ -945,7 +945,8 @@ static size_t partial_floats(int rows, int splits, int ng_max, int D) {
 // every compressed byte crosses HBM once -- unless that leaves most CUs idle
 // (few batch x KV-head rows, short context): then rows of 4 heads, more
 // workgroups re-reading the same small KV from L2.
-LaunchPlan plan_launch(const BlobLayout& L, int Hq, int n_decode, int target_wgs) {
+// round_up: the next split count above one round of the chip.
+LaunchPlan plan_launch(const BlobLayout& L, int Hq, int n_decode, int target_wgs, bool round_up) {
     const int G = Hq / L.Hkv;
     int hpg = kHeads;
     const int rows16 = L.B * L.Hkv * (int)cdiv(G, kHeads);
@@ -957,7 +958,8 @@ LaunchPlan plan_launch(const BlobLayout& L, int Hq, int n_decode, int target_wgs
     p.rows = L.B * L.Hkv * p.head_groups;
     const int quads = (int)cdiv(p.ng_max, 4);
     p.waves = attn_waves(L.D, quads, L.fmt);
-    const int round = two_workgroups_per_cu(L, p.rows, quads, n_decode, target_wgs) ? 2 * target_wgs : target_wgs;
+    int round = two_workgroups_per_cu(L, p.rows, quads, n_decode, target_wgs) ? 2 * target_wgs : target_wgs;
+    if (round_up) round = (int)cdiv(target_wgs, p.rows) * p.rows;
     p.splits = plan_splits(L, p.rows, n_decode, round, p.waves);
     // rows of 2..4 splits keep one record per wave (their merge reads at most
     // 16 records, 32 for 8-wave TurboQuant rows: within kMaxSplits); rows of
@@ -1175,6 +1177,12 @@ constexpr int kScratchRows = 16384;  // rows the counter region serves
 // arrival counters [rows], then the XCD watch words [1 + rows]
 constexpr size_t kScratchArriveBytes = ((size_t)(2 * kScratchRows + 1) * 4 + 255) & ~(size_t)255;
 constexpr int kScratchDevices = 64;
+size_t scratch_query_bytes(const fkv::BlobLayout& L, int Hq) {
+    return ((size_t)L.B * Hq * L.D * 2 + 255) & ~(size_t)255;
+}
+size_t scratch_need(const fkv::BlobLayout& L, const fkv::LaunchPlan& p, int Hq) {
+    return kScratchArriveBytes + scratch_query_bytes(L, Hq) + p.ws_floats * sizeof(float);
+}
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
 namespace {
@@ -1341,9 +1349,16 @@ int attn_call(const char* fn, fkv_attn* h, const void* query, int32_t q_dtype, i
         return set_error(name + ": spike_k > 1 needs the selection buffers of a call with Hq=" + std::to_string(Hq) +
                          " (fkv_attn_call once, or fkv_attn_set_spike_k after one)");
     // the split count follows the longest decode length the call can see
-    const fkv::LaunchPlan p = fkv::plan_launch(L, Hq, n_dec_dev ? dec_stride : n_decode, h->target_wgs);
+    const int n_plan = n_dec_dev ? dec_stride : n_decode;
+    fkv::LaunchPlan p = fkv::plan_launch(L, Hq, n_plan, h->target_wgs);
     CallWorkspace w;
     if (no_alloc) {
+        // a record per wave of 4 splits (16-head rows at D = 128) can be more
+        // than the scratch holds where 5 merged splits fit it
+        if (scratch_need(L, p, Hq) > kScratchBytes) {
+            const fkv::LaunchPlan up = fkv::plan_launch(L, Hq, n_plan, h->target_wgs, true);
+            if (scratch_need(L, up, Hq) <= kScratchBytes) p = up;
+        }
         if (int rc = scratch_workspace(name, h, p, Hq, st, &w)) return rc;
     } else {
         if (int rc = ensure_workspace(name, h, Hq, st)) return rc;
@@ -1505,8 +1520,7 @@ int attn_call(const char* fn, fkv_attn* h, const void* query, int32_t q_dtype, i
 int scratch_workspace(const std::string& name, fkv_attn* h, const fkv::LaunchPlan& p, int Hq, hipStream_t st,
                       CallWorkspace* out) {
     const fkv::BlobLayout& L = h->L;
-    const size_t qbytes = ((size_t)L.B * Hq * L.D * 2 + 255) & ~(size_t)255;
-    const size_t need = kScratchArriveBytes + qbytes + p.ws_floats * sizeof(float);
+    const size_t qbytes = scratch_query_bytes(L, Hq), need = scratch_need(L, p, Hq);
     if (p.rows > kScratchRows || need > kScratchBytes)
         return set_error(name + ": this call needs " + std::to_string(need) + " bytes of scratch (" +
                          std::to_string(p.rows) + " rows x " + std::to_string(p.splits) +

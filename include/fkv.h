@@ -279,12 +279,14 @@ int fkv_attn_call_strided(fkv_attn* h, const void* query, int32_t q_dtype, int32
  * call's split records, arrival counters and fp16 query copy live in one
  * fixed 8 MiB device array per GPU instead of the handle's workspace, so
  * neither this call nor its first use allocates or frees anything.  Calls
- * whose launch plan needs more than the array holds (64 KiB of arrival
- * counters for at most 16384 rows, then the fp16 query copy, then rows x
- * splits x records per split x heads per row x (8 + D) floats of split
- * records, fkv_attn_plan out[1] x out[2] x out[7] x min(out[0], G); C3 at
- * batch 8 needs 2.25 MiB: 64 rows x 4 splits x 4 wave records x 4 heads x
- * 136 floats, C5 1.14 MiB) return FKV_EINVAL, as does a call whose handle's
+ * whose launch plan needs more than the array holds (128 KiB of arrival
+ * counters and watch words for at most 16384 rows, then the fp16 query copy,
+ * then rows x splits x records per split x heads per row x (8 + D) floats of
+ * split records, fkv_attn_plan out[1] x out[2] x out[7] x min(out[0], G); C3
+ * at batch 8 needs 2.25 MiB: 64 rows x 4 splits x 4 wave records x 4 heads x
+ * 136 floats, C5 1.14 MiB) take the next larger split count where its merged
+ * records fit (rows of 16 heads at D = 128: 58 to 63 rows), or return
+ * FKV_EINVAL, as does a call whose handle's
  * device is not current, or, with spike_k > 1, a handle whose top-K
  * selection buffers do not exist yet (fkv_attn_set_spike_k).  Every call on
  * one GPU shares that GPU's array: calls that overlap on one GPU (two

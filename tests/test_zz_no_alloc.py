@@ -156,3 +156,29 @@ def test_noalloc_refuses_a_plan_beyond_its_scratch():
                                    _lib.ptr(fl), _lib.stream_ptr())
     assert rc == _lib.FKV_EINVAL
     assert b"no-alloc entry point holds" in lib.fkv_last_error()
+
+
+@pytest.mark.parametrize("B,G", [(59, 16), (63, 16), (63, 15), (58, 16), (57, 16)])
+def test_noalloc_takes_rows_whose_wave_records_exceed_its_scratch(orc, B, G):
+    """Rows of 15 or 16 heads at D = 128 in 4 splits keep a record per wave,
+    which the array does not hold from 58 rows on; 5 splits merge theirs and
+    fit (57 rows: the call's own plan fits)."""
+    from foveated_kv_amd import _lib
+
+    flush(f"no-alloc {B} rows of {G} heads")
+    h, q, dk, dv, c = _case(B, G, 1, 128, 3000, 3, seed=B + G)
+    plan = (ctypes.c_int64 * 8)()
+    assert _lib.load().fkv_attn_plan(B, 1, 128, h.N_near, h.N_far, G, 3, 256, 0, plan) == 0
+    assert plan[1] == B and plan[2] == 4 and plan[7] == 4
+    assert (B == 57) == (131328 + B * G * 256 + plan[3] * 4 <= 8 << 20)
+    qt = torch.from_numpy(q).cuda()
+    dkt, dvt = torch.from_numpy(dk).cuda(), torch.from_numpy(dv).cuda()
+    got = _call("fkv_attn_call_noalloc", h, qt, dkt, dvt)
+    want = _call("fkv_attn_call", h, qt, dkt, dvt)
+    torch.cuda.synchronize()
+    ko = orc.attend_kernel(q, c["near_k"], c["near_v"], c["near_valid"], c["far_k"], c["far_v"],
+                           c["far_v_scale"], c["far_v_zero"], dk, dv, spike_margin=10.0)[0]
+    for res in (got, want):
+        out = np_(res[0]).astype(np.float64)
+        assert float(np.abs(out - ko).max()) <= ATOL and orc.cosine(out, ko) >= COS
+    assert B != 57 or all(torch.equal(a, b) for a, b in zip(got, want))
