@@ -348,7 +348,9 @@ class FoveatedHandle:
         h = getattr(self, "_h", None)
         if h is not None and h.value:
             self._h = None
-            if _destroy(self._lib, h, self._blob) and _undestroyed:
+            if _destroy is None:  # the interpreter exits and this module's names are gone
+                self._lib.fkv_attn_destroy(h)
+            elif _destroy(self._lib, h, self._blob) and _undestroyed:
                 _destroy_kept()
         self._blob = None
 

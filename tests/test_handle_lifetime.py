@@ -84,6 +84,26 @@ def test_new_handle_destroys_the_kept_ones(capturing):
     assert lib.destroyed == [21] and not ext._undestroyed
 
 
+def test_handle_alive_at_exit():
+    """Destroyed without a message when the interpreter clears its modules."""
+    import subprocess
+    import sys
+
+    code = """
+import ctypes, os, torch
+from foveated_kv_amd import ext
+class Library:
+    def fkv_attn_destroy(self, h, write=os.write):
+        write(1, b"destroyed")
+    fkv_attn_try_destroy = fkv_attn_destroy
+h = ext.FoveatedHandle.__new__(ext.FoveatedHandle)
+h._lib, h._h, h._blob = Library(), ctypes.c_void_p(5), None
+torch.kept_for_the_test = h  # outlives the names of ext
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout == "destroyed" and "Exception ignored" not in r.stderr
+
+
 @pytest.mark.gpu
 def test_handle_dropped_during_a_capture():
     """Replays of the handle's calls are in flight on another stream when it
