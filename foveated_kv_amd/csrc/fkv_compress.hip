@@ -827,12 +827,12 @@ extern "C" int fkv_tier_index_rows(const fkv_tiers* tiers, int32_t B, int32_t H,
     using fkv::set_error;
     if (!tiers) return set_error("fkv_tier_index_rows: tiers is NULL");
     const fkv_tiers tb = *tiers;
-    if (B <= 0 || H <= 0 || S < 0 || tb.n_near_padded < 0 || tb.far_count < 0)
+    if (B < 0 || H < 0 || S < 0 || tb.n_near_padded < 0 || tb.far_count < 0)
         return set_error("fkv_tier_index_rows: bad shape");
-    if ((tb.n_near_padded > 0 && !near_idx) || (tb.far_count > 0 && !far_idx))
-        return set_error("fkv_tier_index_rows: NULL argument");
     const int64_t n = (int64_t)B * H * ((int64_t)tb.n_near_padded + tb.far_count);
     if (n == 0) return FKV_OK;
+    if ((tb.n_near_padded > 0 && !near_idx) || (tb.far_count > 0 && !far_idx))
+        return set_error("fkv_tier_index_rows: NULL argument");
     const int64_t blocks = fkv::cdiv(n, 256);
     hipLaunchKernelGGL(fkv::tier_index_kernel, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0,
                        (hipStream_t)stream, tb, S, (int64_t)B * H, near_idx, far_idx);

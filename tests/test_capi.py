@@ -274,3 +274,16 @@ def test_launch_plan_where_two_workgroups_share_a_cu(fmt):
     assert splits(31, 8, 7, 16384) == (248, 2) and splits(32, 8, 4, 16384) == (256, 2 if fmt == 1 else 1)
     assert splits(33, 4, 4, 1024) == (132, 2 if fmt == 1 else 1)                        # short
     assert splits(18, 4, 7, 16384) == (72, 7) and splits(8, 2, 4, 16384) == (16, 16)
+
+
+def test_tier_index_rows_of_no_rows():
+    """An empty batch or no heads: nothing to write, as for any empty tensor
+    (whose pointer is NULL); a negative count is refused."""
+    from foveated_kv_amd import _lib, ext
+
+    lib = _lib.load()
+    cfg = ext.TierConfig().to_c()
+    tb = _lib.TiersC()
+    assert lib.fkv_tier_boundaries(ctypes.byref(cfg), 500, ctypes.byref(tb)) == _lib.FKV_OK
+    for B, H, want in ((0, 3, _lib.FKV_OK), (2, 0, _lib.FKV_OK), (-1, 3, _lib.FKV_EINVAL), (2, 3, _lib.FKV_EINVAL)):
+        assert lib.fkv_tier_index_rows(ctypes.byref(tb), B, H, 500, None, None, None) == want
