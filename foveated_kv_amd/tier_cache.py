@@ -202,17 +202,18 @@ class FoveatedLayer:
     far_k_scale: Optional[torch.Tensor] = None  # (B,H) fp32: per-head-scaled fp8 keys
     spike_k: int = 1  # spiking far tokens per query head the fused kernel reports
     # position of the next token (None: one past the largest index, which
-    # reads both index tensors back)
+    # reads both index tensors back); an argument only, so that a copy with
+    # other index tensors does not take this layer's
     next_position: Optional[int] = field(default=None, repr=False)
 
     def __post_init__(self):
-        if self.next_position is None:
+        self._next_pos, self.next_position = self.next_position, None
+        if self._next_pos is None:
             max_pos = -1
             for t in (self.near_idx, self.far_idx):
                 if t.numel() > 0:
                     max_pos = max(max_pos, int(t.max().item()))
-            self.next_position = max_pos + 1
-        self._next_pos = self.next_position
+            self._next_pos = max_pos + 1
         self._decode = _DecodeBuffer()
         if self.near_valid is None:
             self.near_valid = torch.full((self.near_k.shape[1],), self.near_k.shape[2],
