@@ -169,6 +169,7 @@ class CompressHandle:
             if importance is not None:
                 near_idx, far_idx = partition_importance(self.cfg, importance, B, H, S)
             if not far:
+                c.k_scale = 0  # no far keys to scale
                 check(lib.fkv_archive_layer(
                     ctypes.byref(c), ptr(k), ptr(v), dtype_code(k.dtype), B, H, S, D, ptr(near_idx), ptr(far_idx),
                     ptr(near_k), ptr(near_v), ptr(near_valid), ptr(arc_k), ptr(arc_v), _lib.stream_ptr(dev)),

@@ -550,3 +550,22 @@ def test_turbo_keys_refused_under_capture(fkv):
             turbo_compress_keys(k, tc)
     want = turbo_compress_keys(k, tc)
     assert all(torch.equal(a, b) for a, b in zip(turbo_compress_keys(k, tc), want))
+
+
+def test_archive_layer_ignores_the_key_scale_option(fkv):
+    """It has no far keys to scale: a configuration with k_scale set (by hand,
+    on a TurboQuant one) gives the layer that one without it does."""
+    from foveated_kv_amd import FoveatedKVCache, TierConfig
+
+    k, v = (torch.randn((1, 2, 300, 64), device="cuda").half() for _ in range(2))
+    layers = []
+    for k_scale in (False, True):
+        cfg = TierConfig(compress_method="turbo")
+        cfg.k_scale = k_scale
+        cache = FoveatedKVCache(cfg)
+        cache.update(k, v, 0)
+        cache.compress()
+        layers.append(cache.layers[0])
+    for n in ("near_k", "near_v", "near_valid", "archive_k", "archive_v", "turbo_far_k_indices", "turbo_far_k_signs",
+              "turbo_far_v_packed"):
+        assert torch.equal(getattr(layers[0], n), getattr(layers[1], n)), n
