@@ -26,13 +26,21 @@ namespace fkv {
 // (v_mfma_f32_32x32x16_f16) at fp32 precision: every fp32 operand is split
 // into fp16 hi + lo after a power-of-two scale that puts its row's (token's)
 // largest value near 1,024 (256), so that lo keeps its 11 bits above fp16's
-// subnormals; the keys are fp16 already, products of fp16 values are exact
-// and summed in fp32, and the lo products run first, while the sums are
-// small (lo x lo, below 2^-24, is left out).  A token with a rotated
-// coordinate that close to a boundary (1 in 6,000) takes its codes from
-// 64-bit sums.  Against 64 bits over N(0, 1) keys with outlier channels, 20 x
-// 262,112 tokens: no code and 62 signs off of 6.7e8 at D = 128 (59 and 121
-// with fp32 FMA chains), none and 36 of 3.4e8 at D = 64 (18 and 48).
+// subnormals: 22 bits of an element down to 2^-13 of its row's largest, an
+// absolute 2^-35 of that below.  The keys are fp16 already; products of fp16
+// values are exact and summed in fp32, and the lo products run first, while
+// the sums are small.  lo x lo, at most 2^-22 of the product of its elements,
+// is left out of the second and third product.  Fewer bits per operand than
+// the fp32 FMA chains had, but a smaller error of a product: rms, over the
+// norms of the vector and the row, 8.1e-9 against the chains' 1.8e-8 at D =
+// 128, 1.1e-8 against 1.8e-8 at D = 64 (both modelled on the CPU).  A token
+// with a rotated coordinate within 6e-8 of its norm of a boundary (1 in
+// 6,000) takes its codes from 64-bit sums: twelve standard deviations of the
+// error measured with the orthonormal Pi and the boundaries of
+// get_turbo_constants; no bound, and not scaled for other matrices.  Against
+// 64 bits over N(0, 1) keys with outlier channels, 20 x 262,112 tokens: no
+// code and 62 signs off of 6.7e8 at D = 128 (59 and 121 with fp32 FMA
+// chains), none and 36 of 3.4e8 at D = 64 (18 and 48).
 // The matrix is the A operand (rows = output dims) and the tokens are the B
 // operand (columns), so a lane's accumulators hold its own token's output
 // dims 32 rb + 8 a + 4 (lane / 32) + b; every product's K slots are numbered
@@ -379,7 +387,7 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
         w[rb] = ~w[rb];  // the codes
     }
     // tokens with a coordinate within twelve standard deviations of the sums'
-    // error (5e-9 of the norm) take their codes from 64-bit sums
+    // error (5e-9 of the norm for an orthonormal Pi) take their codes from 64-bit sums
     const uint64_t close = __ballot(live && nrm > 0.f && nrm < INFINITY && gap < 6e-8f * nrm);
     const bool odd_norm = !(nrm < INFINITY);
     uint32_t redo = (uint32_t)close | (uint32_t)(close >> 32);

@@ -227,11 +227,14 @@ int fkv_turbo_create_at(fkv_attn** out, int32_t B, int32_t Hkv, int32_t D, int32
 /* TurboQuant compression on the GPU (src/foveated_kv/turbo_quantize.py:
  * 25-91): keys (n_tokens, D) in dtype -> out_idx (n_tokens, D/4) u8,
  * out_signs (n_tokens, D/8) u8, out_norm / out_gamma (n_tokens) fp16;
- * Pi, S (D,D), centroids (4), boundaries (3) fp32 device arrays.  fp32
- * precision (codes near a boundary from 64-bit sums); a sign whose projection
- * lies within rounding of 0 can
- * differ from another fp32 evaluation order.  Asynchronous; refused under
- * graph capture (it allocates a workspace). */
+ * Pi, S (D,D), centroids (4), boundaries (3) fp32 device arrays, finite
+ * (boundaries may be infinite).  fp32 precision relative to the largest
+ * element of a matrix row: a sign whose projection lies within rounding of 0
+ * can differ from another fp32 evaluation order, and so can a code whose
+ * coordinate lies within rounding of a boundary, except for an orthonormal Pi
+ * and boundaries below about 0.13 (the library's constants), where a
+ * coordinate within 6e-8 of the norm of a boundary is decided by 64-bit sums.
+ * Asynchronous; refused under graph capture (it allocates a workspace). */
 int fkv_turbo_compress_keys(const void* keys, int32_t dtype, int64_t n_tokens, int32_t D, const float* Pi,
                             const float* S, const float* centroids, const float* boundaries, uint8_t* out_idx,
                             uint8_t* out_signs, void* out_norm, void* out_gamma, void* stream);

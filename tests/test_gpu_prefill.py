@@ -516,9 +516,10 @@ def test_archive_layer_is_the_compress_layer_without_far_codes(fkv, importance, 
 
 @pytest.mark.parametrize("D,dt", [(64, torch.float16), (128, torch.float16), (128, torch.float32)])
 def test_turbo_codes_are_the_64_bit_ones(fkv, D, dt):
-    """Coordinates near a boundary are decided by 64-bit sums: over 200,000
-    tokens (about 30 of them near one; with zero and padded ones) every code
-    is the one that fp64 gives."""
+    """Over 200,000 random tokens (with zero and padded ones) every code is the
+    one that fp64 gives.  About 30 of them lie near a boundary, of which plain
+    fp32 sums would miss one or two: the 64-bit decision itself is held by
+    test_turbo_codes_next_to_a_boundary."""
     from foveated_kv_amd.turbo import get_turbo_constants, turbo_compress_keys
 
     g = torch.Generator(device="cuda").manual_seed(D)
@@ -569,3 +570,69 @@ def test_archive_layer_ignores_the_key_scale_option(fkv):
     for n in ("near_k", "near_v", "near_valid", "archive_k", "archive_v", "turbo_far_k_indices", "turbo_far_k_signs",
               "turbo_far_v_packed"):
         assert torch.equal(getattr(layers[0], n), getattr(layers[1], n)), n
+
+
+def _keys_near_a_boundary(tc, rng):
+    """fp16 keys, one for every dim, boundary and side, whose rotated
+    coordinate lies 1e-9 to 3e-8 of their norm from the boundary in fp64:
+    random keys moved along the dim's row of Pi, then the nearest of 16^4
+    combinations of steps of four of their elements."""
+    Pi, bd = tc.Pi.numpy().astype(np.float64), tc.boundaries.numpy().astype(np.float64)
+    D = Pi.shape[0]
+    grid = np.arange(-8.0, 8.0)
+    out = []
+    for i in range(D):
+        for b in bd:
+            for side in (-1.0, 1.0):
+                k = rng.standard_normal(D)
+                k[:4] *= 8
+                for _ in range(4):
+                    k = k + (b * np.linalg.norm(k) - k @ Pi[i]) * Pi[i]
+                k = k.astype(np.float16).astype(np.float64)
+                # elements well inside their binade: eight steps stay fp16 numbers
+                m, e = np.frexp(np.abs(k))
+                dims = rng.permutation(np.flatnonzero((m > 0.55) & (m < 0.95) & (np.abs(k) > 0.1)))[:4]
+                dot, sq = k @ Pi[i], k @ k
+                for a, d in enumerate(dims):
+                    shape = [1] * 4
+                    shape[a] = 16
+                    s = (grid * 2.0 ** (e[d] - 11.0)).reshape(shape)
+                    dot = dot + s * Pi[i, d]
+                    sq = sq + s * (2 * k[d] + s)
+                off = side * (dot / np.sqrt(sq) - b)
+                at = np.unravel_index(np.argmin(np.where(off >= 1e-9, off, np.inf)), off.shape)
+                for a, d in enumerate(dims):
+                    k[d] += grid[at[a]] * 2.0 ** (e[d] - 11.0)
+                h = k.astype(np.float16)
+                assert np.array_equal(h.astype(np.float64), k)
+                gap = side * (k @ Pi[i] / np.linalg.norm(k) - b)
+                if 1e-9 <= gap <= 3e-8:
+                    out.append(h)
+    return np.stack(out)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_turbo_codes_next_to_a_boundary(fkv, D):
+    """Keys with a coordinate closer to a boundary than the fp32-precision
+    sums decide (their error has a standard deviation of about 5e-9 of the
+    norm): every code is the one of fp64.  Waves of such keys only, and waves
+    that hold some among others."""
+    from foveated_kv_amd import _lib
+    from foveated_kv_amd.turbo import get_turbo_constants
+
+    rng = np.random.default_rng(D)
+    tc = get_turbo_constants(D)
+    near = _keys_near_a_boundary(tc, rng)
+    assert len(near) > 5 * D  # of 6 D
+    other = rng.standard_normal((3 * len(near), D)).astype(np.float16)
+    mixed = np.concatenate([near, other])
+    rng.shuffle(mixed)
+    k = np.concatenate([near, mixed])
+    flush(f"turbo codes next to a boundary D={D} keys={len(near)}")
+    args = [t.numpy() for t in (tc.Pi, tc.S, tc.centroids, tc.boundaries)]
+    got = _turbo_keys(_lib, torch.from_numpy(k).cuda(), *args)
+    kd = k.astype(np.float64)
+    y = (kd @ args[0].astype(np.float64).T) / np.linalg.norm(kd, axis=-1, keepdims=True)
+    want = (y[..., None] >= args[3].astype(np.float64)).sum(-1)
+    assert int((_unpack(got[0].cpu().numpy(), 2) != want).sum()) == 0
+    _check_turbo_keys(k, *args, got)
