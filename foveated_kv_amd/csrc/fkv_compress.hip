@@ -363,10 +363,10 @@ constexpr int kPartRegs = 64;  // most tokens per thread held in registers
 constexpr int kPartBits = 11, kPartBins = 1 << kPartBits, kPartCopies = 4;
 
 // Partition of a (batch, head) whose middle fits the workgroup's registers,
-// R tokens per thread (at most kPartThreads * R in all).  Bound by one CU's
+// q of R tokens per thread (the fewest that hold it).  Bound by one CU's
 // vector instructions, not by memory, so the row is read once and as little
 // as possible is done per token: wave w holds order_key of the middle's
-// tokens w * R * 64 .. in position order (register r: 64 consecutive
+// tokens w * q * 64 .. in position order (register r: 64 consecutive
 // tokens).  A radix select of 11 + 11 + 10 bits over the registers (LDS
 // histograms, one per wave modulo kPartCopies; one per lane modulo 16, free
 // of bank conflicts, was no faster) finds the near_from_mid-th largest key v
@@ -374,13 +374,17 @@ constexpr int kPartBits = 11, kPartBins = 1 << kPartBits, kPartCopies = 4;
 // order: the later token wins a tie, which is what the 64-bit rank key
 // orders by).  The compaction needs no block step per chunk: a token's far
 // row is its position less the near tokens before it, and those follow from
-// one scan of the waves' counts and ballots.  Registers past the middle hold
-// the lowest key: they come after every token in position order, so they
-// only take part in a tie at that key, where they are counted out, and their
-// places lie past the near and far rows (a range test per token and pass
-// made half of the instructions).  64K tokens x 8 heads: 190 us with 8-bit
-// passes that each re-read the row and a block scan per 1,024 tokens, 53 us
-// with the range tests (and their lane masks spilled), 40 us here.
+// one scan of the waves' counts and ballots.  Registers from q on take no
+// part (a test of a scalar): as padding their histogram adds all met in one
+// bin (16,385 tokens in 64 registers per thread 73 us; 53 with the 8-bit
+// passes below, 22 with q; 32,768 tokens 61, 97 and 24).  The fewer than 1,024 places past the middle in
+// the others hold the lowest key: they come after every token in position
+// order, so they only take part in a tie at that key, where they are counted
+// out, and their places lie past the near and far rows (a range test per
+// token and pass made half of the instructions).  64K tokens x 8 heads: 190
+// us with 8-bit passes that each re-read the row and a block scan per 1,024
+// tokens, 53 us with the range tests (and their lane masks spilled), 40 us
+// here.
 template <int R>
 __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const float* __restrict__ imp, int S,
                                                                      fkv_tiers tb, int32_t* __restrict__ near_idx,
@@ -403,16 +407,28 @@ __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const floa
         }
         return;
     }
-    const int i0 = wave * R * kWave + lane;  // the lane's first token of the middle
+    constexpr int C = R < 16 ? 1 : 4;  // registers per test of q
+    const int q = (mlen + C * kPartThreads - 1) / (C * kPartThreads) * C;  // at most R
+    // whether chunk c's registers are in use (tested anew each time: kept, the
+    // results of all chunks would be spilled)
+    auto used = [&](int c) {
+        int qc = q;
+        asm volatile("" : "+s"(qc));
+        return c < qc;
+    };
+    const int i0 = wave * q * kWave + lane;  // the lane's first token of the middle
     const float* row = imp + (int64_t)bh * S + m0;
     uint32_t key[R];
     {
-        float f[R];
+        float f[R] = {};
 #pragma unroll
-        for (int r = 0; r < R; r++) f[r] = row[min(i0 + r * kWave, mlen - 1)];
+        for (int c = 0; c < R; c += C)
+            if (used(c))
+#pragma unroll
+                for (int r = c; r < c + C; r++) f[r] = row[min(i0 + r * kWave, mlen - 1)];
 #pragma unroll
         for (int r = 0; r < R; r++) key[r] = order_key(f[r]);
-        if ((wave + 1) * R * kWave > mlen)
+        if ((wave + 1) * q * kWave > mlen)
 #pragma unroll
             for (int r = 0; r < R; r++)
                 if (i0 + r * kWave >= mlen) key[r] = 0;
@@ -426,10 +442,14 @@ __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const floa
         __syncthreads();
         uint32_t* const h = hist[wave % kPartCopies];
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            PART_PIN(key[r]);
-            if (p == 0 || (key[r] ^ v) >> (shift[p] + bits[p]) == 0)  // the digits already known
-                atomicAdd(&h[(key[r] >> shift[p]) & ((1u << bits[p]) - 1)], 1u);
+        for (int c = 0; c < R; c += C) {
+            if (!used(c)) break;
+#pragma unroll
+            for (int r = c; r < c + C; r++) {
+                PART_PIN(key[r]);
+                if (p == 0 || (key[r] ^ v) >> (shift[p] + bits[p]) == 0)  // the digits already known
+                    atomicAdd(&h[(key[r] >> shift[p]) & ((1u << bits[p]) - 1)], 1u);
+            }
         }
         __syncthreads();
         // thread t takes bins top - 2t and top - 2t - 1: an inclusive scan
@@ -466,21 +486,25 @@ __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const floa
         v |= (uint32_t)__builtin_amdgcn_readfirstlane((int)s_bin) << shift[p];
         rem = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_rem);
     }
-    // tokens equal to v that stay far (the registers past the middle are not tokens)
-    const uint32_t equal_far = s_cnt - (v == 0 ? (uint32_t)(kPartThreads * R - mlen) : 0u) - rem;
+    // tokens equal to v that stay far (the places past the middle are not tokens)
+    const uint32_t equal_far = s_cnt - (v == 0 ? (uint32_t)(kPartThreads * q - mlen) : 0u) - rem;
     // lane r: which of register r's tokens lie above v (near) and at v
     static_assert(R <= kWave, "a lane per register");
     uint32_t nlo = 0, nhi = 0, elo = 0, ehi = 0;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        PART_PIN(key[r]);
-        const uint64_t g = __ballot(key[r] > v), e = __ballot(key[r] == v);
-        // (a select per lane would need R lane masks; the wait states are those
-        // of a scalar register written by a compare and read here)
-        asm volatile("s_nop 1\n\tv_writelane_b32 %0, %4, %8\n\tv_writelane_b32 %1, %5, %8\n\t"
-                     "v_writelane_b32 %2, %6, %8\n\tv_writelane_b32 %3, %7, %8"
-                     : "+v"(nlo), "+v"(nhi), "+v"(elo), "+v"(ehi)
-                     : "s"((uint32_t)g), "s"((uint32_t)(g >> 32)), "s"((uint32_t)e), "s"((uint32_t)(e >> 32)), "n"(r));
+    for (int c = 0; c < R; c += C) {
+        if (!used(c)) break;
+#pragma unroll
+        for (int r = c; r < c + C; r++) {
+            PART_PIN(key[r]);
+            const uint64_t g = __ballot(key[r] > v), e = __ballot(key[r] == v);
+            // (a select per lane would need R lane masks; the wait states are those
+            // of a scalar register written by a compare and read here)
+            asm volatile("s_nop 1\n\tv_writelane_b32 %0, %4, %8\n\tv_writelane_b32 %1, %5, %8\n\t"
+                         "v_writelane_b32 %2, %6, %8\n\tv_writelane_b32 %3, %7, %8"
+                         : "+v"(nlo), "+v"(nhi), "+v"(elo), "+v"(ehi)
+                         : "s"((uint32_t)g), "s"((uint32_t)(g >> 32)), "s"((uint32_t)e), "s"((uint32_t)(e >> 32)), "n"(r));
+        }
     }
     // inclusive sums over the wave's registers
     auto lane_scan = [&](uint32_t x) {
@@ -516,7 +540,7 @@ __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const floa
     const uint32_t upto = near_before + lane_scan(__popcll(near)), first = upto - __popcll(near);
     nrow += tb.n_sinks;
 #pragma unroll 4
-    for (int r = 0; r < R; r++) {
+    for (int r = 0; r < q; r++) {
         const uint32_t lo = __builtin_amdgcn_readlane(nlo, r), hi = __builtin_amdgcn_readlane(nhi, r);
         const int before = (int)__builtin_amdgcn_readlane(first, r) +
                            (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
@@ -534,7 +558,8 @@ __global__ __launch_bounds__(kPartThreads) void partition_regs_kernel(const floa
 // then the middle is compacted in position order into near slots
 // n_sinks.. and far slots 0.. with a block-wide scan per 1024-token chunk.
 // For middles of more than kPartThreads * kPartRegs tokens, which do not fit
-// partition_regs_kernel's registers.
+// partition_regs_kernel's registers: eight passes over the row (8 heads: 181
+// us for 65,537 tokens where 65,536 in registers take 38; 350 us for 131,072).
 __global__ __launch_bounds__(kPartThreads) void partition_kernel(const float* __restrict__ imp, int S, fkv_tiers tb,
                                                                 int32_t* __restrict__ near_idx,
                                                                 int32_t* __restrict__ far_idx) {
@@ -811,7 +836,7 @@ extern "C" int fkv_partition_importance(const fkv_tier_config* cfg, const float*
     if ((S > 0 && !importance) || !near_idx || (tb.far_count > 0 && !far_idx))
         return set_error("fkv_partition_importance: NULL argument");
     // tokens per thread: the smallest compiled count that holds the middle
-    // (a larger one only adds empty registers to every pass)
+    // (a larger one adds a scalar test per empty register to every pass)
     const int64_t per = fkv::cdiv(tb.mid_end - tb.mid_start, fkv::kPartThreads);
     auto* kern = per <= 4    ? fkv::partition_regs_kernel<4>
                  : per <= 16 ? fkv::partition_regs_kernel<16>

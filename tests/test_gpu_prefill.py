@@ -81,6 +81,19 @@ def test_k_scale_finite_in_fp16(fkv, dt, top):
 @pytest.mark.parametrize("mid", [1, 63, 65, 4096, 4097, 16384, 16385, 50001, 65536, 65537])
 @pytest.mark.parametrize("kind", ["normal", "ties", "equal", "special"])
 def test_partition_size_edges(orc, fkv, mid, kind):
+    _check_partition(orc, mid, kind)
+
+
+# registers in use: all but the last, one chunk of four more than a multiple
+# of 1,024 fills, one chunk of a few waves only, the lowest key below and
+# beside the places past the middle
+@pytest.mark.parametrize("mid", [1023, 1024, 1025, 3073, 4100, 5121, 8192, 8193, 17408, 20481, 61440, 61441])
+@pytest.mark.parametrize("kind", ["normal", "special"])
+def test_partition_registers_in_use(orc, fkv, mid, kind):
+    _check_partition(orc, mid, kind)
+
+
+def _check_partition(orc, mid, kind):
     from foveated_kv_amd import ext
 
     S = mid + 36
