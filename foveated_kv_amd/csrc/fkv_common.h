@@ -91,8 +91,10 @@ __device__ inline void store8(void* p, uint32_t lo, uint32_t hi) {
 }
 
 // 8 consecutive elements, read once (non-temporal), as packed fp16 bits
-// (astype(float16) semantics: RNE)
-__device__ inline uint4 load8(const void* base, int dtype, int64_t elem) {
+// (astype(float16) semantics: RNE).  float32 elements, whose 32 bytes take two
+// loads, pass the caches by only with nt32: what the first load brings the
+// second one then has to fetch again from beyond them.
+__device__ inline uint4 load8(const void* base, int dtype, int64_t elem, bool nt32 = true) {
     if (dtype == FKV_F16) return load16_nt((const uint16_t*)base + elem);
     auto pk = [](float a, float b) { return (uint32_t)f2h(a) | ((uint32_t)f2h(b) << 16); };
     if (dtype == FKV_BF16) {
@@ -100,7 +102,8 @@ __device__ inline uint4 load8(const void* base, int dtype, int64_t elem) {
         auto two = [&](uint32_t u) { return pk(__uint_as_float(u << 16), __uint_as_float(u & 0xFFFF0000u)); };
         return make_uint4(two(w.x), two(w.y), two(w.z), two(w.w));
     }
-    const uint4 a = load16_nt((const float*)base + elem), b = load16_nt((const float*)base + elem + 4);
+    const uint4* p = (const uint4*)((const float*)base + elem);
+    const uint4 a = nt32 ? load16_nt(p) : p[0], b = nt32 ? load16_nt(p + 1) : p[1];
     auto two = [&](uint32_t x, uint32_t y) { return pk(__uint_as_float(x), __uint_as_float(y)); };
     return make_uint4(two(a.x, a.y), two(a.z, a.w), two(b.x, b.y), two(b.z, b.w));
 }

@@ -42,6 +42,7 @@ struct CompressArgs {
     // per-head-scaled fp8 keys (cfg->k_scale): (B*H) fp32 scales the far
     // keys are divided by before encoding; NULL = unscaled (the reference)
     const float* kscale;
+    bool nt_in;  // float32 K and V pass the caches by (load8)
 };
 
 // Packed-half integer operations (two fp16 bit patterns per dword).
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(256) void compress_kernel(CompressArgs a) {
     else if (t >= tb.mid_start && t < tb.near_mid_start) f = t - tb.mid_start;
 
     const int64_t src = ((int64_t)bh * a.S + t) * D + sub * 8;
-    const uint4 kw = load8(a.k, a.dtype, src), vw = load8(a.v, a.dtype, src);
+    const uint4 kw = load8(a.k, a.dtype, src, a.nt_in), vw = load8(a.v, a.dtype, src, a.nt_in);
     if (slot >= 0) {
         const int64_t o = ((int64_t)bh * npad + slot) * D + sub * 8;
         store16<NT>(a.near_k + o, kw);
@@ -684,8 +685,8 @@ __global__ __launch_bounds__(256) void compress_gather_kernel(CompressArgs a, co
     else t = far_idx[(int64_t)bh * F + (r - npad)];
     if (t >= 0 && t < a.S) {
         const int64_t src = ((int64_t)bh * a.S + t) * D + sub * 8;
-        kw = load8(a.k, a.dtype, src);
-        vw = load8(a.v, a.dtype, src);
+        kw = load8(a.k, a.dtype, src, a.nt_in);
+        vw = load8(a.v, a.dtype, src, a.nt_in);
     }
     if (near) {
         const int64_t o = ((int64_t)bh * npad + r) * D + sub * 8;
@@ -753,6 +754,7 @@ int compress_setup(const char* fn, const fkv_tier_config* cfg, const void* keys,
     a.arc_k = (uint16_t*)archive_k;
     a.arc_v = (uint16_t*)archive_v;
     a.kscale = nullptr;
+    a.nt_in = true;
     return FKV_OK;
 }
 
@@ -790,6 +792,11 @@ int compress_launch(const char* fn, const fkv_tier_config* cfg, fkv::CompressArg
     // both): from three quarters of the cache on.
     const size_t tiers = (size_t)B * H * ((size_t)a.tb.n_near_padded * D * 4 + (size_t)a.tb.far_count * (D + D / 2));
     const bool nt = tiers > ((size_t)192 << 20);
+    // the same line for float32 K and V, whose rows take two loads per lane:
+    // what stays in that cache is better read through it (126 MB: 38 us, 43-45
+    // past it, 42 before either; 150 MB 43-48, 52 and 48; 250 MB 79-80, 78 and
+    // 86; 512 MB 162, 154 and 171)
+    a.nt_in = (size_t)B * H * a.S * D * 8 > ((size_t)192 << 20);
     if (!near_idx) {
         const int rows = a.S + a.tb.headroom;
         dim3 grid((unsigned)fkv::cdiv(rows > 0 ? rows : 1, rpb), (unsigned)(B * H));

@@ -509,6 +509,24 @@ def test_compress_past_the_cache(fkv, importance):
             assert torch.equal(getattr(big, n)[b:b + 4], getattr(part, n)), n
 
 
+def test_float32_compress_past_the_cache(fkv):
+    """float32 K and V of 262 MB (read past the caches) give the bytes that a
+    batch at a time gives (65 MB, read through them), with key scales too."""
+    from foveated_kv_amd import ext
+
+    B, H, S, D = 4, 8, 8000, 128
+    g = torch.Generator(device="cuda").manual_seed(4)
+    k, v = (torch.randn((B, H, S, D), generator=g, device="cuda") for _ in range(2))
+    flush("float32 compress past the cache")
+    for ks in (0, 1):
+        h = ext.CompressHandle(_cfg(k_scale=ks))
+        big = h.compress_layer(k, v)
+        for b in range(B):
+            part = h.compress_layer(k[b:b + 1], v[b:b + 1])
+            for n in ("near_k", "near_v", "far_k", "far_v", "far_v_scale", "far_v_zero", "archive_k", "archive_v"):
+                assert torch.equal(getattr(big, n)[b:b + 1], getattr(part, n)), n
+
+
 @pytest.mark.parametrize("importance", [False, True])
 @pytest.mark.parametrize("dt,S,D", [(torch.float16, 700, 128), (torch.bfloat16, 37, 64), (torch.float32, 2100, 64),
                                     (torch.float16, 20, 128)])
