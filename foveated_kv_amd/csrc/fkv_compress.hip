@@ -219,6 +219,18 @@ __global__ __launch_bounds__(256) void compress_kernel(CompressArgs a) {
 constexpr int kScaleThreads = 256;
 constexpr int kScaleRows = 4;      // rows a lane group loads together
 constexpr int kScaleBlocks = 2048; // workgroups the reduction aims for
+constexpr int kScaleOneThreads = 1024, kScaleOneSweeps = 4;  // one workgroup per (batch, head)
+
+// Whether one workgroup of 1,024 threads takes a (batch, head)'s far rows and
+// writes the scale: up to 1,024 rows of 128 (2,048 of 64).  The second launch
+// costs a small call more than the rows do: 300 tokens of 128, 1 head, a call
+// 33 us with one workgroup of 256 threads, 35-36 with two launches, 32 here
+// (in a graph 13.5, 7.4 and 6.3); 2,000 tokens of 64 35, 36 and 33 (28, 7.7 and
+// 8.7).  At 3,000 tokens of 64 the rows of one workgroup take 10.4 in a graph
+// against 7.8.
+__host__ __device__ inline bool kscale_one(int F, int D) {
+    return F <= kScaleOneSweeps * kScaleRows * (kScaleOneThreads / (D / 8));
+}
 
 // Workgroups per (batch, head) of the reduction: each takes at least
 // kScaleRows rows per lane group, so their maxima (one fp32 each) always fit
@@ -259,6 +271,8 @@ struct FiniteMax {
     }
 };
 
+__device__ inline float kscale_of(float amax) { return amax > 0.f ? amax / 240.0f : 1.0f; }
+
 // Bound by the one read of the far keys.  A maximum does not depend on the
 // order, so the rows of a (batch, head) are dealt over as many workgroups as
 // fill the chip (one workgroup per head read 121 MB of keys at 8 heads x 59K
@@ -267,11 +281,12 @@ struct FiniteMax {
 // 16 rows in flight: no faster).
 // Far rows are positions mid_start.. (far_idx NULL) or far_idx[bh][f];
 // out-of-range indices are zero rows.
-template <int D, int DT>
-__global__ __launch_bounds__(kScaleThreads) void kscale_kernel(CompressArgs a, const int32_t* __restrict__ far_idx,
-                                                               float* __restrict__ part_max) {
-    constexpr int LPR = D / 8, RPB = kScaleThreads / LPR, NQ = DT == FKV_F32 ? 2 : 1;  // 16-byte loads per lane and row
-    __shared__ float red[kScaleThreads / kWave];
+template <int D, int DT, bool ONE>
+__global__ __launch_bounds__(ONE ? kScaleOneThreads : kScaleThreads) void kscale_kernel(
+    CompressArgs a, const int32_t* __restrict__ far_idx, float* __restrict__ out) {
+    constexpr int NT = ONE ? kScaleOneThreads : kScaleThreads;
+    constexpr int LPR = D / 8, RPB = NT / LPR, NQ = DT == FKV_F32 ? 2 : 1;  // 16-byte loads per lane and row
+    __shared__ float red[NT / kWave];
     const int bh = blockIdx.y, sub = threadIdx.x % LPR, parts = gridDim.x;
     const int F = a.tb.far_count;
     FiniteMax<DT> amax;
@@ -308,8 +323,9 @@ __global__ __launch_bounds__(kScaleThreads) void kscale_kernel(CompressArgs a, c
     __syncthreads();
     if (threadIdx.x == 0) {
         float m = 0.f;
-        for (int w = 0; w < kScaleThreads / kWave; w++) m = fmaxf(m, red[w]);
-        part_max[(int64_t)bh * parts + blockIdx.x] = m;
+        for (int w = 0; w < NT / kWave; w++) m = fmaxf(m, red[w]);
+        if (ONE) out[bh] = kscale_of(m);
+        else out[(int64_t)bh * parts + blockIdx.x] = m;
     }
 }
 
@@ -320,7 +336,7 @@ __global__ __launch_bounds__(kWave) void kscale_finish_kernel(const float* __res
     float m = 0.f;
     for (int i = threadIdx.x; i < parts; i += kWave) m = fmaxf(m, part_max[(int64_t)bh * parts + i]);
     m = wave_max(m);
-    if (threadIdx.x == 0) out[bh] = m > 0.f ? m / 240.0f : 1.0f;
+    if (threadIdx.x == 0) out[bh] = kscale_of(m);
 }
 
 // ---------------------------------------------------------------------------
@@ -766,20 +782,27 @@ int compress_launch(const char* fn, const fkv_tier_config* cfg, fkv::CompressArg
     const bool g32 = cfg->v_group == 32;
     if (cfg->k_scale) {
         if (!far_k_scale) return fkv::set_error(std::string(fn) + ": k_scale needs far_k_scale");
-        const int parts = fkv::kscale_parts(a.tb.far_count, D, B * H);
-        // the far code buffer holds the workgroups' maxima until they are
-        // reduced (the compress launch then writes the codes over them); with
-        // no far rows there is no buffer: the scales are 1
-        float* part_max = a.tb.far_count > 0 ? (float*)a.far_k : nullptr;
-        if (part_max) {
-            auto* kern = a.dtype == FKV_F16    ? (D == 128 ? fkv::kscale_kernel<128, FKV_F16> : fkv::kscale_kernel<64, FKV_F16>)
-                         : a.dtype == FKV_BF16 ? (D == 128 ? fkv::kscale_kernel<128, FKV_BF16> : fkv::kscale_kernel<64, FKV_BF16>)
-                                               : (D == 128 ? fkv::kscale_kernel<128, FKV_F32> : fkv::kscale_kernel<64, FKV_F32>);
-            hipLaunchKernelGGL(kern, dim3((unsigned)parts, (unsigned)(B * H)), dim3(fkv::kScaleThreads), 0, st, a,
-                               near_idx ? far_idx : nullptr, part_max);
+        const int F = a.tb.far_count;
+        const int32_t* idx = near_idx ? far_idx : nullptr;
+        auto pick = [&](auto ONE) {
+            constexpr bool one = ONE.value;
+            return a.dtype == FKV_F16    ? (D == 128 ? fkv::kscale_kernel<128, FKV_F16, one> : fkv::kscale_kernel<64, FKV_F16, one>)
+                   : a.dtype == FKV_BF16 ? (D == 128 ? fkv::kscale_kernel<128, FKV_BF16, one> : fkv::kscale_kernel<64, FKV_BF16, one>)
+                                         : (D == 128 ? fkv::kscale_kernel<128, FKV_F32, one> : fkv::kscale_kernel<64, FKV_F32, one>);
+        };
+        if (fkv::kscale_one(F, D)) {
+            hipLaunchKernelGGL(pick(std::true_type{}), dim3(1, (unsigned)(B * H)), dim3(fkv::kScaleOneThreads), 0, st, a,
+                               idx, far_k_scale);
+        } else {
+            // the far code buffer holds the workgroups' maxima until they are
+            // reduced (the compress launch then writes the codes over them)
+            const int parts = fkv::kscale_parts(F, D, B * H);
+            float* part_max = (float*)a.far_k;
+            hipLaunchKernelGGL(pick(std::false_type{}), dim3((unsigned)parts, (unsigned)(B * H)), dim3(fkv::kScaleThreads),
+                               0, st, a, idx, part_max);
+            hipLaunchKernelGGL(fkv::kscale_finish_kernel, dim3((unsigned)(B * H)), dim3(fkv::kWave), 0, st, part_max, parts,
+                               far_k_scale);
         }
-        hipLaunchKernelGGL(fkv::kscale_finish_kernel, dim3((unsigned)(B * H)), dim3(fkv::kWave), 0, st, part_max,
-                           part_max ? parts : 0, far_k_scale);
         a.kscale = far_k_scale;
     }
     const int rpb = 256 / (D / 8);

@@ -34,9 +34,12 @@ def _cfg(**kw):
 
 
 # far rows below one lane group's batch, just past one, several workgroups
-# with a ragged last one, and more rows than one sweep of the grid
+# with a ragged last one, and more rows than one sweep of the grid; the most
+# rows that one workgroup takes and one more
 @pytest.mark.parametrize("B,H,D,S,near_pct", [(1, 1, 128, 44, 0.0), (1, 2, 64, 166, 0.0), (2, 3, 128, 101, 0.0),
-                                              (1, 1, 128, 4099, 0.1), (40, 8, 64, 1500, 0.1)])
+                                              (1, 1, 128, 4099, 0.1), (40, 8, 64, 1500, 0.1),
+                                              (1, 2, 128, 1060, 0.0), (1, 2, 128, 1061, 0.0),
+                                              (2, 1, 64, 2084, 0.0), (2, 1, 64, 2085, 0.0)])
 def test_k_scale_reduction_edges(fkv, B, H, D, S, near_pct):
     """The scale is the exact maximum over every far row: a maximum planted in
     the first, the last and a middle far row of each head is found, one
@@ -58,22 +61,32 @@ def test_k_scale_reduction_edges(fkv, B, H, D, S, near_pct):
         assert np.array_equal(cl.far_k_scale.cpu().numpy(), want)
 
 
+def test_k_scale_without_far_rows(fkv):
+    from foveated_kv_amd import ext
+
+    k = torch.randn((2, 3, 30, 64), device="cuda").half()
+    cl = ext.CompressHandle(_cfg(k_scale=1)).compress_layer(k, k)
+    assert cl.far_k.shape[2] == 0 and torch.equal(cl.far_k_scale, torch.ones((2, 3), device="cuda"))
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("top", [65504.0, 65519.0, 65520.0, 65280.0, 65536.0, float("inf"), float("nan"), 6e-8, 2e-8, 0.0])
 def test_k_scale_finite_in_fp16(fkv, dt, top):
     """The maximum is over the keys as fp16: one that overflows there is left
-    out, as infinities and NaN are, whatever type it came in."""
+    out, as infinities and NaN are, whatever type it came in (one workgroup
+    per head, and several)."""
     from foveated_kv_amd import ext
 
-    flush(f"k_scale of {top} from {dt}")
-    k = torch.full((1, 2, 300, 64), 1e-8 if 0 < top < 1e-3 or top == 0 else 3.0)
-    k[0, 0, 150, 5], k[0, 0, 151, 6] = top, -top
-    k = k.to(dt).cuda()
-    cl = ext.CompressHandle(_cfg(k_scale=1)).compress_layer(k, k)
-    far = cl.archive_k.float()
-    far = torch.where(torch.isfinite(far), far.abs(), torch.zeros_like(far)).amax((2, 3)).cpu().numpy()
-    want = np.where(far > 0, far / np.float32(240), np.float32(1)).astype(np.float32)
-    assert np.array_equal(cl.far_k_scale.cpu().numpy(), want)
+    for S in (300, 3000):
+        flush(f"k_scale of {top} from {dt} S={S}")
+        k = torch.full((1, 2, S, 64), 1e-8 if 0 < top < 1e-3 or top == 0 else 3.0)
+        k[0, 0, 150, 5], k[0, 0, 151, 6] = top, -top
+        k = k.to(dt).cuda()
+        cl = ext.CompressHandle(_cfg(k_scale=1)).compress_layer(k, k)
+        far = cl.archive_k.float()
+        far = torch.where(torch.isfinite(far), far.abs(), torch.zeros_like(far)).amax((2, 3)).cpu().numpy()
+        want = np.where(far > 0, far / np.float32(240), np.float32(1)).astype(np.float32)
+        assert np.array_equal(cl.far_k_scale.cpu().numpy(), want)
 
 
 # the edges of the tokens a thread holds (4, 16, 64 per thread of 1,024),
