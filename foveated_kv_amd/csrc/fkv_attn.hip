@@ -920,21 +920,20 @@ static int plan_splits(const BlobLayout& L, int rows, int n_dec, int target, int
 // Whether a round is two workgroups per CU.  Two fit at D = 64 with one or
 // two head quads (137-183 VGPRs, 72-80 KB of LDS; nothing else does), and
 // the second one overlaps the first's chains: worth it for TurboQuant from
-// 20 rows on (below, a row's merge of more records outweighs it) and for two
-// quads that 256 workgroups split into at most 3; one quad of fp8 keys is
-// bound by memory, so there only where more than a fifth of the CUs would
-// stay idle.  Contexts under 32 tiles: one.  Measured with one / two per CU,
+// 20 rows on (below, a row's merge of more records outweighs it), for rows of
+// 32 tiles and more that leave over a fifth of the CUs without a workgroup,
+// and for two quads that 256 workgroups split into at most 3 from 64 tiles on
+// (one quad of fp8 keys is bound by memory).  Measured with one / two per CU,
 // 16,384 tokens unless said, us: TurboQuant 7 heads, 172 rows 157.8 / 115.6,
 // 24 rows of 4 heads 22.0 / 15.8; fp8 7 heads, 132 rows 89.5 / 52.4, 72 rows
-// 37.0 / 30.4, 36 rows 22.5 / 21.0 (8,192: 16.2 / 16.4); fp8 4 heads, 132 rows
-// 62.8 / 47.3, 64 rows 23.6 / 24.5, 16 rows 12.5 / 14.7, 200 rows of 1,024
-// tokens 8.8 / 9.9.
+// 37.0 / 30.4 (2,048: 11.9 / 13.3), 36 rows 22.5 / 21.0 (8,192: 16.2 / 16.4);
+// fp8 4 heads, 132 rows 62.8 / 47.3, 64 rows 23.6 / 24.5, 16 rows 12.5 / 14.7,
+// 200 rows of 1,024 tokens 8.8 / 9.9.
 static bool two_workgroups_per_cu(const BlobLayout& L, int rows, int quads, int n_dec, int target) {
     if (L.D != 64 || quads > 2) return false;
-    const int one = target / (rows > 0 ? rows : 1);
+    const int one = target / (rows > 0 ? rows : 1), tiles = plan_tiles(L, n_dec);
     if (L.fmt == 1) return one <= 12;
-    if (plan_tiles(L, n_dec) < 32) return false;
-    return quads == 2 ? one <= 3 : one * rows * 5 < target * 4;
+    return (tiles >= 32 && one * rows * 5 < target * 4) || (tiles >= 64 && quads == 2 && one <= 3);
 }
 
 static size_t partial_floats(int rows, int splits, int ng_max, int D) {

@@ -273,6 +273,7 @@ def test_launch_plan_where_two_workgroups_share_a_cu(fmt):
     assert splits(31, 8, 4, 16384) == (248, 2 if fmt == 1 else 1)                       # one quad, few CUs idle
     assert splits(31, 8, 7, 16384) == (248, 2) and splits(32, 8, 4, 16384) == (256, 2 if fmt == 1 else 1)
     assert splits(33, 4, 4, 1024) == (132, 2 if fmt == 1 else 1)                        # short
+    assert splits(18, 4, 7, 2048) == (72, 4 if fmt == 1 else 3)                         # two quads, few CUs idle
     assert splits(18, 4, 7, 16384) == (72, 7) and splits(8, 2, 4, 16384) == (16, 16)
 
 
