@@ -47,18 +47,20 @@ class TurboConstants:
 
     def on(self, device):
         device = torch.device(device)
-        if device.type == "cuda" and device.index is None:
+        if device.index is None and device.type == "cuda":
             device = torch.device("cuda", torch.cuda.current_device())
+        hit = self.__dict__.get("_device_copies", {}).get(device)
+        if hit is not None and hit[0] == (self.Pi._version, self.S._version, self.centroids._version,
+                                          self.boundaries._version):
+            return hit[1]
         src = (self.Pi, self.S, self.centroids, self.boundaries)
         if any(not isinstance(t, torch.Tensor) or t.is_inference() for t in src):
             # nothing says whether these were written to: copied on each call
             return TurboConstants(*(torch.as_tensor(t).to(device) for t in src))
         versions = tuple(t._version for t in src)
-        copies = self.__dict__.setdefault("_device_copies", {})
-        hit = copies.get(device)
-        if hit is None or hit[0] != versions:
-            hit = copies[device] = (versions, TurboConstants(*(t.to(device) for t in src)))
-        return hit[1]
+        copies = TurboConstants(*(t.to(device) for t in src))
+        self.__dict__.setdefault("_device_copies", {})[device] = (versions, copies)
+        return copies
 
     def __getstate__(self):
         return {k: v for k, v in self.__dict__.items() if k != "_device_copies"}
@@ -149,9 +151,10 @@ def turbo_compress_keys(keys: torch.Tensor, tc: TurboConstants):
         return idx, sgn, nrm, gam
     c = tc.on(dev)
     # the kernel reads D * D, 4 and 3 elements whatever the constants hold
-    for name, n in (("Pi", D * D), ("S", D * D), ("centroids", 4), ("boundaries", 3)):
-        if getattr(c, name).numel() != n:
-            raise ValueError(f"{name} has {getattr(c, name).numel()} elements, keys of {D} dims need {n}")
+    if c.Pi.numel() != D * D or c.S.numel() != D * D or c.centroids.numel() != 4 or c.boundaries.numel() != 3:
+        raise ValueError(f"keys of {D} dims need Pi and S of ({D}, {D}), centroids of (4,) and boundaries of (3,), got "
+                         f"Pi {tuple(c.Pi.shape)}, S {tuple(c.S.shape)}, centroids {tuple(c.centroids.shape)}, "
+                         f"boundaries {tuple(c.boundaries.shape)}")
     lib = _lib.load()
     with torch.cuda.device(dev):
         check(lib.fkv_turbo_compress_keys(ptr(k), dtype_code(k.dtype), B * H * N, D, ptr(_f32(c.Pi, dev)),
