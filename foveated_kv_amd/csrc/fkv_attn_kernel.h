@@ -58,7 +58,7 @@ constexpr int kSmallGrid = 64;  // fewer workgroups than this: rows of 4 query h
 constexpr int kHdr = 8;
 constexpr int kMaxSplits = 64;
 
-// Waves per workgroup of the attention kernel (one workgroup per CU): 8 for
+// Waves per workgroup of the attention kernel (one per CU at D = 128): 8 for
 // TurboQuant rows of one head quad at D = 128 -- two waves per SIMD, whose
 // far tile is bound by dependent VALU / MFMA chains that the second wave
 // overlaps (8 KB ring units, registers within 256) while the query rotation
