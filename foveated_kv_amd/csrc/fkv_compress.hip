@@ -75,6 +75,16 @@ __device__ inline uint32_t encode_e4m3x4(uint32_t w0, uint32_t w1) {
     return (codes & ~mask) | (mask & 0x7E7E7E7Eu);
 }
 
+// fp16(a / b), the quotient rounded to fp32 first (y = 1.0f / b).  The empty
+// asm keeps the two roundings apart: the compiler would fuse the quotient's
+// last fma with the conversion into one that rounds once, which gives another
+// fp16 value where fp32's rounding has moved the quotient onto a tie.
+__device__ inline uint16_t quotient_h(float a, float b, float y) {
+    float q = div_by<1>(a, b, y);
+    asm volatile("" : "+v"(q));
+    return f2h(q);
+}
+
 // The fp16 value a key is encoded from with a per-head scale: fp16(key /
 // scale), fp32 division rounded to nearest even.  One correction step is
 // enough for every fp16 key and every scale that is an fp16 amax over 240
@@ -83,7 +93,7 @@ __device__ inline uint32_t encode_e4m3x4(uint32_t w0, uint32_t w1) {
 // are.
 __device__ inline uint32_t scaled_keys(uint32_t w, float scale, float rscale) {
     const uint16_t lo = (uint16_t)w, hi = (uint16_t)(w >> 16);
-    const uint16_t ql = f2h(div_by<1>(h2f(lo), scale, rscale)), qh = f2h(div_by<1>(h2f(hi), scale, rscale));
+    const uint16_t ql = quotient_h(h2f(lo), scale, rscale), qh = quotient_h(h2f(hi), scale, rscale);
     const uint32_t q = ((lo & 0x7C00u) == 0x7C00u ? lo : ql) | ((uint32_t)((hi & 0x7C00u) == 0x7C00u ? hi : qh) << 16);
     return (q & 0x7FFF7FFFu) | (w & 0x80008000u);
 }

@@ -187,6 +187,38 @@ def test_far_rows_special_values(fkv, D, vg, dt, importance):
         assert np.array_equal(cl.far_k.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("exponent", [15, 0, -15])
+def test_scaled_keys_every_pair(fkv, exponent):
+    """Every fp16 key against every mantissa that a head's largest key can
+    have: the code of fp16(fp32(key / scale)), both roundings apart (one
+    rounding to fp16 of the quotient gives another code where fp32's has
+    moved it onto a tie: 0.958 / (5 / 240) among others)."""
+    import oracle
+    from foveated_kv_amd import ext
+
+    B, H, D = 16, 64, 64
+    keys = np.arange(0x7C00, dtype=np.uint16).view(np.float16)
+    keys[1::2] *= -1
+    # mantissas of one binade (the subnormal one for the least exponent)
+    top = (np.arange(1024, dtype=np.float64) + 1024) * 2.0 ** (exponent - 10)
+    if exponent == -15:
+        top = (np.arange(1024, dtype=np.float64) + 1) * 2.0 ** -24
+    top = top.astype(np.float16).reshape(B, H, 1)
+    flat = np.clip(keys, -top, top)
+    flat[..., 0] = top[..., 0]
+    rows = flat.reshape(B, H, 496, D)
+    pad = [np.zeros((B, H, n, D), np.float16) for n in (4, 32)]
+    k = torch.from_numpy(np.concatenate([pad[0], rows, pad[1]], 2)).cuda()
+    flush(f"scaled keys, every pair, largest key 2^{exponent}")
+    cl = ext.CompressHandle(_cfg(k_scale=1, near_pct=0.0)).compress_layer(k, k, with_archive=False)
+    scale = top.astype(np.float32) / np.float32(240)
+    assert np.array_equal(cl.far_k_scale.cpu().numpy(), scale[..., 0])
+    with np.errstate(all="ignore"):
+        want = oracle.encode_fp8((rows.astype(np.float32) / scale[..., None]).astype(np.float16))
+    bad = cl.far_k.cpu().numpy() != want
+    assert not bad.any(), (int(bad.sum()), rows[bad][:4])
+
+
 def _unpack(p, bits):
     per = 8 // bits
     return ((p[..., None] >> (bits * np.arange(per))) & ((1 << bits) - 1)).reshape(p.shape[:-1] + (-1,))
