@@ -339,14 +339,23 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
     for (int s = 0; s < NS; s++)
 #pragma unroll
         for (int e = 0; e < 8; e++) ss[e] = fmaf((float)kb[s][e], (float)kb[s][e], ss[e]);
-    const float nrm = sqrtf(tq_half_sum(ss));
-    {
-        // y >= b  <=>  k Pi^T >= b max(n, 1e-8)
-        const float nc = fmaxf(nrm, 1e-8f);
-        b0 *= nc;
-        b1 *= nc;
-        b2 *= nc;
+    const float norm = sqrtf(tq_half_sum(ss));
+    // Keys of a small norm times 2^14 (exact; everything below scales with
+    // them): products of fp16 subnormals would be summed with fewer bits (keys
+    // of standard deviation 2^-22, 400,000 tokens of 128: 85 codes off 64 bits).
+    const bool tiny = norm < 0x1p-6f;
+    float nrm = norm, nc = fmaxf(norm, 1e-8f);
+    if (__ballot(tiny)) {
+        const float up = tiny ? 0x1p14f : 1.0f;
+#pragma unroll
+        for (int s = 0; s < NS; s++) kb[s] *= (_Float16)up;
+        nrm *= up;
+        nc *= up;
     }
+    // y >= b  <=>  k Pi^T >= b max(n, 1e-8)
+    b0 *= nc;
+    b1 *= nc;
+    b2 *= nc;
     TqGemm<D> g{op_s, lane, {}};
     // ---- codes ----
     ready();
@@ -474,8 +483,8 @@ __global__ __launch_bounds__(256, 2) void tq_compress_keys_kernel(const void* __
         }
     const float gamma = sqrtf(tq_half_sum(ss));
     if (live && h == 0) {
-        out_norm[t] = f2h(nrm);
-        out_gamma[t] = f2h(gamma);
+        out_norm[t] = f2h(norm);
+        out_gamma[t] = f2h(tiny ? gamma * 0x1p-14f : gamma);
     }
     // the residual scaled so that its largest value is at most 512 (only the
     // sign of its projections is kept); a non-finite one gives no sign

@@ -648,6 +648,32 @@ def test_archive_layer_ignores_the_key_scale_option(fkv):
         assert torch.equal(getattr(layers[0], n), getattr(layers[1], n)), n
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("e", [-6, -9, -16, -20, -22])
+def test_turbo_codes_of_small_keys(fkv, D, e):
+    """Keys down to a few units of fp16's subnormals, alone and beside large
+    ones in a wave: every code is the one of fp64, norms and residual norms
+    are those of the keys, and so are the signs away from rounding."""
+    from foveated_kv_amd import _lib
+    from foveated_kv_amd.turbo import get_turbo_constants
+
+    g = torch.Generator(device="cuda").manual_seed(D - e)
+    k = (torch.randn((200_003, D), generator=g, device="cuda") * 2.0 ** e).half()
+    k[7::64] = (k[7::64].float() * 2.0 ** (3 - e)).half()
+    k[5] = 0
+    k[6] = 2.0 ** -24
+    flush(f"turbo codes of small keys D={D} 2^{e}")
+    tc = get_turbo_constants(D)
+    args = [t.numpy() for t in (tc.Pi, tc.S, tc.centroids, tc.boundaries)]
+    got = _turbo_keys(_lib, k, *args)
+    kd = k.double()
+    y = (kd @ tc.Pi.cuda().double().T.contiguous()) / kd.norm(dim=-1, keepdim=True).clamp_min(np.float32(1e-8))
+    want = torch.bucketize(y, tc.boundaries.cuda().double(), right=True)
+    codes = ((got[0].unsqueeze(-1) >> torch.tensor([0, 2, 4, 6], device="cuda", dtype=torch.uint8)) & 3).flatten(-2)
+    assert int((codes != want).sum()) == 0
+    _check_turbo_keys(k[:20000].cpu().numpy(), *args, tuple(t[:20000] for t in got))
+
+
 def _keys_near_a_boundary(tc, rng):
     """fp16 keys, one for every dim, boundary and side, whose rotated
     coordinate lies 1e-9 to 3e-8 of their norm from the boundary in fp64:
