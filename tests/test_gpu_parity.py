@@ -187,6 +187,30 @@ def test_attention_partial_quad_rows(fkv, orc, args, vg):
     run_attention(fkv, orc, v_group=vg, **args)
 
 
+# D = 64 rows split for two workgroups per CU: many rows of one and two
+# quads, in whole groups of 8 rows (split merge within an XCD) and not
+TWO_PER_CU = [
+    dict(B=33, Hq=16, Hkv=4, D=64, S=2200, n_dec=3, seed=56),                # 132 rows, 3 splits
+    dict(B=18, Hq=28, Hkv=4, D=64, S=4400, n_dec=0, seed=57, spikes=0.02),   # 72 rows of two quads, 7 splits
+]
+
+
+@pytest.mark.parametrize("vg", [0, 32])
+@pytest.mark.parametrize("args", TWO_PER_CU, ids=[f"B{a['B']}_Hq{a['Hq']}_S{a['S']}" for a in TWO_PER_CU])
+def test_attention_two_workgroups_per_cu(fkv, orc, args, vg):
+    from foveated_kv_amd import _lib
+
+    out = (ctypes.c_int64 * 8)()
+    tb = orc.tier_boundaries(args["S"], promo_headroom_min=8)
+    assert _lib.load().fkv_attn_plan(args["B"], args["Hkv"], 64, tb["N_near_padded"], tb["far_count"],
+                                     args["Hq"], args["n_dec"], 256, 2 if vg else 0, out) == 0
+    assert 256 < out[1] * out[2] <= 512
+    # against the kernel's oracle only: at these sizes the formulation's fp16
+    # dequantisation leaves that oracle by up to 1.6e-3 by itself, and half an
+    # fp16 unit of an output past 2 is 1e-3 more
+    run_attention(fkv, orc, v_group=vg, check_formulation=False, **args)
+
+
 GROUP32 = [
     dict(B=1, Hq=14, Hkv=2, D=64, S=512, n_dec=16, seed=31),
     dict(B=1, Hq=32, Hkv=8, D=128, S=4096, n_dec=64, seed=32, heavy_tail=True),

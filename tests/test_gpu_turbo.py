@@ -88,6 +88,8 @@ CASES = [
     (1, 8, 2, 128, 0, 64, (40, 64), 2),
     (2, 24, 2, 128, 8000, 896, (800, 750), 4),  # G = 12: rows of three head quads
     (1, 28, 4, 128, 9000, 1000, (900, 850, 1000, 700), 3),  # G = 7: 16-head rows, second quad partial
+    (9, 12, 4, 64, 3900, 400, (300, 400, 350, 390), 2),     # two workgroups per CU: 36 rows, 8 splits
+    (34, 28, 4, 64, 1100, 128, (128, 100, 90, 110), 3),     # 136 rows of two quads, 2 splits
 ]
 
 
